@@ -1,5 +1,6 @@
 // mps_api_internal.h -- host-side preparation shared by the single and batched forms.
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #include <string>
@@ -27,6 +28,15 @@ struct HostPrep {
     int32_t bc_mode = 0, vel_ramp = 0;
     mps_solver_cfg cfg{};
 };
+
+// Tables of the spread form (mps_common.h); nb = 0: the mesh does not take it.
+struct SpreadTables {
+    int32_t nb = 0, stride = 0;
+    std::vector<int4> node;
+    std::vector<uint16_t> lx;
+    std::vector<int32_t> pos, own;
+};
+void build_spread(const HostPrep& hp, SpreadTables* sp);
 
 std::string fmt(const char* f, ...);
 void material_consts(int law, double E, double nu, double rho, double* pa, double* pb, double* c);

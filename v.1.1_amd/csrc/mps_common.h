@@ -40,9 +40,9 @@
 //     pc            double[24*n_sgp]  the step's surface forces [(g*8 + a)*3 + dir]
 //   uprev           double[3N]   displacement of the previous step (bulk viscosity only; NULL otherwise)
 //   ctl             MpsCtl       step control (time, dt, go flags), running work sums, reduction counters
-//   dtred           u64[2*MPS_DT_SLOTS*MPS_DT_STRIDE]  stable-dt reduction slots by step parity; in the
+//   dtred           u64[MPS_DT_WORDS]  stable-dt reduction slots by step parity; in the
 //                   single-instance form followed by MPS_DT_SLOTS + 1 counters (same stride) of the
-//                   stable-dt certificate (MPS_DT_COUNT_WORDS)
+//                   stable-dt certificate (MPS_DT_COUNT_WORDS) and the spread form's slots (MPS_DT_SPREAD_WORDS)
 //   hist            double[MPS_HIST_COLS*hist_cap]     per-step history ring, column c at c*hist_cap
 //   energy bookkeeping (solves with energies only):
 //     epart         double[3*n_patch + 2*MPS_NODE_PARTS*node_blocks]  per-block energy sums: element phase, then
@@ -50,6 +50,7 @@
 //     rprev         double[3*R]       previous step's support force fint - fext of each Dirichlet record
 //     lfprev        double[3*n_lnode] previous step's external force of each flagged node
 #pragma once
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #define MPS_MAX_NEN 8
@@ -57,7 +58,11 @@
 #define MPS_DT_SLOTS 16   // stable-dt reduction slots per step parity: workgroup b min-reduces into slot b % 16
 #define MPS_DT_STRIDE 32  // u64 between two slots (256 B), so the slots' atomics do not share a line
 #define MPS_DT_SKIP_HOLD 64  // steps without the stable-dt skip after a failed certificate
+#define MPS_DT_WORDS (2 * MPS_DT_SLOTS * MPS_DT_STRIDE)
+#define MPS_DT_SPREAD_WORDS (3 * MPS_DT_SLOTS * MPS_DT_STRIDE)  // the spread form's three sets, after the counters
 #define MPS_DT_COUNT_WORDS ((MPS_DT_SLOTS + 1) * MPS_DT_STRIDE)  // certificate counters after the dt slots
+#define MPS_SPREAD_HEX 8     // elements per workgroup of the spread form, hex8: one wave of eight lanes per element
+#define MPS_SPREAD_TET 64    // and tet4: one wave
 #define MPS_NODE_LOADED 0x80000000u  // ninfo bit: the node has nodal force entries
 #define MPS_REC_MASK 0x7FFFFFFFu     // ninfo bits below the loaded flag
 #define MPS_ITEM_FORCE 0u            // load item kinds (lcode >> 30)
@@ -96,10 +101,16 @@ struct MpsStepSlot {
 //   B = step whose forces are in part, written only by the element kernel, read by node/energy.
 // slot[k&1] holds step k; the dtred slots of parity k&1 receive the min over elements for
 // step k (computed from u_{k-1}); the node kernel of step k resets them.
+// In the spread form (mps_spread.hip) A stays the first step of a launch sequence until its end and B is the last step
+// begun.  The step with index ci in the sequence keeps its scalars in sslot[ci&1] and reads the min of set ci%3 of the
+// spread dt slots (the first step: slot[] and dtred), reduces into set (ci+1)%3 and resets the third, so that every
+// address is known before anything is read; the end of the sequence hands over to slot[], dtred and A.
 struct MpsCtl {
     MpsStepSlot slot[2];
     long long A;
     long long B;
+    MpsStepSlot sslot[2];  // spread form: scalars of the step by its index in the launch sequence
+    long long spread_last; // spread form: parity of the last step's index
     int32_t status;     // MPS_RUNNING / MPS_DONE / MPS_ERR_DT
     int32_t nonfinite;  // set when u[1] is non-finite
     long long nan_step; // first step with non-finite u[1] (LLONG_MAX if none)
@@ -181,6 +192,16 @@ struct MpsInst {
     // stable-dt skip: on/off, and the threshold's margin over the previous step's min (MpsCtl::dt_skip)
     int32_t dt_skip_on;
     double dt_skip_margin;
+    // spread form (mps_spread.hip; sp_nb = 0: not set up): sp_nb workgroups of consecutive elements, each with up to
+    // sp_stride distinct nodes
+    int32_t sp_nb, sp_stride;
+    const int4* sp_node;      // [sp_nb*sp_stride] {node (bit 31: owned by this workgroup), first position, count, end bits
+                              // of the patches among its positions}; x = -1: padding
+    const uint16_t* sp_lx;    // [nen*Ne] index of each element slot's node among its workgroup's nodes
+    const int32_t* sp_pos;    // [nen*Ne] position of each element slot in node order
+    const int32_t* sp_own;    // [N] entry of sp_node that owns the node
+    void* sp_f;               // [2][3*nen*Ne] element forces in node order, by the parity of the step's index
+    double* sp_uw;            // [6*N] alternate u and w
     // per-step DOF series (mps_set_dof_series): n_series entries, recorded into ser_ring[(k-1)%hist_cap][i]
     int32_t n_series;
     const int32_t* ser_dof;   // node + N*dir

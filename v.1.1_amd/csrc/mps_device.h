@@ -36,13 +36,31 @@ __device__ __forceinline__ constexpr int sxi(int a) { return (a == 1 || a == 2 |
 __device__ __forceinline__ constexpr int seta(int a) { return (a == 2 || a == 3 || a == 6 || a == 7) ? 1 : -1; }
 __device__ __forceinline__ constexpr int szeta(int a) { return (a >= 4) ? 1 : -1; }
 
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
+// The arithmetic of the element forces is written with explicit FMAs and without contraction, so that an element's
+// forces have the same bits in every kernel that computes them (one work-item per element, eight per element, batched,
+// with energies), whatever the compiler places around it.
+template <typename T>
+__device__ __forceinline__ T diff2(T a, T b, T c, T d) {  // a b - c d
+#pragma clang fp contract(off)
+    return fma_t(a, b, -(c * d));
+}
+template <typename T>
+__device__ __forceinline__ T dot3(T a, T b, T c, T d, T e, T f) {  // a b + c d + e f
+#pragma clang fp contract(off)
+    return fma_t(e, f, fma_t(a, b, c * d));
+}
+
 // ---------------------------------------------------------------------------
 // 3x3 helpers (row-major)
 // ---------------------------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ T det3(const T* A) {
-    return A[0] * (A[4] * A[8] - A[7] * A[5]) - A[1] * (A[3] * A[8] - A[6] * A[5]) +
-           A[2] * (A[3] * A[7] - A[6] * A[4]);
+#pragma clang fp contract(off)
+    const T m0 = diff2(A[4], A[8], A[7], A[5]), m1 = diff2(A[3], A[8], A[6], A[5]), m2 = diff2(A[3], A[7], A[6], A[4]);
+    return fma_t(A[2], m2, fma_t(A[0], m0, -(A[1] * m1)));
 }
 
 __device__ __forceinline__ double rcp(double x);
@@ -112,27 +130,30 @@ __host__ __device__ inline double det3_strict(const double* A) {
 // det(I+H) - 1 without cancellation: tr H + i2(H) + det H.
 template <typename T>
 __device__ __forceinline__ T detIpH_m1(const T* H) {
-    T tr = H[0] + H[4] + H[8];
-    T i2 = H[0] * H[4] + H[4] * H[8] + H[0] * H[8] - H[1] * H[3] - H[5] * H[7] - H[2] * H[6];
+#pragma clang fp contract(off)
+    const T tr = H[0] + H[4] + H[8];
+    const T p = fma_t(H[0], H[8], fma_t(H[0], H[4], H[4] * H[8]));
+    const T i2 = fma_t(-H[2], H[6], fma_t(-H[5], H[7], fma_t(-H[1], H[3], p)));
     return tr + i2 + det3(H);
 }
 
 // Cofactor matrix cof(A)(i,j) = (-1)^(i+j) minor_ij; A^-1 = cof(A)^T / det A.
 template <typename T>
 __device__ __forceinline__ void cof3(const T* A, T* C) {
-    C[0] = A[4] * A[8] - A[5] * A[7];
-    C[1] = A[5] * A[6] - A[3] * A[8];
-    C[2] = A[3] * A[7] - A[4] * A[6];
-    C[3] = A[2] * A[7] - A[1] * A[8];
-    C[4] = A[0] * A[8] - A[2] * A[6];
-    C[5] = A[1] * A[6] - A[0] * A[7];
-    C[6] = A[1] * A[5] - A[2] * A[4];
-    C[7] = A[2] * A[3] - A[0] * A[5];
-    C[8] = A[0] * A[4] - A[1] * A[3];
+    C[0] = diff2(A[4], A[8], A[5], A[7]);
+    C[1] = diff2(A[5], A[6], A[3], A[8]);
+    C[2] = diff2(A[3], A[7], A[4], A[6]);
+    C[3] = diff2(A[2], A[7], A[1], A[8]);
+    C[4] = diff2(A[0], A[8], A[2], A[6]);
+    C[5] = diff2(A[1], A[6], A[0], A[7]);
+    C[6] = diff2(A[1], A[5], A[2], A[4]);
+    C[7] = diff2(A[2], A[3], A[0], A[5]);
+    C[8] = diff2(A[0], A[4], A[1], A[3]);
 }
 
 // Reciprocal: hardware estimate refined by Newton steps (<= 1 ulp for FP64).
 __device__ __forceinline__ double rcp(double x) {
+#pragma clang fp contract(off)
     double r = __builtin_amdgcn_rcp(x);
     double e = fma(-x, r, 1.0);
     r = fma(e, r, r);
@@ -145,6 +166,7 @@ __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x);
 // log(1+x) = 2 atanh(t) = 2 (t + t^3/3 + ... + t^15/15); for |x| < 0.1, |t| < 0.0527 and the
 // truncation error is below 2^-60 relative.  Outside that range the library log is used.
 __device__ __forceinline__ double log_near1(double J) {
+#pragma clang fp contract(off)
     const double x = J - 1.0;
     if (fabs(x) >= 0.1) return log(J);
     const double t = x * rcp(2.0 + x);
@@ -162,6 +184,7 @@ __device__ __forceinline__ double log_near1(double J) {
 // log(1+x) (FP32): Taylor series to x^9 for |x| < 0.05 (truncation < 2e-13 relative);
 // otherwise Goldberg's form log(u) * x / (u - 1), u = 1 + x.
 __device__ __forceinline__ float log1p_fast(float x) {
+#pragma clang fp contract(off)
     if (fabsf(x) < 0.05f) {
         float p = 1.f / 9.f;
         p = fmaf(p, x, -1.f / 8.f);
@@ -190,23 +213,21 @@ __device__ __forceinline__ float log1p_fast(float x) {
 // Both are written in H, which carries no cancellation at small strain.  (pa, pb) = (lambda, mu).
 template <typename T, int LAW>
 __device__ __forceinline__ void pk1_svk_lin(const T* H, T lam, T mu, T* P) {
+#pragma clang fp contract(off)
     T E[9];
 #pragma unroll
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++) {
             T e = T(0.5) * (H[i * 3 + j] + H[j * 3 + i]);
-            if (LAW == 2) e += T(0.5) * (H[i] * H[j] + H[3 + i] * H[3 + j] + H[6 + i] * H[6 + j]);
+            if (LAW == 2) e = fma_t(T(0.5), dot3(H[i], H[j], H[3 + i], H[3 + j], H[6 + i], H[6 + j]), e);
             E[i * 3 + j] = e;
         }
     const T ltr = lam * (E[0] + E[4] + E[8]);
     const T mu2 = T(2) * mu;
     T S[9];
 #pragma unroll
-    for (int i = 0; i < 9; i++) S[i] = mu2 * E[i];
-    S[0] += ltr;
-    S[4] += ltr;
-    S[8] += ltr;
+    for (int i = 0; i < 9; i++) S[i] = (i % 4) == 0 ? fma_t(mu2, E[i], ltr) : mu2 * E[i];
     if (LAW == 3) {
 #pragma unroll
         for (int i = 0; i < 9; i++) P[i] = S[i];
@@ -216,48 +237,31 @@ __device__ __forceinline__ void pk1_svk_lin(const T* H, T lam, T mu, T* P) {
     for (int i = 0; i < 3; i++)
 #pragma unroll
         for (int j = 0; j < 3; j++)
-            P[i * 3 + j] = S[i * 3 + j] + H[i * 3] * S[j] + H[i * 3 + 1] * S[3 + j] + H[i * 3 + 2] * S[6 + j];
+            P[i * 3 + j] = fma_t(H[i * 3 + 2], S[6 + j], fma_t(H[i * 3 + 1], S[3 + j], fma_t(H[i * 3], S[j], S[i * 3 + j])));
 }
 
 __device__ __forceinline__ double defo_energy(int law, const double* F, double lambda, double mu);
 
-// FP64: F-based, as the reference (neo-Hookean laws).  With W and Jout (energy steps) also the energy density
-// W(F) (defo_energy) and J = det F, from the quantities P is computed with; P is the same either way.
+// FP64: F-based, as the reference (neo-Hookean laws, LAW 0 and 1).  With W and Jout (energy steps) also the energy
+// density W(F) (defo_energy) and J = det F, from the quantities P is computed with; P is the same either way.
 template <int LAW>
-__device__ __forceinline__ void pk1(const double* H, double pa, double pb, double* P, double* W = nullptr,
-                                    double* Jout = nullptr) {
-    if (LAW >= 2) {
-        pk1_svk_lin<double, LAW>(H, pa, pb, P);
-        if (W) {
-            double F[9];
-#pragma unroll
-            for (int i = 0; i < 9; i++) F[i] = H[i] + ((i % 4) == 0 ? 1.0 : 0.0);
-            *W = defo_energy(LAW, F, pa, pb);
-            *Jout = 1.0 + detIpH_m1(H);
-        }
-        return;
-    }
-    double F[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) F[i] = H[i];
-    F[0] += 1.0;
-    F[4] += 1.0;
-    F[8] += 1.0;
+__device__ __forceinline__ void pk1_F(const double* F, double pa, double pb, double* P, double* W = nullptr,
+                                      double* Jout = nullptr) {
+#pragma clang fp contract(off)
     double cF[9];
     cof3(F, cF);
-    const double J = F[0] * cF[0] + F[1] * cF[1] + F[2] * cF[2];
+    const double J = dot3(F[0], cF[0], F[1], cF[1], F[2], cF[2]);
     if (Jout) *Jout = J;
     if (LAW == 0) {  // pa = lambda, pb = mu
         const double l = log_near1(J);
-        const double alpha = pa * l - pb;
-        const double s = alpha * rcp(J);
+        const double s = fma(pa, l, -pb) * rcp(J);
 #pragma unroll
-        for (int i = 0; i < 9; i++) P[i] = pb * F[i] + s * cF[i];
+        for (int i = 0; i < 9; i++) P[i] = fma(pb, F[i], s * cF[i]);
         if (W) {  // 1/2 lambda (ln J)^2 - mu ln J + 1/2 mu tr C (hyperElasticNeoHookean.cpp:291-304)
             double trC = 0.0;
 #pragma unroll
-            for (int i = 0; i < 9; i++) trC += F[i] * F[i];
-            *W = 0.5 * pa * l * l - pb * l + 0.5 * pb * trC;
+            for (int i = 0; i < 9; i++) trC = fma(F[i], F[i], trC);
+            *W = fma(0.5 * pb, trC, fma(0.5 * pa * l, l, -(pb * l)));
         }
     } else {  // pa = mu, pb = K1 (no defoEnergy: W = 0, constitutiveModels.h:91-94)
         if (W) *W = 0.0;
@@ -266,7 +270,7 @@ __device__ __forceinline__ void pk1(const double* H, double pa, double pb, doubl
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = i; j < 3; j++) {
-                B[i * 3 + j] = F[i * 3] * F[j * 3] + F[i * 3 + 1] * F[j * 3 + 1] + F[i * 3 + 2] * F[j * 3 + 2];
+                B[i * 3 + j] = dot3(F[i * 3], F[j * 3], F[i * 3 + 1], F[j * 3 + 1], F[i * 3 + 2], F[j * 3 + 2]);
                 B[j * 3 + i] = B[i * 3 + j];
             }
         const double trB = B[0] + B[4] + B[8];
@@ -274,18 +278,34 @@ __device__ __forceinline__ void pk1(const double* H, double pa, double pb, doubl
         // inlined pow (which held the FP64 Belytschko kernel at one wave per SIMD)
         const double rf1 = exp(-(5.0 / 3.0) * log_near1(J));
         const double f2 = pa * rf1;
-        const double f3 = -(pa / 3.0) * trB * rf1 + pb * (J - 1.0);
+        const double f3 = fma(-(pa / 3.0) * trB, rf1, pb * (J - 1.0));
         double sg[9];
 #pragma unroll
-        for (int i = 0; i < 9; i++) sg[i] = f2 * B[i];
-        sg[0] += f3;
-        sg[4] += f3;
-        sg[8] += f3;
+        for (int i = 0; i < 9; i++) sg[i] = (i % 4) == 0 ? fma(f2, B[i], f3) : f2 * B[i];
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = 0; j < 3; j++)
-                P[i * 3 + j] = sg[i * 3] * cF[j] + sg[i * 3 + 1] * cF[3 + j] + sg[i * 3 + 2] * cF[6 + j];
+                P[i * 3 + j] = dot3(sg[i * 3], cF[j], sg[i * 3 + 1], cF[3 + j], sg[i * 3 + 2], cF[6 + j]);
+    }
+}
+
+// FP64 from H = F - I, every law.
+template <int LAW>
+__device__ __forceinline__ void pk1(const double* H, double pa, double pb, double* P, double* W = nullptr,
+                                    double* Jout = nullptr) {
+#pragma clang fp contract(off)
+    double F[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) F[i] = H[i] + ((i % 4) == 0 ? 1.0 : 0.0);
+    if constexpr (LAW >= 2) {
+        pk1_svk_lin<double, LAW>(H, pa, pb, P);
+        if (W) {
+            *W = defo_energy(LAW, F, pa, pb);
+            *Jout = 1.0 + detIpH_m1(H);
+        }
+    } else {
+        pk1_F<LAW>(F, pa, pb, P, W, Jout);
     }
 }
 
@@ -297,6 +317,7 @@ __device__ __forceinline__ void pk1(const double* H, double pa, double pb, doubl
 // b = (mu s + lambda lnJ (1 + tr H))/J: every term is of the order of the strain.
 template <int LAW>
 __device__ __forceinline__ void pk1(const float* H, float pa, float pb, float* P) {
+#pragma clang fp contract(off)
     if (LAW >= 2) {
         pk1_svk_lin<float, LAW>(H, pa, pb, P);
         return;
@@ -305,19 +326,18 @@ __device__ __forceinline__ void pk1(const float* H, float pa, float pb, float* P
         float cH[9];
         cof3(H, cH);
         const float tr = H[0] + H[4] + H[8];
-        const float sv = (cH[0] + cH[4] + cH[8]) + (H[0] * cH[0] + H[1] * cH[1] + H[2] * cH[2]);
+        const float sv = (cH[0] + cH[4] + cH[8]) + dot3(H[0], cH[0], H[1], cH[1], H[2], cH[2]);
         const float Jm1 = tr + sv;
         const float lt = pa * log1p_fast(Jm1);
         const float rJ = rcp(1.f + Jm1);
         const float a = (pb - lt) * rJ;
-        const float b = (pb * sv + lt * (1.f + tr)) * rJ;
+        const float b = fma_t(pb, sv, lt * (1.f + tr)) * rJ;
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 3; j++) P[i * 3 + j] = pb * H[i * 3 + j] + a * (H[j * 3 + i] - cH[i * 3 + j]);
-        P[0] += b;
-        P[4] += b;
-        P[8] += b;
+            for (int j = 0; j < 3; j++)
+                P[i * 3 + j] = fma_t(pb, H[i * 3 + j], i == j ? fma_t(a, H[j * 3 + i] - cH[i * 3 + j], b)
+                                                              : a * (H[j * 3 + i] - cH[i * 3 + j]));
         return;
     }
     const float Jm1 = detIpH_m1(H);
@@ -336,24 +356,21 @@ __device__ __forceinline__ void pk1(const float* H, float pa, float pb, float* P
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = i; j < 3; j++) {
-                Bm[i * 3 + j] = H[i * 3 + j] + H[j * 3 + i] + H[i * 3] * H[j * 3] + H[i * 3 + 1] * H[j * 3 + 1] +
-                                H[i * 3 + 2] * H[j * 3 + 2];
+                Bm[i * 3 + j] = fma_t(H[i * 3 + 2], H[j * 3 + 2], fma_t(H[i * 3 + 1], H[j * 3 + 1],
+                                fma_t(H[i * 3], H[j * 3], H[i * 3 + j] + H[j * 3 + i])));
                 Bm[j * 3 + i] = Bm[i * 3 + j];
             }
         const float tr3 = (Bm[0] + Bm[4] + Bm[8]) * (1.f / 3.f);
         const float f2 = pa * __expf(-(5.f / 3.f) * lnJ);
-        const float vol = pb * Jm1 - f2 * tr3;
+        const float vol = diff2(pb, Jm1, f2, tr3);
         float sg[9];
 #pragma unroll
-        for (int i = 0; i < 9; i++) sg[i] = f2 * Bm[i];
-        sg[0] += vol;
-        sg[4] += vol;
-        sg[8] += vol;
+        for (int i = 0; i < 9; i++) sg[i] = (i % 4) == 0 ? fma_t(f2, Bm[i], vol) : f2 * Bm[i];
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
             for (int j = 0; j < 3; j++)
-                P[i * 3 + j] = sg[i * 3] * cF[j] + sg[i * 3 + 1] * cF[3 + j] + sg[i * 3 + 2] * cF[6 + j];
+                P[i * 3 + j] = dot3(sg[i * 3], cF[j], sg[i * 3 + 1], cF[3 + j], sg[i * 3 + 2], cF[6 + j]);
     }
 }
 
@@ -436,6 +453,13 @@ __device__ __forceinline__ void sqrt_n(double* v) {
     }
 }
 
+// Twice the inscribed-sphere radius 3 V / A.
+__device__ __forceinline__ double length_of(double V, double A) {
+#pragma clang fp contract(off)
+    double r = 3.0 * V / A;
+    return 2 * r;
+}
+
 // Volume term of inscribedSphereHex: |det| of the edges from node 0 to nodes 1, 3, 4 (geometry.cpp:308-355).
 __device__ __forceinline__ double hex_corner_volume(const double (*x)[3]) {
 #pragma clang fp contract(off)
@@ -463,9 +487,7 @@ __device__ __forceinline__ double hex_char_length(const double (*x)[3]) {
         double s = 0.5 * n2[2 * f] + 0.5 * n2[2 * f + 1];
         A = (f == 0) ? fabs(s) : A + fabs(s);
     }
-    double V = hex_corner_volume(x);
-    double r = 3.0 * V / A;
-    return 2 * r;
+    return length_of(hex_corner_volume(x), A);
 }
 
 // True when the element's stable dt min(l, l0)/c (l = hex_char_length(x)) is certainly above t, without
@@ -537,26 +559,35 @@ __device__ __forceinline__ bool tet_dt_above(const double (*x)[3], double l0, do
 // FP32 characteristic lengths for the precision form (the reference formulas with FP32 areas, volume and
 // ratio, hardware square root and reciprocal).  Tet: edge vectors differenced in FP64, so there is no
 // cancellation against the absolute coordinates; hex: from node positions relative to their centroid.
-__device__ __forceinline__ float area_tri_pf(const float* p, const float* q, const float* r) {
+// Norm of the cross product, twice the triangle's area.
+__device__ __forceinline__ float norm_tri_pf(const float* p, const float* q, const float* r) {
+#pragma clang fp contract(off)
     const float A0 = p[0] - r[0], A1 = p[1] - r[1], A2 = p[2] - r[2];
     const float B0 = q[0] - r[0], B1 = q[1] - r[1], B2 = q[2] - r[2];
-    const float C0 = A1 * B2 - A2 * B1, C1 = A2 * B0 - A0 * B2, C2 = A0 * B1 - A1 * B0;
-    return 0.5f * __builtin_amdgcn_sqrtf(C0 * C0 + C1 * C1 + C2 * C2);  // hardware sqrt, 1 ulp
+    const float C0 = diff2(A1, B2, A2, B1), C1 = diff2(A2, B0, A0, B2), C2 = diff2(A0, B1, A1, B0);
+    return __builtin_amdgcn_sqrtf(dot3(C0, C0, C1, C1, C2, C2));  // hardware sqrt, 1 ulp
 }
 
+// Twice the inscribed-sphere radius from the area sum A and the corner edges M (rows 0-1, 0-3, 0-4).
+__device__ __forceinline__ float hex_length_pf(const float* M, float A) {
+#pragma clang fp contract(off)
+    return 6.0f * fabsf(det3(M)) * __builtin_amdgcn_rcpf(A);
+}
 __device__ __forceinline__ float hex_char_length_pf(const float (*x)[3]) {
+#pragma clang fp contract(off)
     const int fc[6][4] = {{0, 1, 2, 3}, {4, 5, 6, 7}, {0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {0, 3, 7, 4}};
     float A = 0.0f;
 #pragma unroll
     for (int f = 0; f < 6; f++)
-        A += area_tri_pf(x[fc[f][0]], x[fc[f][1]], x[fc[f][2]]) + area_tri_pf(x[fc[f][0]], x[fc[f][2]], x[fc[f][3]]);
+        A += fma_t(0.5f, norm_tri_pf(x[fc[f][0]], x[fc[f][1]], x[fc[f][2]]),
+                   0.5f * norm_tri_pf(x[fc[f][0]], x[fc[f][2]], x[fc[f][3]]));
     float M[9];
     const int c[3] = {1, 3, 4};
 #pragma unroll
     for (int j = 0; j < 3; j++)
 #pragma unroll
         for (int d = 0; d < 3; d++) M[j * 3 + d] = x[c[j]][d] - x[0][d];
-    return 6.0f * fabsf(det3(M)) * __builtin_amdgcn_rcpf(A);
+    return hex_length_pf(M, A);
 }
 
 // Tet: from the deformed edge vectors e_j = x_{j+1} - x_0 = Jm(:,j) + Du(:,j), whose parts the element already
@@ -596,27 +627,33 @@ __device__ __forceinline__ double elem_dt(double l, double l0, double c) {
 // A[0]=xi, A[1]=eta, A[2]=zeta, A[3]=xi*eta, A[4]=eta*zeta, A[5]=xi*zeta, A[6]=xi*eta*zeta,
 // A[m] = sum_a sigma_m(a) x_a with sigma the product of the node signs.
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ void hex_butterfly1(const double* x, double* A) {  // one component
+    double s0 = x[0] + x[1], d0 = x[1] - x[0];
+    double s1 = x[3] + x[2], d1 = x[2] - x[3];
+    double s2 = x[4] + x[5], d2 = x[5] - x[4];
+    double s3 = x[7] + x[6], d3 = x[6] - x[7];
+    double ssm = s0 + s1, sdm = s1 - s0, dsm = d0 + d1, ddm = d1 - d0;
+    double ssp = s2 + s3, sdp = s3 - s2, dsp = d2 + d3, ddp = d3 - d2;
+    A[2] = ssp - ssm;
+    A[1] = sdm + sdp;
+    A[4] = sdp - sdm;
+    A[0] = dsm + dsp;
+    A[5] = dsp - dsm;
+    A[3] = ddm + ddp;
+    A[6] = ddp - ddm;
+}
 __device__ __forceinline__ void hex_butterfly(const double (*x)[3], double (*A)[3]) {
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        double s0 = x[0][d] + x[1][d], d0 = x[1][d] - x[0][d];
-        double s1 = x[3][d] + x[2][d], d1 = x[2][d] - x[3][d];
-        double s2 = x[4][d] + x[5][d], d2 = x[5][d] - x[4][d];
-        double s3 = x[7][d] + x[6][d], d3 = x[6][d] - x[7][d];
-        double ssm = s0 + s1, sdm = s1 - s0, dsm = d0 + d1, ddm = d1 - d0;
-        double ssp = s2 + s3, sdp = s3 - s2, dsp = d2 + d3, ddp = d3 - d2;
-        A[2][d] = ssp - ssm;
-        A[1][d] = sdm + sdp;
-        A[4][d] = sdp - sdm;
-        A[0][d] = dsm + dsp;
-        A[5][d] = dsp - dsm;
-        A[3][d] = ddm + ddp;
-        A[6][d] = ddp - ddm;
+        double y[8], C[7];
+#pragma unroll
+        for (int a = 0; a < 8; a++) y[a] = x[a][d];
+        hex_butterfly1(y, C);
+#pragma unroll
+        for (int m = 0; m < 7; m++) A[m][d] = C[m];
     }
 }
 
-__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
 // The last two levels of the inverse transform from the pair sums and differences t.. (shared by both forms below).
 template <typename T>
@@ -828,6 +865,57 @@ __device__ __forceinline__ void hex_jac(const T (*A)[3], const GpSigns<T>& s, T*
     }
 }
 
+// At a Gauss point, from J and the displacement gradient Du in natural coordinates: cof(J), det J, 1/det J and
+// H = Du J^-1, H(i,j) = sum_k Du(i,k) cof(J)(j,k) / det J; Fd: the diagonal of F = I + H, rounded once.
+template <typename T>
+__device__ __forceinline__ void hex_grad(const T* Jm, const T* Du, T* cJ, T* H, T* Fd, T* dJ, T* rJ) {
+#pragma clang fp contract(off)
+    cof3(Jm, cJ);
+    *dJ = dot3(Jm[0], cJ[0], Jm[1], cJ[1], Jm[2], cJ[2]);
+    *rJ = rcp(*dJ);
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            const T m = dot3(Du[i * 3], cJ[j * 3], Du[i * 3 + 1], cJ[j * 3 + 1], Du[i * 3 + 2], cJ[j * 3 + 2]);
+            H[i * 3 + j] = m * *rJ;
+            if (i == j) Fd[i] = fma_t(m, *rJ, T(1));
+        }
+}
+
+// Stress at a hex8 Gauss point from hex_grad's H and Fd.
+template <int LAW>
+__device__ __forceinline__ void hex_pk1(const double* H, const double* Fd, double pa, double pb, double* P,
+                                        double* W = nullptr, double* Jout = nullptr) {
+    if constexpr (LAW < 2) {
+        const double F[9] = {Fd[0], H[1], H[2], H[3], Fd[1], H[5], H[6], H[7], Fd[2]};
+        pk1_F<LAW>(F, pa, pb, P, W, Jout);
+    } else {
+        pk1<LAW>(H, pa, pb, P, W, Jout);
+    }
+}
+template <int LAW>
+__device__ __forceinline__ void hex_pk1(const float* H, const float*, float pa, float pb, float* P) {
+    pk1<LAW>(H, pa, pb, P);
+}
+
+// Columns Q[k][i] of wJ P J^-T: weight 1 (GPsDistribution.cpp:392-432), so wJ J^-T = sign(det J) cof(J) and
+// Q(i,k) = sign(det J) sum_J P(i,J) cof(J)(J,k).  The sign is folded into P only when some lane of the wave has
+// det J <= 0 (a positively oriented mesh never takes that branch).
+template <typename T>
+__device__ __forceinline__ void hex_stress_columns(T* P, const T* cJ, T dJ, T (*Q)[3]) {
+#pragma clang fp contract(off)
+    if (!__all(dJ > T(0))) {
+        const T sg = dJ < T(0) ? T(-1) : T(1);
+#pragma unroll
+        for (int i = 0; i < 9; i++) P[i] *= sg;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int k = 0; k < 3; k++) Q[k][i] = dot3(P[i * 3], cJ[k], P[i * 3 + 1], cJ[3 + k], P[i * 3 + 2], cJ[6 + k]);
+}
+
 // ---------------------------------------------------------------------------
 // Hex8 element: nodal forces f[a][i] (T) and the element dt contribution (FP64).
 // VISC adds bulk viscosity from the displacement increment u - uprev over the step (rdt = 1/dt, 0 when
@@ -905,29 +993,20 @@ __device__ __forceinline__ double hex8_element(const MpsInst& I, int e, const do
     for (int gp = 0; gp < 8; gp++) {
         // Gauss point signs in the reference order (GPsDistribution.cpp:392-432)
         const GpSigns<T> s = gp_signs<T>(gp);
-        T Jm[9], Du[9], H[9], P[9];
+        T cJ[9], P[9], Q[3][3], dJ, rJ;
+        T Jm[9], Du[9], H[9], Fd[3];
         hex_jac<T>(Ax, s, Jm);
         hex_jac<T>(Au, s, Du);
-        // J^-1 = cof(J)^T / det J ; weight 1 (GPsDistribution.cpp:392-432) so wJ J^-T = sign(det J) cof(J)
-        T cJ[9];
-        cof3(Jm, cJ);
-        const T dJ = Jm[0] * cJ[0] + Jm[1] * cJ[1] + Jm[2] * cJ[2];
-        const T rJ = rcp(dJ);
-        // H = Du J^-1: H(i,j) = sum_k Du(i,k) cof(J)(j,k) / det J
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int j = 0; j < 3; j++)
-                H[i * 3 + j] = (Du[i * 3] * cJ[j * 3] + Du[i * 3 + 1] * cJ[j * 3 + 1] + Du[i * 3 + 2] * cJ[j * 3 + 2]) * rJ;
+        hex_grad<T>(Jm, Du, cJ, H, Fd, &dJ, &rJ);
         if constexpr (EN) {  // weight 1: wJ = |det J| (classGPs.cpp:26-27)
             double Wg, Jg;
-            pk1<LAW>(H, tpa, tpb, P, &Wg, &Jg);
+            hex_pk1<LAW>(H, Fd, tpa, tpb, P, &Wg, &Jg);
             const double wJ = fabs(dJ);
-            e_def += Wg * wJ;
-            e_vol += wJ * Jg;
+            e_def = fma(Wg, wJ, e_def);
+            e_vol = fma(wJ, Jg, e_vol);
             vs[gp * MPS_PATCH] = wJ;
         } else {
-            pk1<LAW>(H, tpa, tpb, P);
+            hex_pk1<LAW>(H, Fd, tpa, tpb, P);
         }
         if (VISC) {  // tr of grad(u - uprev) = sum_ik Dd(i,k) cof(J)(i,k) / det J
             // the memory clobber keeps the 21 LDS reads at each Gauss point: hoisted out of the loop
@@ -946,19 +1025,7 @@ __device__ __forceinline__ double hex8_element(const MpsInst& I, int e, const do
             }
             add_bulk_visc<T>(H, tr * rJ * trs, qa, qb, P);
         }
-        // Q = wJ P J^-T: Q(i,k) = sign(det J) sum_J P(i,J) cof(J)(J,k); columns Q(:,k).  The sign is
-        // folded into P only when some lane of the wave has det J <= 0 (a positively oriented
-        // mesh never takes that branch).
-        if (!__all(dJ > T(0))) {
-            const T sg = dJ < T(0) ? T(-1) : T(1);
-#pragma unroll
-            for (int i = 0; i < 9; i++) P[i] *= sg;
-        }
-        T Q[3][3];
-#pragma unroll
-        for (int i = 0; i < 3; i++)
-#pragma unroll
-            for (int k = 0; k < 3; k++) Q[k][i] = P[i * 3] * cJ[k] + P[i * 3 + 1] * cJ[3 + k] + P[i * 3 + 2] * cJ[6 + k];
+        hex_stress_columns<T>(P, cJ, dJ, Q);
         // moment sums, one FMA per (moment, column) pair: a +-1 factor makes each product exact
 #pragma unroll
         for (int i = 0; i < 3; i++) {
@@ -1015,6 +1082,19 @@ __device__ __forceinline__ TetConsts tet_consts(const MpsInst& I, int e, bool wa
     asm volatile("" : "+v"(k.c));
     k.l0 = want_dt ? I.l0[e] : 0.0;
     return k;
+}
+
+// A staged node of the tet4 kernel: X and u of the patch's j-th distinct node at sxu[6j..6j+5], read as three
+// 16-byte pieces (one address per node, the pieces at fixed offsets from it).
+__device__ __forceinline__ void staged_node(const double* __restrict__ sxu, int j, double* x, double* u) {
+    const double2* s = reinterpret_cast<const double2*>(sxu + 6 * j);
+    const double2 a = s[0], b = s[1], c = s[2];
+    x[0] = a.x;
+    x[1] = a.y;
+    x[2] = b.x;
+    u[0] = b.y;
+    u[1] = c.x;
+    u[2] = c.y;
 }
 
 // tet4_core takes the element's node coordinates x, displacements uu and constants; nd (node ids) is
@@ -1095,6 +1175,32 @@ __device__ __forceinline__ double tet4_core(const MpsInst& I, int e, const int* 
         for (int i = 0; i < 3; i++)
             f[a][i] = wJ * P[i * 3] * dphi[a][0] + wJ * P[i * 3 + 1] * dphi[a][1] + wJ * P[i * 3 + 2] * dphi[a][2];
     return dte;
+}
+
+// Stable dt of a tet4 element alone, as tet4_core and the staged kernel take it: strict FP64 length from the deformed
+// positions, or FP32 length from the edge vectors.
+template <typename T>
+__device__ __forceinline__ double tet_dt(const double (*x)[3], const double (*uu)[3], const TetConsts& k) {
+    double l;
+    if constexpr (sizeof(T) == 8) {
+        double xd[4][3];
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) xd[a][d] = x[a][d] + uu[a][d];
+        l = tet_char_length(xd);
+    } else {
+        T Jm[9], Du[9];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                Jm[i * 3 + j] = (T)(x[j + 1][i] - x[0][i]);
+                Du[i * 3 + j] = (T)(uu[j + 1][i] - uu[0][i]);
+            }
+        l = (double)tet_char_length_f32(Jm, Du);
+    }
+    return elem_dt(l, k.l0, k.c);
 }
 
 // Kinetic energy of tet4 element e at its Gauss point (dataExtraction.cpp:631-707): wJ rho/2 |v(gp)|^2 with
@@ -1259,6 +1365,11 @@ __device__ __forceinline__ void node_fext(const MpsInst& I, int n, uint32_t info
     }
 }
 
+__device__ __forceinline__ double node_fext1(const MpsInst& I, int n, uint32_t info, int i) {
+    if (info & MPS_NODE_LOADED) return I.lf[3 * (size_t)I.lidx[n] + i];
+    return (i == 2 && I.fgrav) ? I.fgrav[n] : 0.0;
+}
+
 // Surface forces of pressure Gauss point q at time t (BCsPressureRamp / BCsPressureInst,
 // boundaryConditions.cpp:370-496): F of the bulk element at the point (classSpatialPoint::getF,
 // classSpatialPoint.cpp:41-68: node terms first, then the identity), J = det F, n = F^-T n0, and
@@ -1391,25 +1502,26 @@ __device__ __forceinline__ void node_rhs(const double* fi, const double* fe, dou
 // the previous step (its velocity on constrained DOFs); rhs = -fint + fext of the node (read for free DOFs
 // only).  With wkin, 1/2 m (V^2 - w^2) of each constrained DOF, whose velocity the prescribed V replaces, is
 // added to *wkin.
+__device__ __forceinline__ void node_update1(const MpsInst& I, uint32_t info, int i, long long k, double dt, double m,
+                                             double rhs, double w, double* v, double* a, double* wkin = nullptr) {
+#pragma clang fp contract(off)
+    if ((info >> i) & 1u) {
+        double U, V;
+        bc_motion(I, I.bcval[3 * (size_t)((info & MPS_REC_MASK) >> 3) + i], k, dt, &U, &V);
+        if (wkin) *wkin += 0.5 * m * (V * V - w * w);
+        *v = V;
+        *a = 0.;
+    } else {
+        const double an = (m != 0.0) ? rhs / m : 0.0;
+        *v = half_velocity(dt, w, an);
+        *a = an;
+    }
+}
 __device__ __forceinline__ void node_update(const MpsInst& I, uint32_t info, long long k, double dt, double m,
                                             const double* rhs, const double* w, double* v, double* a,
                                             double* wkin = nullptr) {
-#pragma clang fp contract(off)
-    const uint32_t mask = info & 7u;
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-        if ((mask >> i) & 1u) {
-            double U, V;
-            bc_motion(I, I.bcval[3 * (size_t)((info & MPS_REC_MASK) >> 3) + i], k, dt, &U, &V);
-            if (wkin) *wkin += 0.5 * m * (V * V - w[i] * w[i]);
-            v[i] = V;
-            a[i] = 0.;
-        } else {
-            const double an = (m != 0.0) ? rhs[i] / m : 0.0;
-            v[i] = half_velocity(dt, w[i], an);
-            a[i] = an;
-        }
-    }
+    for (int i = 0; i < 3; i++) node_update1(I, info, i, k, dt, m, rhs[i], w[i], v + i, a + i, wkin);
 }
 
 // Gather + lumped-mass solve of node n at step k (node_partial_sum, node_fext, node_update): v, a of the step
@@ -1499,14 +1611,19 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
 __device__ __forceinline__ unsigned long long umin64(unsigned long long a, unsigned long long b) { return b < a ? b : a; }
 
 // Stable-dt reduction slots (MpsInst::dtred): workgroups atomicMin into one of MPS_DT_SLOTS slots of the
-// step parity, 256 B apart, so that thousands of workgroups do not queue on one address.
+// step's parity, 256 B apart, so that thousands of workgroups do not queue on one address.
+__device__ __forceinline__ int dt_parity(long long k) { return (int)(k & 1); }
+// Slot s of set q of the spread form.
+__device__ __forceinline__ unsigned long long* dt_spread(const MpsInst& I, int q, int s) {
+    return I.dtred + MPS_DT_WORDS + MPS_DT_COUNT_WORDS + (size_t)(q * MPS_DT_SLOTS + s) * MPS_DT_STRIDE;
+}
 __device__ __forceinline__ unsigned long long* dt_slot(const MpsInst& I, int parity, int s) {
     return I.dtred + (size_t)(parity * MPS_DT_SLOTS + s) * MPS_DT_STRIDE;
 }
 // Certificate counters (single-instance form): s < MPS_DT_SLOTS counts the element-kernel workgroups b with
 // b % MPS_DT_SLOTS == s that are done, s = MPS_DT_SLOTS the residues whose workgroups are all done.
 __device__ __forceinline__ unsigned int* dt_count(const MpsInst& I, int s) {
-    return reinterpret_cast<unsigned int*>(I.dtred + (size_t)(2 * MPS_DT_SLOTS + s) * MPS_DT_STRIDE);
+    return reinterpret_cast<unsigned int*>(I.dtred + MPS_DT_WORDS + (size_t)s * MPS_DT_STRIDE);
 }
 // Min over the slots of one parity, returned in every lane; all 64 lanes of the wave must call it.
 __device__ __forceinline__ unsigned long long dt_read_min(const MpsInst& I, int parity) {

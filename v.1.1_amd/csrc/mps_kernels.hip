@@ -204,10 +204,10 @@ __device__ void dt_certify(const MpsInst& I, long long k, double dtsk, unsigned 
     if (!last) return;
     __threadfence();
     if (threadIdx.x < 64) {  // wave 0 decides for the workgroup
-        unsigned long long m = dt_read_min_now(I, (k + 1) & 1);
+        unsigned long long m = dt_read_min_now(I, dt_parity(k + 1));
         for (int t = 0; t < 8 && !(bits2d(m) <= dtsk); t++) {
             __builtin_amdgcn_s_sleep(127);
-            m = dt_read_min_now(I, (k + 1) & 1);
+            m = dt_read_min_now(I, dt_parity(k + 1));
         }
         if (threadIdx.x == 0) fail = !(bits2d(m) <= dtsk);
     }
@@ -217,7 +217,7 @@ __device__ void dt_certify(const MpsInst& I, long long k, double dtsk, unsigned 
         for (int e = threadIdx.x; e < I.Ne; e += blockDim.x) mm = umin64(mm, d2bits(elem_dt_exact<NEN, O32>(I, e)));
         mm = block_min_u64(mm, sh);
         if (threadIdx.x == 0) {
-            atomicMin(dt_slot(I, (k + 1) & 1, 0), mm);
+            atomicMin(dt_slot(I, dt_parity(k + 1), 0), mm);
             I.ctl->skip_hold = k + 1 + MPS_DT_SKIP_HOLD;
         }
     }
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(MPS_PATCH) __attribute__((amdgpu_waves_per_eu(VISC 
                                                                                     rdt, eflags, env, swj, dtsk);
     if (mode == 0) {
         m = block_min_u64(m, sh);
-        if (threadIdx.x == 0) atomicMin(dt_slot(I, (k + 1) & 1, blockIdx.x & (MPS_DT_SLOTS - 1)), m);
+        if (threadIdx.x == 0) atomicMin(dt_slot(I, dt_parity(k + 1), blockIdx.x & (MPS_DT_SLOTS - 1)), m);
         if constexpr (EN) {
             // hex8 kinetic energy of the current v, after the force phase and its barriers: kept apart from the
             // force arithmetic, whose compiled form (and rounding) it would otherwise share a basic block with
@@ -283,19 +283,6 @@ __global__ __launch_bounds__(MPS_PATCH) __attribute__((amdgpu_waves_per_eu(VISC 
 __host__ __device__ __forceinline__ size_t tet_shared_bytes(int pu, int tsize) {
     const size_t a = 48 * (size_t)pu, b = 12 * (size_t)MPS_PATCH * tsize;
     return a > b ? a : b;
-}
-
-// A staged node of the tet4 kernel: X and u of the patch's j-th distinct node at sxu[6j..6j+5], read as three
-// 16-byte pieces (one address per node, the pieces at fixed offsets from it).
-__device__ __forceinline__ void staged_node(const double* __restrict__ sxu, int j, double* x, double* u) {
-    const double2* s = reinterpret_cast<const double2*>(sxu + 6 * j);
-    const double2 a = s[0], b = s[1], c = s[2];
-    x[0] = a.x;
-    x[1] = a.y;
-    x[2] = b.x;
-    u[0] = b.y;
-    u[1] = c.x;
-    u[2] = c.y;
 }
 
 // Tet4 element kernel with node staging (inviscid).  Each block first loads the U_p distinct nodes of
@@ -404,7 +391,7 @@ __global__ __launch_bounds__(MPS_PATCH) __attribute__((amdgpu_waves_per_eu(sizeo
     patch_sums<T, 4, MPS_PATCH, true>(I, p, sf, spc, I.prow + base + p);
     if (mode == 0) {
         dmin = block_min_u64(dmin, sh);
-        if (threadIdx.x == 0) atomicMin(dt_slot(I, (k + 1) & 1, blockIdx.x & (MPS_DT_SLOTS - 1)), dmin);
+        if (threadIdx.x == 0) atomicMin(dt_slot(I, dt_parity(k + 1), blockIdx.x & (MPS_DT_SLOTS - 1)), dmin);
         if constexpr (EN) elem_energy_publish(I, env, smem);
         if constexpr (SKIP) dt_certify<4, false>(I, k, dtsk, sh);
     }
@@ -443,7 +430,7 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) void k_
         if (I.ctl->slot[k & 1].go) {
             unsigned long long m = patch_forces<T, NEN, LAW, BS>(I, W.begin / MPS_PATCH, true, sf, nullptr, nullptr);
             m = block_min_u64(m, sh);
-            if (threadIdx.x == 0) atomicMin(dt_slot(I, (k + 1) & 1, w & (MPS_DT_SLOTS - 1)), m);
+            if (threadIdx.x == 0) atomicMin(dt_slot(I, dt_parity(k + 1), w & (MPS_DT_SLOTS - 1)), m);
         }
         __syncthreads();
     }
@@ -490,11 +477,11 @@ __device__ __forceinline__ bool node_item(const MpsInst& I, int n, bool first, i
     MpsStepSlot nx;
     nx.go = 0;
     int st = MPSD_RUNNING;
-    const unsigned long long mb = fuse ? dt_read_min(I, (k + 1) & 1) : 0ull;
+    const unsigned long long mb = fuse ? dt_read_min(I, dt_parity(k + 1)) : 0ull;
     if (fuse) st = begin_scalars(I, k + 1, s, mb, &nx);
     if (first) {
         ctl->A = k + 1;
-        dt_reset(I, k & 1);
+        dt_reset(I, dt_parity(k));
         if (fuse) {
             ctl->dt_skip = dt_skip_next(I, k + 1, mb);
             ctl->slot[(k + 1) & 1] = nx;
@@ -686,7 +673,7 @@ __device__ __forceinline__ void begin_item(const MpsInst& I, int n, bool first) 
     const long long k = ctl->A;
     const MpsStepSlot prev = ctl->slot[(k - 1) & 1];
     MpsStepSlot nx;
-    const unsigned long long mb = dt_read_min(I, k & 1);
+    const unsigned long long mb = dt_read_min(I, dt_parity(k));
     const int st = begin_scalars(I, k, prev, mb, &nx);
     if (first) {
         ctl->dt_skip = dt_skip_next(I, k, mb);

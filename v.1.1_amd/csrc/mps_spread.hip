@@ -1,0 +1,610 @@
+// mps_spread.hip -- the spread form of the explicit step, for meshes that leave most of the chip idle.
+//
+// A small mesh is bound by latency, not by throughput: in the patch form (mps_kernels.hip) a step of 1,000 hex8 elements
+// takes as long as one of 30,000, about 19 us, of which 14 us is one wavefront walking through 2,700 instructions per
+// element and 5 us the node kernel's chain of dependent loads.  Here a step is ONE launch (a launch in a replayed graph
+// costs 1.6 us, no more than a grid barrier among as many workgroups), and the element work is spread over idle lanes:
+//   - workgroup b first brings the distinct nodes of its elements to step k: it sums the element forces of step k-1 at
+//     each node, solves step k-1 and predicts u_k, for every node it needs (a node shared by several workgroups is
+//     updated by each of them, with the same bits; its owner writes it back).  u and the half-step velocity w are
+//     double-buffered, since neighbours still read the old ones;
+//   - then it computes the forces of its elements from the nodes in LDS -- eight lanes per hex8 element, one Gauss point
+//     each -- and writes every nodal force to its place in node order, so that the next step reads each node's forces as
+//     one contiguous run.  A second wave takes the stable dt meanwhile, exact for every element: no skip, no certificate.
+// Two dependent global loads are left (tables and control; state and forces), about 1 us each, then 1.4 us of element
+// work.  Every sum keeps the patch form's order -- the forces of a node are added per patch of MPS_PATCH elements and then
+// over the patches -- and an element's arithmetic is the same function by function, so both forms give the same bits.
+//
+// Measured, us per step, patch form / here.  hex8 FP64: 1,000 elements 19.0 / 5.6, 8,000 19.4 / 7.2, 15,600 19.9 / 9.9,
+// 29,800 19.9 / 16.4, 64,000 21.0 / 29.4; FP32 form: 1,000 15.9 / 5.6, 15,600 16.7 / 9.1, 29,800 16.9 / 14.3; tet4 FP64:
+// 750 13.6 / 6.8, 10,400 12.9 / 6.8, 48,000 13.8 / 10.0, 93,800 14.6 / 18.0; FP32 form: 10,400 10.5 / 6.8, 48,000 11.3 /
+// 10.2, 93,800 12.0 / 16.7.  Every node is updated by all the workgroups that hold it (4.5 per 8 hex8 elements where the
+// patch form has 1.03 per element), so past the size where the lanes are no longer idle the patch form is the better one.
+// Tried: 16 and 32 hex8 elements per workgroup: fewer shared nodes, but 0.4 to 1.8 us more up to 2,000 elements and
+// nothing gained above.
+#include "../../include/mps_gpu.h"
+#include "mps_device.h"
+#include "mps_kernels.h"
+
+using namespace mpsd;
+
+namespace {
+
+// LDS of the hex8 element phase, in values of T per element: butterfly coefficients of X and u (42), later the moment
+// sums (21); stress columns of the eight points (72); face triangle areas (12); FP32 node positions (24).  Coefficients
+// and columns are read in 16-byte pieces; with these strides the eight elements of a wave fall into different banks.
+constexpr int kCoef = 44, kCol = 76, kArea = 12, kPos = 24;
+
+// LDS exchange between the lanes of one wavefront: LDS operations of a wave stay in order, so only the compiler has to
+// be kept from moving them.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Buffers of u and w: index 0 the solve's own arrays (u, v holding w), 1 the alternate ones.  The step with index ci in
+// its launch sequence reads buffer ci & 1 and writes the other; index 0 finds v and a.
+__device__ __forceinline__ void uw_buffers(const MpsInst& I, int which, double** u, double** w) {
+    *u = which ? I.sp_uw : I.u;
+    *w = which ? I.sp_uw + 3 * (size_t)I.N : I.v;
+}
+
+// Element forces of the step with index ci in its launch sequence.
+template <typename T>
+__device__ __forceinline__ T* spread_forces(const MpsInst& I, int ci) {
+    return reinterpret_cast<T*>(I.sp_f) + (ci & 1 ? 3 * (size_t)I.nen * I.Ne : 0);
+}
+
+// What the update of one node in one direction reads, loaded before any of it is used.  At index 0 of a sequence w and m
+// are v and a, and the forces are not used.
+template <typename T, int FLIGHT>
+struct NodeLoads {
+    double X, u, w, m;
+    uint32_t info;
+    T c[FLIGHT];  // the first element forces
+    __device__ __forceinline__ void load(const MpsInst& I, const int4& E, int d, bool first, const double* __restrict__ ur,
+                                         const double* __restrict__ wr, const T* __restrict__ f) {
+        const int n = E.x & 0x7FFFFFFF;
+        const size_t i = (size_t)d * I.N + n;
+        X = I.X[i];
+        u = ur[i];
+        w = wr[i];  // (at index 0 the buffer is v)
+        m = *(first ? I.a + i : I.mass + n);
+        info = I.ninfo[n];
+        const T* p = f + 3 * (size_t)E.y + d;
+#pragma unroll
+        for (int q = 0; q < FLIGHT; q++) c[q] = p[3 * min(q, E.z - 1)];
+    }
+    // Internal force of the node in direction d: its entries added per patch (end bits E.w), then over the patches --
+    // the order and the roundings of patch_sums and node_partial_sum.  Without branches: entries past the end add 0.0 to
+    // sums that are never -0.0.
+    __device__ __forceinline__ double force(const int4& E, const T* __restrict__ f, int d) {
+#pragma clang fp contract(off)
+        double fi = 0.0, s = 0.0;
+        for (int q0 = 0; q0 < E.z; q0 += FLIGHT) {
+            if (q0 > 0) {
+                const T* p = f + 3 * (size_t)E.y + d;
+#pragma unroll
+                for (int q = 0; q < FLIGHT; q++) c[q] = p[3 * min(q0 + q, E.z - 1)];
+            }
+#pragma unroll
+            for (int q = 0; q < FLIGHT; q++) {
+                s += q0 + q < E.z ? (double)c[q] : 0.0;
+                const bool end = ((uint32_t)E.w >> (q0 + q)) & 1u;  // q0 + q <= 31
+                fi += end ? (sizeof(T) == 4 ? (double)(float)s : s) : 0.0;
+                s = end ? 0.0 : s;
+            }
+        }
+        return fi;
+    }
+};
+
+// Min over the 16 lanes of a row, in every lane of it, by DPP rotations (a shuffle goes through LDS and takes several
+// times as long).
+template <int ROT>
+__device__ __forceinline__ unsigned long long row_min_step(unsigned long long v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)v, 0x120 + ROT, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(v >> 32), 0x120 + ROT, 0xf, 0xf, false);
+    return umin64(v, ((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ unsigned long long row_min(unsigned long long v) {
+    static_assert(MPS_DT_SLOTS == 16, "one slot per lane of a row");
+    return row_min_step<1>(row_min_step<2>(row_min_step<4>(row_min_step<8>(v))));
+}
+__device__ __forceinline__ void spread_reset(const MpsInst& I, int q) {
+#pragma unroll
+    for (int s = 0; s < MPS_DT_SLOTS; s++) *dt_spread(I, q, s) = 0x7FF0000000000000ull;
+}
+
+__device__ __forceinline__ void check_finite(const MpsInst& I, int n, int d, long long k, double u) {
+    if (n == I.dof1_node && d == I.dof1_dir && !isfinite(u)) {
+        I.ctl->nonfinite = 1;
+        atomicMin((unsigned long long*)&I.ctl->nan_step, (unsigned long long)k);
+    }
+}
+
+// Vertices of the face triangles of hex_char_length: triangle t = (p, q, r), three bits each.
+__device__ __forceinline__ int hex_triangle(int t) {
+    constexpr int fc[6][4] = {{0, 1, 2, 3}, {4, 5, 6, 7}, {0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {0, 3, 7, 4}};
+    unsigned long long lo = 0, hi = 0;
+#pragma unroll
+    for (int f = 0; f < 6; f++)
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const unsigned long long c = fc[f][0] | fc[f][1 + h] << 3 | fc[f][2 + h] << 6;
+            if (f < 3) lo |= c << (9 * (2 * f + h));
+            else hi |= c << (9 * (2 * (f - 3) + h));
+        }
+    return (int)((t < 6 ? lo >> (9 * t) : hi >> (9 * (t - 6))) & 511u);
+}
+
+// The unscaled inverse butterfly of coefficient vectors R for node a alone (hex_unbutterfly, same operations).
+template <typename T>
+__device__ __forceinline__ void unbutterfly_node(int a, const T* tss, const T* tsd, const T* tds, const T* tdd, T* f) {
+#pragma clang fp contract(off)
+    const T ys = unit_signed(T(), ((a >> 1) & 1) ^ 1), xs = unit_signed(T(), ((a ^ (a >> 1)) & 1) ^ 1);
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const T us = fma_t(ys, tsd[d], tss[d]), ud = fma_t(ys, tdd[d], tds[d]);
+        f[d] = fma_t(xs, ud, us);
+    }
+}
+
+// n values of T (a multiple of 16 bytes) from LDS in 16-byte pieces.
+template <int N, typename T>
+__device__ __forceinline__ void lds_read(const T* __restrict__ p, T* v) {
+    constexpr int V = 16 / sizeof(T);
+    struct alignas(16) Piece { T x[V]; };
+    const Piece* q = reinterpret_cast<const Piece*>(p);
+#pragma unroll
+    for (int i = 0; i < N / V; i++) {
+        const Piece t = q[i];
+#pragma unroll
+        for (int k = 0; k < V; k++) v[i * V + k] = t.x[k];
+    }
+}
+
+// Forces of a hex8 element by its eight lanes: lane j takes component j of the butterflies (j < 6), Gauss point j, its
+// share of the moment sums and node j.  sn: staged node values [9][ss] (X, u, X + u); lx: the element's local node indices.
+template <typename T>
+__device__ __forceinline__ void hex_coefficients(const double* __restrict__ sn, int ss, const uint16_t* __restrict__ lx,
+                                                 T* __restrict__ sc, int j) {
+#pragma clang fp contract(off)
+    if (j < 6) {
+        const double* s = sn + j * ss;
+        double x[8], A[7];
+#pragma unroll
+        for (int a = 0; a < 8; a++) x[a] = s[lx[a]];
+        hex_butterfly1(x, A);
+        const double g = MPS_GP;
+        T* c = sc + (j < 3 ? j : 18 + j);
+        c[0] = (T)(0.125 * A[0]);
+        c[3] = (T)(0.125 * A[1]);
+        c[6] = (T)(0.125 * A[2]);
+        c[9] = (T)((0.125 * g) * A[3]);
+        c[12] = (T)((0.125 * g) * A[4]);
+        c[15] = (T)((0.125 * g) * A[5]);
+        c[18] = (T)((0.125 * g * g) * A[6]);
+    }
+}
+template <typename T, int LAW>
+__device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restrict__ sq, int j, double pa, double pb, T* f) {
+#pragma clang fp contract(off)
+    {  // Gauss point j
+        T A[44];
+        lds_read<44>(sc, A);
+        const T(*Ax)[3] = reinterpret_cast<const T(*)[3]>(A);
+        const T(*Au)[3] = reinterpret_cast<const T(*)[3]>(A + 21);
+        const GpSigns<T> s = gp_signs<T>(j);
+        T Jm[9], Du[9], cJ[9], H[9], Fd[3], P[9], Q[3][3], dJ, rJ;
+        hex_jac<T>(Ax, s, Jm);
+        hex_jac<T>(Au, s, Du);
+        hex_grad<T>(Jm, Du, cJ, H, Fd, &dJ, &rJ);
+        hex_pk1<LAW>(H, Fd, (T)pa, (T)pb, P);
+        hex_stress_columns<T>(P, cJ, dJ, Q);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int i = 0; i < 3; i++) sq[i * 24 + j * 3 + k] = Q[k][i];
+    }
+    wave_sync();
+    // Moment sums over the points in order, with the roundings of hex8_element (its products with +-1 are exact, so
+    // that its FMAs add and subtract): lanes 0-2 the sums 0, 1, 2, 6 of their component, lanes 3-5 the sums 3, 4, 5.
+    if (j < 6) {
+        const int i = j < 3 ? j : j - 3;
+        T q[24];
+        lds_read<24>(sq + 24 * i, q);
+        T G[4] = {T(0), T(0), T(0), T(0)};
+        if (j < 3) {
+#pragma unroll
+            for (int gp = 0; gp < 8; gp++) {
+                const T x = T(sxi(gp)), y = T(seta(gp)), z = T(szeta(gp));
+                G[0] += q[3 * gp];
+                G[1] += q[3 * gp + 1];
+                G[2] += q[3 * gp + 2];
+                G[3] = fma_t(x * y, q[3 * gp + 2], fma_t(x * z, q[3 * gp + 1], fma_t(y * z, q[3 * gp], G[3])));
+            }
+        } else {
+#pragma unroll
+            for (int gp = 0; gp < 8; gp++) {
+                const T x = T(sxi(gp)), y = T(seta(gp)), z = T(szeta(gp));
+                G[0] = fma_t(x, q[3 * gp + 1], fma_t(y, q[3 * gp], G[0]));
+                G[1] = fma_t(y, q[3 * gp + 2], fma_t(z, q[3 * gp + 1], G[1]));
+                G[2] = fma_t(x, q[3 * gp + 2], fma_t(z, q[3 * gp], G[2]));
+            }
+        }
+        T* g = sc + i + (j < 3 ? 0 : 9);
+        g[0] = G[0];
+        g[3] = G[1];
+        g[6] = G[2];
+        if (j < 3) g[18] = G[3];
+    }
+    wave_sync();
+    {  // force at node j: hex_unbutterfly_scaled for one node
+        T g[24];
+        lds_read<24>(sc, g);
+        const T s1 = (T)0.125, s2 = (T)(0.125 * MPS_GP), s3 = (T)(0.125 * MPS_GP * MPS_GP);
+        const T zs = unit_signed(T(), (j >> 2) ^ 1);
+        T tss[3], tsd[3], tds[3], tdd[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            tss[d] = zs * (g[6 + d] * s1);
+            tsd[d] = fma_t(g[3 + d], s1, zs * (g[12 + d] * s2));
+            tds[d] = fma_t(g[d], s1, zs * (g[15 + d] * s2));
+            tdd[d] = fma_t(g[9 + d], s2, zs * (g[18 + d] * s3));
+        }
+        unbutterfly_node<T>(j, tss, tsd, tds, tdd, f);
+    }
+}
+
+// Stable dt of the eight elements of a force wave, by a wave of their own: the 96 face triangles over its lanes, then one
+// lane per element.  sc: the elements' coefficients (FP32 form), sp: their node positions (FP32 form).  Returns the
+// element's dt in lanes 0-7.
+template <typename T>
+__device__ __forceinline__ double hex_spread_dt(const double* __restrict__ sn, int ss, const uint16_t* __restrict__ slx,
+                                                const T* __restrict__ sc, T* __restrict__ sa, T* __restrict__ sp, int lane,
+                                                double c, double l0) {
+#pragma clang fp contract(off)
+    if constexpr (sizeof(T) == 4) {  // node positions relative to the centroid (hex8_element), node j of element el
+        const int el = lane >> 3, j = lane & 7;
+        T A[44];
+        lds_read<44>(sc + el * kCoef, A);
+        const T ig = (T)(1.0 / MPS_GP), ig2 = (T)(1.0 / (MPS_GP * MPS_GP));
+        const T zs = unit_signed(T(), (j >> 2) ^ 1);
+        T tss[3], tsd[3], tds[3], tdd[3], x[3];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            tss[d] = zs * (A[6 + d] + A[27 + d]);
+            tsd[d] = (A[3 + d] + A[24 + d]) + zs * ((A[12 + d] + A[33 + d]) * ig);
+            tds[d] = (A[d] + A[21 + d]) + zs * ((A[15 + d] + A[36 + d]) * ig);
+            tdd[d] = (A[9 + d] + A[30 + d]) * ig + zs * ((A[18 + d] + A[39 + d]) * ig2);
+        }
+        unbutterfly_node<T>(j, tss, tsd, tds, tdd, x);
+#pragma unroll
+        for (int d = 0; d < 3; d++) sp[el * kPos + j * 3 + d] = x[d];
+        wave_sync();
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int it = lane + 64 * r;
+        if (it < 96) {
+            const int el = it / 12, t = it - 12 * el, code = hex_triangle(t);
+            T p[3][3];
+#pragma unroll
+            for (int v = 0; v < 3; v++) {
+                const int a = (code >> (3 * v)) & 7;
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+                    p[v][d] = sizeof(T) == 8 ? (T)sn[(6 + d) * ss + slx[el * 8 + a]] : sp[el * kPos + a * 3 + d];
+            }
+            if constexpr (sizeof(T) == 8) {
+                double n2 = tri_norm2(p[0], p[1], p[2]);
+                sqrt_n<1>(&n2);
+                sa[it] = 0.5 * n2;
+            } else {
+                sa[it] = 0.5f * norm_tri_pf(p[0], p[1], p[2]);
+            }
+        }
+    }
+    wave_sync();
+    if (lane >= 8) return 0.0;
+    T a[12], A = T(0);
+    lds_read<12>(sa + lane * kArea, a);
+#pragma unroll
+    for (int q = 0; q < 6; q++) {
+        const T s = a[2 * q] + a[2 * q + 1];
+        if constexpr (sizeof(T) == 8) A = q == 0 ? fabs(s) : A + fabs(s);
+        else A += s;
+    }
+    if constexpr (sizeof(T) == 8) {
+        double x[5][3];
+        const int nd[4] = {0, 1, 3, 4};
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) x[nd[v]][d] = sn[(6 + d) * ss + slx[lane * 8 + nd[v]]];
+        return elem_dt(length_of(hex_corner_volume((const double(*)[3])x), A), l0, c);
+    } else {
+        float M[9];
+        const int cn[3] = {1, 3, 4};
+        const T* x = sp + lane * kPos;
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+#pragma unroll
+            for (int d = 0; d < 3; d++) M[q * 3 + d] = x[cn[q] * 3 + d] - x[d];
+        return elem_dt((double)hex_length_pf(M, A), l0, c);
+    }
+}
+
+// Threads of a workgroup: hex8 eight lanes per element for the forces and as many for the stable dt; tet4 a wave for the
+// forces, one for the dt and one more for the nodes.
+template <int NEN>
+constexpr int spread_threads() {
+    return NEN == 8 ? 16 * MPS_SPREAD_HEX : 3 * MPS_SPREAD_TET;
+}
+template <typename T, int NEN>
+constexpr size_t fixed_lds() {
+    return NEN == 8 ? sizeof(T) * MPS_SPREAD_HEX * (kCol + kCoef + kArea + (sizeof(T) == 4 ? kPos : 0)) : 0;
+}
+// Bytes of dynamic LDS: staged node values (hex8 X, u, X + u; tet4 X, u), then the element phase's arrays.
+template <int NEN>
+__host__ __device__ size_t stage_lds(int ss) {
+    return ((size_t)(NEN == 8 ? 9 : 6) * ss * 8 + 15) / 16 * 16;
+}
+
+}  // namespace
+
+// Step k = A + ci, ci its index in the launch sequence: solve of step k-1 (ci > 0), begin of step k, its element forces
+// and the stable dt for step k+1 (the file's head).
+template <typename T, int NEN, int LAW>
+__global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int ci) {
+    extern __shared__ __align__(16) double smem[];
+    constexpr int EB = NEN == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET;  // elements of a workgroup
+    __shared__ uint16_t slx[NEN == 8 ? EB * 8 : 1];
+    constexpr int NT = spread_threads<NEN>(), FLIGHT = NEN == 8 ? 8 : 16;
+    const int b = xcd_tile(blockIdx.x, gridDim.x), t = threadIdx.x, ss = I.sp_stride;
+    // tables first: their addresses depend on nothing.  Work item it: direction it % 3 of the workgroup's node it / 3.
+    const int4* tab = I.sp_node + (size_t)b * ss;
+    int4 E = make_int4(-1, 0, 0, 0);
+    if (t < 3 * ss) E = tab[t / 3];
+    // role in the element phase: wave of forces or of stable dt
+    const bool force = t < 64;
+    const int lane = t & 63, j = t & 7;
+    const int el = NEN == 8 ? (force ? lane >> 3 : j) : lane;  // a dt wave's lanes 0-7: its elements
+    const int e = b * EB + el;
+    const bool mine = e < I.Ne && (NEN == 8 || t < 128);
+    const int ec = min(e, I.Ne - 1);
+    int pos[NEN == 8 ? 1 : 4];
+    uint2 l4 = make_uint2(0u, 0u);
+    if constexpr (NEN == 8) {
+        pos[0] = I.sp_pos[(size_t)ec * 8 + j];
+        if (force) slx[t] = I.sp_lx[(size_t)ec * 8 + j];
+    } else {
+        const int4 q = *reinterpret_cast<const int4*>(I.sp_pos + (size_t)ec * 4);
+        pos[0] = q.x;
+        pos[1] = q.y;
+        pos[2] = q.z;
+        pos[3] = q.w;
+        l4 = *reinterpret_cast<const uint2*>(I.sp_lx + (size_t)ec * 4);
+    }
+    const TetConsts kc = tet_consts(I, ec, true);
+    // step control, the same in every workgroup: read now, used once the nodes' loads are on their way
+    MpsCtl* ctl = I.ctl;
+    const long long A = ctl->A, k = A + ci;
+    const MpsStepSlot* pp = ci == 0 ? ctl->slot + ((A - 1) & 1) : ctl->sslot + ((ci - 1) & 1);
+    MpsStepSlot prev;
+    prev.time = pp->time;
+    prev.dt = pp->dt;
+    prev.go = pp->go;
+    const int row = t & (MPS_DT_SLOTS - 1);
+    const unsigned long long m16 = *(ci == 0 ? dt_slot(I, dt_parity(A), row) : dt_spread(I, ci % 3, row));
+    const size_t N = (size_t)I.N;
+    double *ur, *wr, *uo, *wo;
+    uw_buffers(I, ci & 1, &ur, &wr);
+    uw_buffers(I, (ci & 1) ^ 1, &uo, &wo);
+    const T* fr = spread_forces<T>(I, ci + 1);  // step k-1
+    NodeLoads<T, FLIGHT> L;
+    if (E.x != -1) L.load(I, E, t - 3 * (t / 3), ci == 0, ur, wr, fr);
+    MpsStepSlot nx;
+    const int st = begin_scalars(I, k, prev, row_min(m16), &nx);
+    if (blockIdx.x == 0 && t == 0) {
+        ctl->sslot[ci & 1] = nx;
+        if (st != MPSD_RUNNING) ctl->status = st;
+        if (nx.go) {
+            ctl->B = k;
+            if (I.hist_cap > 0) {
+                const size_t idx = (size_t)((k - 1) % I.hist_cap);
+                I.hist[idx] = nx.time;
+                I.hist[(size_t)I.hist_cap + idx] = nx.dt;
+            }
+        }
+        spread_reset(I, (ci + 2) % 3);
+    }
+    if (!nx.go) return;
+    for (int it = t; it < 3 * ss; it += NT) {
+        const int q = it / 3, d = it - 3 * q;
+        if (it != t) {
+            E = tab[q];
+            if (E.x != -1) L.load(I, E, d, ci == 0, ur, wr, fr);
+        }
+        if (E.x == -1) break;  // the rest is padding
+        const int n = E.x & 0x7FFFFFFF;
+        double u = L.u, w;
+        if (ci == 0) {
+            w = half_velocity(nx.dt, L.w, L.m);
+        } else {
+            double v, acc;
+            const double fi = L.force(E, fr, d);
+            node_update1(I, L.info, d, k - 1, prev.dt, L.m, -fi + node_fext1(I, n, L.info, d), L.w, &v, &acc);
+            if (E.x < 0) check_finite(I, n, d, k - 1, u);
+            w = half_velocity(nx.dt, v, acc);
+        }
+        u += step_increment(I, L.info, d, k, nx.dt, w);
+        if (E.x < 0) {
+            uo[d * N + n] = u;
+            wo[d * N + n] = w;
+        }
+        if constexpr (NEN == 8) {
+            smem[d * ss + q] = L.X;
+            smem[(3 + d) * ss + q] = u;
+            smem[(6 + d) * ss + q] = L.X + u;
+        } else {
+            smem[6 * q + d] = L.X;
+            smem[6 * q + 3 + d] = u;
+        }
+    }
+    __syncthreads();
+    T* fo = spread_forces<T>(I, ci);
+    unsigned long long dmin = 0x7FF0000000000000ull;
+    if constexpr (NEN == 8) {
+        T* base = reinterpret_cast<T*>(reinterpret_cast<char*>(smem) + stage_lds<8>(ss));
+        T* sc = base + EB * kCol;  // the elements' coefficients
+        if (force) hex_coefficients<T>(smem, ss, slx + el * 8, sc + el * kCoef, j);
+        if constexpr (sizeof(T) == 4) __syncthreads();  // the FP32 lengths are taken from the coefficients
+        else wave_sync();
+        if (force) {
+            T f[3];
+            hex_spread_force<T, LAW>(sc + el * kCoef, base + el * kCol, j, kc.pa, kc.pb, f);
+            if (mine) {
+                T* dst = fo + 3 * (size_t)pos[0];
+#pragma unroll
+                for (int i = 0; i < 3; i++) dst[i] = f[i];
+            }
+            return;
+        }
+        const double dte = hex_spread_dt<T>(smem, ss, slx, sc, base + EB * (kCol + kCoef), base + EB * (kCol + kCoef + kArea),
+                                            lane, kc.c, kc.l0);
+        if (lane < 8 && mine) dmin = d2bits(dte);
+    } else {
+        if (t >= 128) return;
+        const int l[4] = {(int)(l4.x & 0xffffu), (int)(l4.x >> 16), (int)(l4.y & 0xffffu), (int)(l4.y >> 16)};
+        double x[4][3], uu[4][3];
+#pragma unroll
+        for (int a = 0; a < 4; a++) staged_node(smem, l[a], x[a], uu[a]);
+        if (force) {
+            T f[4][3];
+            tet4_core<T, LAW, false>(I, e, nullptr, x, uu, kc, f, false, 0.0);
+            if (!mine) return;
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                T* dst = fo + 3 * (size_t)pos[a];
+#pragma unroll
+                for (int i = 0; i < 3; i++) dst[i] = f[a][i];
+            }
+            return;
+        }
+        const double dte = tet_dt<T>(x, uu, kc);
+        if (mine) dmin = d2bits(dte);
+    }
+    // one atomic per workgroup; all lanes of its dt wave are here
+#pragma unroll
+    for (int off = NEN == 8 ? 4 : 32; off > 0; off >>= 1) dmin = umin64(dmin, (unsigned long long)__shfl_xor((long long)dmin, off, 64));
+    if (lane == 0) atomicMin(dt_spread(I, (ci + 1) % 3, b & (MPS_DT_SLOTS - 1)), dmin);
+}
+
+// After a launch sequence: solve of its last step (B), from the buffer that step wrote, into u, v and a.
+template <typename T>
+__global__ __launch_bounds__(256) void k_spread_end(MpsInst I) {
+    const MpsCtl* ctl = I.ctl;
+    const long long A = ctl->A, k = ctl->B;
+    if (k < A) return;  // no step was begun
+    const int ss = I.sp_stride;
+    const double dt = ctl->sslot[(k - A) & 1].dt;
+    const size_t N = (size_t)I.N;
+    double *ur, *wr;
+    uw_buffers(I, (int)((k - A) & 1) ^ 1, &ur, &wr);
+    const T* fr = spread_forces<T>(I, (int)(k - A));
+    for (int it = threadIdx.x; it < 3 * ss; it += 256) {
+        const int q = it / 3, d = it - 3 * q;
+        const int4 E = I.sp_node[(size_t)xcd_tile(blockIdx.x, gridDim.x) * ss + q];
+        if (E.x == -1) break;
+        if (E.x >= 0) continue;  // another workgroup owns the node
+        const int n = E.x & 0x7FFFFFFF;
+        const size_t i = d * N + n;
+        NodeLoads<T, 8> L;
+        L.load(I, E, d, false, ur, wr, fr);
+        double v, a;
+        const double u = L.u, fi = L.force(E, fr, d);
+        node_update1(I, L.info, d, k, dt, L.m, -fi + node_fext1(I, n, L.info, d), L.w, &v, &a);
+        check_finite(I, n, d, k, u);
+        I.u[i] = u;
+        I.v[i] = v;
+        I.a[i] = a;
+    }
+}
+
+// Closes a launch sequence: its steps count as done, and the scalars and the pending min go where the patch form and the
+// next sequence find them.
+__global__ __launch_bounds__(64) void k_spread_close(MpsInst I) {
+    MpsCtl* ctl = I.ctl;
+    const long long A = ctl->A, k = ctl->B;
+    if (k < A) return;
+    const int ci = (int)(k - A);
+    const unsigned long long mb = row_min(*dt_spread(I, (ci + 1) % 3, threadIdx.x & (MPS_DT_SLOTS - 1)));
+    if (threadIdx.x != 0) return;
+    MpsStepSlot s = ctl->sslot[ci & 1];
+    s.go = 1;
+    ctl->slot[k & 1] = s;
+    dt_reset(I, 0);
+    dt_reset(I, 1);
+    *dt_slot(I, dt_parity(k + 1), 0) = mb;
+    for (int q = 0; q < 3; q++) spread_reset(I, q);
+    ctl->spread_last = ci & 1;
+    ctl->A = k + 1;
+}
+
+// Internal force at DOF idx[i] = node + N*dir of the last step, from its element forces.
+template <typename T>
+__global__ void k_spread_pick(MpsInst I, const int32_t* __restrict__ idx, int64_t n, double* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int4 E = I.sp_node[I.sp_own[idx[i] % I.N]];
+    const int d = idx[i] / I.N;
+    const T* f = spread_forces<T>(I, I.ctl->spread_last);
+    NodeLoads<T, 8> L;
+#pragma unroll
+    for (int q = 0; q < 8; q++) L.c[q] = f[3 * ((size_t)E.y + min(q, E.z - 1)) + d];
+    out[i] = L.force(E, f, d);
+}
+
+namespace mpsk {
+
+hipError_t launch_spread(const MpsInst& I, int ci, hipStream_t st) {
+    const unsigned nb = (unsigned)I.sp_nb;
+#define MPS_SPREAD(T, NEN, LAW) \
+    k_spread<T, NEN, LAW><<<nb, spread_threads<NEN>(), stage_lds<NEN>(I.sp_stride) + fixed_lds<T, NEN>(), st>>>(I, ci)
+#define MPS_SPREAD_LAW(T, NEN)                       \
+    switch (I.law) {                                 \
+        case 0: MPS_SPREAD(T, NEN, 0); break;        \
+        case 1: MPS_SPREAD(T, NEN, 1); break;        \
+        case 2: MPS_SPREAD(T, NEN, 2); break;        \
+        default: MPS_SPREAD(T, NEN, 3); break;       \
+    }
+    if (I.nen == 8) {
+        if (I.precision == 1) { MPS_SPREAD_LAW(float, 8) } else { MPS_SPREAD_LAW(double, 8) }
+    } else {
+        if (I.precision == 1) { MPS_SPREAD_LAW(float, 4) } else { MPS_SPREAD_LAW(double, 4) }
+    }
+#undef MPS_SPREAD_LAW
+#undef MPS_SPREAD
+    return hipGetLastError();
+}
+
+hipError_t launch_spread_end(const MpsInst& I, hipStream_t st) {
+    const unsigned nb = (unsigned)I.sp_nb;
+    if (I.precision == 1) k_spread_end<float><<<nb, 256, 0, st>>>(I);
+    else k_spread_end<double><<<nb, 256, 0, st>>>(I);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    k_spread_close<<<1, 64, 0, st>>>(I);
+    return hipGetLastError();
+}
+
+hipError_t launch_spread_pick(const MpsInst& I, const int32_t* idx, int64_t n, double* out, hipStream_t st) {
+    const unsigned nb = (unsigned)((n + 255) / 256);
+    if (I.precision == 1) k_spread_pick<float><<<nb, 256, 0, st>>>(I, idx, n, out);
+    else k_spread_pick<double><<<nb, 256, 0, st>>>(I, idx, n, out);
+    return hipGetLastError();
+}
+
+}  // namespace mpsk
