@@ -149,7 +149,7 @@ int mps_set_state(mps_handle h, const double *u, const double *v, const double *
 
 /* Set the Neumann loads: n_loads blocks in input order (replacing any earlier call; 0 blocks: none).  At most
  * one GRAVITY block.  Valid only before the first step.  Every step evaluates them at its own time and
- * displacement: nodal forces and gravity in the node kernel, pressure faces in a surface kernel before it.
+ * displacement: one kernel for the nodes that carry items, before the node kernel; gravity alone in the node kernel.
  * Replaces: NeumannCommonManagement's FORCE, GRAVITY and PRESSURE RAMP / INST entries
  * (inputFile.cpp:4703-4735) and their per-step evaluation in NeumannBCManagement (boundaryConditions.cpp:75-140). */
 int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load *loads);

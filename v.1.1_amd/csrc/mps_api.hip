@@ -1248,7 +1248,7 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
     I.n_sgp = 0;
     I.lidx = I.lnn = I.lrow = I.lcode = I.sge = I.sgb = nullptr;
     I.lm = I.lwin = I.fgrav = I.sgd = I.sblk = nullptr;
-    I.pc = I.lf = I.lfprev = nullptr;
+    I.lf = I.lfprev = nullptr;
     auto upload = [&](const void* src, size_t bytes, void** dst) -> hipError_t {
         hipError_t e = hipMalloc(dst, bytes < 256 ? 256 : bytes);
         if (e != hipSuccess) return e;
@@ -1289,8 +1289,6 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
         I.sgd = (const double*)p;
         HCHK(h, upload(sblk.data(), sblk.size() * 8, &p));
         I.sblk = (const double*)p;
-        HCHK(h, upload(nullptr, sge.size() * 24 * 8, &p));
-        I.pc = (double*)p;
         I.n_sgp = (int32_t)sge.size();
     }
     HCHK(h, hipMemcpy((void*)I.ninfo, ninfo.data(), (size_t)N * 4, hipMemcpyHostToDevice));
@@ -1542,7 +1540,7 @@ static hipError_t enqueue_steps(mps_solver_s* h, long long count, std::vector<in
         const bool out_v = every > 0 && k % every == 0;
         const unsigned vaf = (i == 0 ? MPS_N_IN_VA : (every > 0 && (k - 1) % every == 0) ? MPS_N_IN_WA : 0u) |
                              (out_v ? MPS_N_OUT_V : 0u);
-        if (e == hipSuccess && (I.n_sgp > 0 || I.n_lnode > 0)) e = mpsk::launch_loads(I, h->stream);
+        if (e == hipSuccess && I.n_lnode > 0) e = mpsk::launch_loads(I, h->stream);
         if (e == hipSuccess && I.n_series > 0) e = mpsk::launch_series(I, h->stream, vaf);
         if (e != hipSuccess) break;
         const bool last = (i == count - 1);

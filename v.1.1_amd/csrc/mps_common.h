@@ -37,7 +37,6 @@
 //     sge, sgb      int32[n_sgp]   pressure surface Gauss point: bulk element, block
 //     sgd           double[MPS_SGP_STRIDE*n_sgp]  bulk dphi (24), n0 (3), w|J_s| (1), scatter phi (8)
 //     sblk          double[8*blocks]  block type, P, t0, tf, traction (3), -
-//     pc            double[24*n_sgp]  the step's surface forces [(g*8 + a)*3 + dir]
 //   uprev           double[3N]   displacement of the previous step (bulk viscosity only; NULL otherwise)
 //   ctl             MpsCtl       step control (time, dt, go flags), running work sums, reduction counters
 //   dtred           u64[MPS_DT_WORDS]  stable-dt reduction slots by step parity; in the
@@ -178,7 +177,6 @@ struct MpsInst {
     const int32_t* sgb;
     const double* sgd;
     const double* sblk;
-    double* pc;
     // bulk artificial viscosity (solverExplicit.cpp:381-421, 505-542): active when uprev != NULL
     double visc_c1, visc_cl;   // quadratic and linear coefficients
     double visc_h, visc_c0;    // element size and sound speed (> 0), or <= 0: the element's l0 and c

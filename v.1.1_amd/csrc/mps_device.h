@@ -1324,32 +1324,6 @@ __device__ __forceinline__ void predict_node(const MpsInst& I, int n, long long 
     for (int i = 0; i < 3; i++) u[i] += step_increment(I, info, i, k, dt, w[i]);
 }
 
-// External force of flagged node j (lnn[j]) at time t (NeumannBCManagement, boundaryConditions.cpp:75-140):
-// zero, then its load items in input order -- nodal force entries (BCsNodalForces :1120-1134 with
-// classNeumann::getTracAmount, classNodes.h:101-108: F/(tf-t0) * t for t0 <= t <= tf, else 0), the step's
-// surface forces of pressure faces, and its gravity load (BCsGravity :1146-1172, constant, summed over the
-// Gauss points at set-up) at the place of *GRAVITY.
-__device__ __forceinline__ void loaded_node_fext(const MpsInst& I, int j, double t, double* fe) {
-#pragma clang fp contract(off)
-    fe[0] = 0.0;
-    fe[1] = 0.0;
-    fe[2] = 0.0;
-    const int n = I.lnn[j];
-    for (int q = I.lrow[j]; q < I.lrow[j + 1]; q++) {
-        const uint32_t code = (uint32_t)I.lcode[q];
-        const uint32_t kind = code >> 30;
-        const size_t idx = code & MPS_ITEM_INDEX;
-        if (kind == MPS_ITEM_FORCE) {
-            const bool in = t >= I.lwin[2 * idx] && t <= I.lwin[2 * idx + 1];
-            for (int d = 0; d < 3; d++) fe[d] += in ? I.lm[3 * idx + d] * t : 0.0;
-        } else if (kind == MPS_ITEM_PRESSURE) {
-            for (int d = 0; d < 3; d++) fe[d] += I.pc[3 * idx + d];
-        } else {
-            fe[2] += I.fgrav ? I.fgrav[n] : 0.0;
-        }
-    }
-}
-
 // External force of node n in the node kernel: the flagged node's value of this step (lf), else its
 // gravity load alone (zero without gravity).
 __device__ __forceinline__ void node_fext(const MpsInst& I, int n, uint32_t info, double* fe) {
@@ -1370,35 +1344,46 @@ __device__ __forceinline__ double node_fext1(const MpsInst& I, int n, uint32_t i
     return (i == 2 && I.fgrav) ? I.fgrav[n] : 0.0;
 }
 
-// Surface forces of pressure Gauss point q at time t (BCsPressureRamp / BCsPressureInst,
+// Force of scatter node a at surface Gauss point q at time t.  Pressure (BCsPressureRamp / BCsPressureInst,
 // boundaryConditions.cpp:370-496): F of the bulk element at the point (classSpatialPoint::getF,
 // classSpatialPoint.cpp:41-68: node terms first, then the identity), J = det F, n = F^-T n0, and
-// pc[(q*8 + a)*3 + i] = w|J_s| phi_a J P(t) n_i for the scatter nodes a.  FP64, reference operation order.
-__device__ __forceinline__ void surface_point(const MpsInst& I, int q, double t) {
+// w|J_s| phi_a J P(t) n_i.  Traction (BCsTractionRamp / Inst, :218-271): w|J_s| phi_a T_i(t).  FP64, reference operation
+// order; everything it reads is loaded before it is used.
+__device__ __forceinline__ void surface_force(const MpsInst& I, int q, int a, double t, double* out) {
 #pragma clang fp contract(off)
-    const size_t N = (size_t)I.N;
-    const int nen = I.nen;
-    const int e = I.sge[q];
     const double* D = I.sgd + (size_t)q * MPS_SGP_STRIDE;
     const double* B = I.sblk + MPS_SBLK_STRIDE * (size_t)I.sgb[q];
-    double* out = I.pc + (size_t)q * 24;
-    if (B[0] >= 4.0) {  // traction (BCsTractionRamp / Inst, boundaryConditions.cpp:218-271): w|J_s| phi_a T_i
-        const bool tramp = B[0] == 4.0;
-        double T[3] = {0., 0., 0.};
-        if (t >= B[2] && t <= B[3])
-            for (int i = 0; i < 3; i++) T[i] = tramp ? B[4 + i] / (B[3] - B[2]) * (t - B[2]) : B[4 + i];
-        for (int a = 0; a < 8; a++)
-            for (int i = 0; i < 3; i++) out[a * 3 + i] = D[27] * D[28 + a] * T[i];
+    const double ws = D[27], ph = D[28 + a];
+    const bool in = t >= B[2] && t <= B[3];
+    if (B[0] >= 4.0) {
+        for (int i = 0; i < 3; i++) {
+            const double T = in ? (B[0] == 4.0 ? B[4 + i] / (B[3] - B[2]) * (t - B[2]) : B[4 + i]) : 0.;
+            out[i] = ws * ph * T;
+        }
         return;
     }
+    const size_t N = (size_t)I.N;
+    const int nen = I.nen;
+    const int32_t* cn = I.conn + (size_t)I.sge[q] * nen;
+    int nd[8];
+    double disp[8][3], d[8][3];
+#pragma unroll
+    for (int b = 0; b < 8; b++) nd[b] = cn[b < nen ? b : 0];
+#pragma unroll
+    for (int b = 0; b < 8; b++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            disp[b][i] = I.u[i * N + nd[b]];
+            d[b][i] = D[b * 3 + i];
+        }
     double F[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-    for (int a = 0; a < nen; a++) {
-        const int nd = I.conn[(size_t)e * nen + a];
-        double disp[3];
-        for (int i = 0; i < 3; i++) disp[i] = I.u[i * N + nd];
-        for (int i = 0; i < 3; i++)
-            for (int j = 0; j < 3; j++) F[i * 3 + j] += D[a * 3 + j] * disp[i];
-    }
+#pragma unroll
+    for (int b = 0; b < 8; b++)
+        if (b < nen)
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+#pragma unroll
+                for (int j = 0; j < 3; j++) F[i * 3 + j] += d[b][j] * disp[b][i];
     for (int i = 0; i < 3; i++)
         for (int j = 0; j < 3; j++) F[i * 3 + j] += (i == j) ? 1.0 : 0.0;
     const double J = det3_strict(F);
@@ -1413,21 +1398,60 @@ __device__ __forceinline__ void surface_point(const MpsInst& I, int q, double t)
     Fi[2] = idet * (F[1] * F[5] - F[2] * F[4]);
     Fi[5] = -idet * (F[0] * F[5] - F[2] * F[3]);
     Fi[8] = idet * (F[0] * F[4] - F[1] * F[3]);
-    const double* n0 = D + 24;
-    double nv[3];
+    const double P = in ? (B[0] == 2.0 ? B[1] / (B[3] - B[2]) * (t - B[2]) : B[1]) : 0.;
+#pragma unroll
     for (int i = 0; i < 3; i++) {
         double r = 0.0;
-        for (int j = 0; j < 3; j++) r += Fi[j * 3 + i] * n0[j];  // (F^-1)^T, row i
-        nv[i] = r;
+#pragma unroll
+        for (int j = 0; j < 3; j++) r += Fi[j * 3 + i] * D[24 + j];  // (F^-1)^T, row i
+        out[i] = ws * ph * J * P * r;
     }
-    const bool ramp = B[0] == 2.0;
-    double P = 0.;
-    if (t >= B[2] && t <= B[3]) P = ramp ? B[1] / (B[3] - B[2]) * (t - B[2]) : B[1];
-    const double ws = D[27];
-    for (int a = 0; a < 8; a++) {
-        const double ph = D[28 + a];
-        for (int i = 0; i < 3; i++) out[a * 3 + i] = ws * ph * J * P * nv[i];
+}
+
+// One load item of node n at time t: a nodal force entry (BCsNodalForces, boundaryConditions.cpp:1120-1134 with
+// classNeumann::getTracAmount, classNodes.h:101-108: F/(tf-t0) * t for t0 <= t <= tf, else 0), a surface force, or the
+// node's gravity load (BCsGravity :1146-1172, constant, summed over the Gauss points at set-up).
+__device__ __forceinline__ void load_item(const MpsInst& I, int n, uint32_t code, double t, double* c) {
+#pragma clang fp contract(off)
+    const uint32_t kind = code >> 30;
+    const size_t idx = code & MPS_ITEM_INDEX;
+    if (kind == MPS_ITEM_PRESSURE) {
+        surface_force(I, (int)(idx >> 3), (int)(idx & 7), t, c);
+    } else if (kind == MPS_ITEM_FORCE) {
+        const bool in = t >= I.lwin[2 * idx] && t <= I.lwin[2 * idx + 1];
+        for (int d = 0; d < 3; d++) c[d] = in ? I.lm[3 * idx + d] * t : 0.0;
+    } else {
+        c[0] = c[1] = 0.0;
+        c[2] = I.fgrav ? I.fgrav[n] : 0.0;
     }
+}
+
+// External force of the flagged nodes lb*MPS_LOAD_NODES .. +MPS_LOAD_NODES-1 at time t into lf, by one workgroup of 256
+// (NeumannBCManagement, boundaryConditions.cpp:75-140: zero, then the node's load items in input order).  32 lanes per
+// node take one item each and three of them add the items up in order, from sh (256*3 doubles): a node on a loaded face
+// has 16 items and more, whose dependent loads one work-item would walk through one after the other.  No barrier: a
+// node's lanes are half a wave.
+#define MPS_LOAD_NODES 8
+__device__ __forceinline__ void loads_block(const MpsInst& I, int lb, double t, double* sh, double* lf) {
+#pragma clang fp contract(off)
+    const int l = threadIdx.x & 31, j = lb * MPS_LOAD_NODES + (int)(threadIdx.x >> 5);
+    const bool on = j < I.n_lnode;
+    const int q0 = on ? I.lrow[j] : 0, q1 = on ? I.lrow[j + 1] : 0, n = on ? I.lnn[j] : 0;
+    double* s = sh + (threadIdx.x & ~31) * 3;
+    double fe = 0.0;
+    for (int q = q0; __any(q < q1); q += 32) {
+        double c[3] = {0.0, 0.0, 0.0};
+        if (q + l < q1) load_item(I, n, (uint32_t)I.lcode[q + l], t, c);
+#pragma unroll
+        for (int d = 0; d < 3; d++) s[l * 3 + d] = c[d];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (l < 3)
+            for (int r = 0; r < min(32, q1 - q); r++) fe += s[r * 3 + l];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (on && l < 3) lf[3 * (size_t)j + l] = fe;
 }
 
 // Partial nodal force g (FP64 partials; FP32 in the precision form).

@@ -29,8 +29,8 @@ hipError_t launch_fint(const MpsInst& I, double* fint, hipStream_t st);
 hipError_t launch_gravity(const MpsInst& I, double grav, double* tslot, double* fgrav, hipStream_t st);
 // External force fext[3N] at time t from the instance's loads (surface forces from the current u).
 hipError_t launch_fext(const MpsInst& I, double t, double* fext, hipStream_t st);
-// External force of the flagged nodes for the step in flight (surface kernel, then the per-node sums);
-// runs after the step's element kernel, before its node kernel.
+// External force of the flagged nodes for the step in flight; runs after the step's element kernel, before its node
+// kernel.
 hipError_t launch_loads(const MpsInst& I, hipStream_t st);
 // Standalone energy pass: MPS_E_DEF / MPS_E_KIN of step ctl->B between its element and node kernels, or
 // MPS_E_KIN_NOW after the last node kernel of a launch; block sums only (added up by the next kernel).

@@ -922,31 +922,18 @@ __global__ __launch_bounds__(256) void k_grav_node(MpsInst I, const double* __re
     fgrav[n] = acc;
 }
 
-// Surface forces of every pressure Gauss point: mode 0 at the time of the step in flight (ctl->B, after its
-// element kernel), mode 1 at time t (standalone evaluation).
-__global__ __launch_bounds__(256) void k_press(MpsInst I, int mode, double t) {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    if (mode == 0) {
-        const MpsStepSlot s = I.ctl->slot[I.ctl->B & 1];
-        if (!s.go) return;
-        t = s.time;
-    }
-    if (q < I.n_sgp) surface_point(I, q, t);
-}
-
-// External force of every flagged node: mode 0 at the time of the step in flight (after its surface
-// kernel), mode 1 at time t.
+// External force of every flagged node: mode 0 at the time of the step in flight (ctl->B, after its element kernel), mode
+// 1 at time t (standalone evaluation).  A node's items are evaluated by 32 lanes at once (loads_block): two kernels that
+// walked a point's nodes and a node's items one after the other took 11.5 + 11.4 us per step for the top face of a
+// 33x31x35 mesh, nearly all of it latency.
 __global__ __launch_bounds__(256) void k_loads(MpsInst I, int mode, double t) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double sh[256 * 3];
     if (mode == 0) {
         const MpsStepSlot s = I.ctl->slot[I.ctl->B & 1];
         if (!s.go) return;
         t = s.time;
     }
-    if (j >= I.n_lnode) return;
-    double fe[3];
-    loaded_node_fext(I, j, t, fe);
-    for (int d = 0; d < 3; d++) I.lf[3 * (size_t)j + d] = fe[d];
+    loads_block(I, blockIdx.x, t, sh, I.lf);
 }
 
 // External force of every DOF (NeumannBCManagement, boundaryConditions.cpp:75-140) from the values of k_loads.
@@ -1314,15 +1301,13 @@ hipError_t launch_gravity(const MpsInst& I, double grav, double* tslot, double* 
 }
 
 hipError_t launch_fext(const MpsInst& I, double t, double* fext, hipStream_t st) {
-    if (I.n_sgp > 0) k_press<<<blocks_for(I.n_sgp, 256), 256, 0, st>>>(I, 1, t);
-    if (I.n_lnode > 0) k_loads<<<blocks_for(I.n_lnode, 256), 256, 0, st>>>(I, 1, t);
+    if (I.n_lnode > 0) k_loads<<<blocks_for(I.n_lnode, MPS_LOAD_NODES), 256, 0, st>>>(I, 1, t);
     k_fext<<<blocks_for(I.N, 256), 256, 0, st>>>(I, fext);
     return hipGetLastError();
 }
 
 hipError_t launch_loads(const MpsInst& I, hipStream_t st) {
-    if (I.n_sgp > 0) k_press<<<blocks_for(I.n_sgp, 256), 256, 0, st>>>(I, 0, 0.0);
-    if (I.n_lnode > 0) k_loads<<<blocks_for(I.n_lnode, 256), 256, 0, st>>>(I, 0, 0.0);
+    if (I.n_lnode > 0) k_loads<<<blocks_for(I.n_lnode, MPS_LOAD_NODES), 256, 0, st>>>(I, 0, 0.0);
     return hipGetLastError();
 }
 
