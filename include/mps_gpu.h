@@ -348,10 +348,9 @@ typedef struct mps_batch_cfg {
     int32_t max_instances;/* instance slots (0: 1024) */
     int32_t precision;    /* MPS_PREC_* for every instance */
     int32_t steps_per_launch; /* steps captured per graph launch (0: 32) */
-    int32_t elem_block;   /* work-items per element workgroup, 64/128/256 (0: 256 until mps_batch_autotune;
-                             the server tunes it per mix size when both this and grid_mult are 0) */
-    int32_t grid_mult;    /* persistent grid = grid_mult * CUs workgroups (0: 2 until mps_batch_autotune;
-                             tuned by the server as elem_block) */
+    int32_t elem_block;   /* work-items per element workgroup, 64/128/256 (0: 256) */
+    int32_t grid_mult;    /* persistent grid = grid_mult * CUs workgroups (0: one workgroup per unit of work, up
+                             to 16 per CU, following the content; mps_batch_autotune fixes it) */
     int32_t device;
 } mps_batch_cfg;
 
@@ -375,7 +374,7 @@ int mps_batch_query(mps_batch b, int32_t slot, mps_report *rep);
 int mps_batch_get_state(mps_batch b, int32_t slot, double *u, double *v, double *a);
 /* Free a slot for reuse. */
 int mps_batch_remove(mps_batch b, int32_t slot);
-/* Autotune elem_block / grid_mult on the current batch content; writes the choice. */
+/* Autotune grid_mult on the current batch content (elem_block: 256); writes the choice. */
 int mps_batch_autotune(mps_batch b, int32_t *elem_block, int32_t *grid_mult);
 int mps_batch_destroy(mps_batch b);
 const char *mps_batch_last_error(mps_batch b);
@@ -407,7 +406,7 @@ typedef struct mps_server_stats {
     double solves_per_s;            /* completed / span */
     double busy_ms;                 /* time with a graph launch in flight */
     int32_t elem_block, grid_mult;  /* tuning of the latest launch */
-    int32_t tunings;                /* mix sizes the online tuner has settled */
+    int32_t tunings;                /* mix sizes launched so far (half-decades of active elements) */
     int32_t _pad;
 } mps_server_stats;
 

@@ -105,6 +105,7 @@ struct Table {
     int cap = 0;
     hipEvent_t last_use = nullptr;  // recorded after the last launch that read this buffer
     hipGraphExec_t exec = nullptr;  // graph captured for this buffer
+    int grid_mult = 0;              // and the grid it was captured with
 };
 
 }  // namespace
@@ -152,8 +153,7 @@ struct mps_batch_s {
     int steps_per_launch = 32;
     hipEvent_t last_launch = nullptr;
     bool any_launch = false;
-    hipEvent_t tl0 = nullptr, tl1 = nullptr;  // around the graph launches of the last enqueue
-    bool timed = false;
+    bool grid_rule = true;  // grid_mult follows the content (flush_tables); false: given by the caller or autotuned
     std::string err;
     int fail(int code, const std::string& m) {
         err = m;
@@ -182,8 +182,6 @@ static void batch_release(mps_batch_s* b) {
     if (b->ctl) (void)hipFree(b->ctl);
     if (b->insts) (void)hipFree(b->insts);
     if (b->last_launch) (void)hipEventDestroy(b->last_launch);
-    if (b->tl0) (void)hipEventDestroy(b->tl0);
-    if (b->tl1) (void)hipEventDestroy(b->tl1);
     if (b->up) (void)hipStreamDestroy(b->up);
     if (b->stream) (void)hipStreamDestroy(b->stream);
 }
@@ -203,7 +201,8 @@ extern "C" int mps_batch_create(const mps_batch_cfg* cfg, mps_batch* out) {
     b->device = cfg->device;
     b->steps_per_launch = cfg->steps_per_launch > 0 ? cfg->steps_per_launch : 32;
     b->bs = cfg->elem_block > 0 ? cfg->elem_block : 256;
-    b->grid_mult = cfg->grid_mult > 0 ? cfg->grid_mult : 2;
+    b->grid_mult = cfg->grid_mult > 0 ? cfg->grid_mult : 1;
+    b->grid_rule = cfg->grid_mult == 0;
     int rc = MPS_OK;
     hipDeviceProp_t p;
     if (hipSetDevice(b->device) != hipSuccess || hipGetDeviceProperties(&p, b->device) != hipSuccess) {
@@ -214,7 +213,6 @@ extern "C" int mps_batch_create(const mps_batch_cfg* cfg, mps_batch* out) {
         if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess ||
             hipStreamCreateWithFlags(&b->up, hipStreamNonBlocking) != hipSuccess ||
             hipEventCreateWithFlags(&b->last_launch, hipEventDisableTiming) != hipSuccess ||
-            hipEventCreate(&b->tl0) != hipSuccess || hipEventCreate(&b->tl1) != hipSuccess ||
             hipMalloc(&b->arena, (size_t)b->cfg.arena_bytes) != hipSuccess ||
             hipMalloc(&b->ctl, sizeof(MpsCtl) * M) != hipSuccess ||
             hipMalloc(&b->insts, sizeof(MpsInst) * M) != hipSuccess) {
@@ -425,6 +423,7 @@ static int capture(mps_batch_s* b, int t) {
         T.exec = nullptr;
     }
     const int grid = b->grid_mult * b->cus;
+    T.grid_mult = b->grid_mult;
     const int S = b->steps_per_launch;
     const int prec = b->cfg.precision;
     hipGraph_t g = nullptr;
@@ -463,11 +462,18 @@ static int flush_tables(mps_batch_s* b) {
             we.push_back({s, e0, std::min(e0 + MPS_PATCH, S.inst.Ne), e0 == 0});
         for (int n0 = 0; n0 < S.inst.N; n0 += bs) wn.push_back({s, n0, std::min(n0 + bs, S.inst.N), n0 == 0});
     }
+    // one workgroup per patch up to 16 per CU: the hardware then places them as CUs become free, where a smaller
+    // persistent grid fixes each workgroup's patches beforehand.  The multiple moves in powers of two, so that an
+    // admission rarely needs a new graph (workgroups without a patch end at once).
+    if (b->grid_rule) {
+        b->grid_mult = 1;
+        while (b->grid_mult < 16 && (size_t)b->grid_mult * b->cus < we.size()) b->grid_mult *= 2;
+    }
     const int nt = 1 - b->cur;
     Table& T = b->tab[nt];
     BCHK(b, hipEventSynchronize(T.last_use));  // launches that read this buffer are done
     const int need = (int)std::max(we.size(), wn.size());
-    bool recap = T.exec == nullptr;
+    bool recap = T.exec == nullptr || T.grid_mult != b->grid_mult;
     if (need > T.cap) {
         if (T.elem) (void)hipFree(T.elem);
         if (T.node) (void)hipFree(T.node);
@@ -504,10 +510,7 @@ static int enqueue(mps_batch_s* b, int64_t launches) {
         rc = capture(b, b->cur);
         if (rc) return rc;
     }
-    BCHK(b, hipEventRecord(b->tl0, b->stream));
     for (int64_t i = 0; i < launches; i++) BCHK(b, hipGraphLaunch(T.exec, b->stream));
-    BCHK(b, hipEventRecord(b->tl1, b->stream));
-    b->timed = launches > 0;
     BCHK(b, hipEventRecord(T.last_use, b->stream));
     BCHK(b, hipEventRecord(b->last_launch, b->stream));
     b->any_launch = true;
@@ -598,24 +601,7 @@ extern "C" int mps_batch_info(mps_batch b, int64_t* free_bytes, int64_t* largest
     return MPS_OK;
 }
 
-// Element-steps the next `launches` graph launches will perform: every active solve advances by
-// steps_per_launch steps per launch until its own step count (progress from the last sync; a solve admitted
-// since then starts at step 1).
-double mps_batch_launch_work(mps_batch b, int64_t launches) {
-    double w = 0.0;
-    const int64_t S = (int64_t)b->steps_per_launch * launches;
-    for (size_t s = 0; s < b->slots.size(); s++) {
-        const Slot& sl = b->slots[s];
-        if (!sl.used) continue;
-        const MpsCtl& c = b->ctl_h[s];
-        if (c.status != MPS_RUNNING || c.nan_step != LLONG_MAX) continue;
-        const int64_t left = sl.n_steps - (c.A - 1);
-        if (left > 0) w += (double)sl.inst.Ne * (double)std::min(left, S);
-    }
-    return w;
-}
-
-// Active elements (the mix size the serving tuner keys on).
+// Active elements (the mix size of the serving statistics).
 int64_t mps_batch_active_elements(mps_batch b) {
     int64_t n = 0;
     for (auto& sl : b->slots)
@@ -623,42 +609,14 @@ int64_t mps_batch_active_elements(mps_batch b) {
     return n;
 }
 
-// Device milliseconds of the graph launches of the last enqueue (valid after a sync); < 0 if none.
-double mps_batch_last_launch_ms(mps_batch b) {
-    if (!b->timed) return -1.0;
-    float ms = 0.f;
-    if (hipEventElapsedTime(&ms, b->tl0, b->tl1) != hipSuccess) return -1.0;
-    return ms;
-}
-
 void mps_batch_tuning(mps_batch b, int* elem_block, int* grid_mult) {
     *elem_block = b->bs;
     *grid_mult = b->grid_mult;
 }
 
-// Element block size and resident-block multiple for the following launches.  Results do not depend on
-// them (every sum has a fixed order), so they may change between launches of a running batch.  Call only
-// when no launch is in flight (after a sync): the captured graphs are released and re-captured.
-int mps_batch_set_tuning(mps_batch b, int elem_block, int grid_mult) {
-    if (elem_block != 64 && elem_block != 128 && elem_block != 256) return MPS_ERR_ARG;
-    if (grid_mult < 1 || grid_mult > 64) return MPS_ERR_ARG;
-    if (elem_block == b->bs && grid_mult == b->grid_mult) return MPS_OK;
-    (void)hipSetDevice(b->device);
-    int rc = wait_launches(b);
-    if (rc) return rc;
-    b->bs = elem_block;
-    b->grid_mult = grid_mult;
-    b->dirty = true;
-    for (auto& t : b->tab)
-        if (t.exec) {
-            (void)hipGraphExecDestroy(t.exec);
-            t.exec = nullptr;
-        }
-    return MPS_OK;
-}
-
-// Autotuner: times S-step graph launches for every (block size, grid multiple) on the current
-// content, restores the state after each trial, keeps the fastest.
+// Autotuner: times S-step graph launches for every grid multiple on the current content, restores the state after
+// each trial, keeps the fastest.  One work-item per element always: with 128 and 64 per patch an element phase of 20
+// FP32 cubes of 6..40 elements a side took 67 and 107 us against 42, of 9 FP64 cubes of 6..24 24 and 38 us against 16.
 extern "C" int mps_batch_autotune(mps_batch b, int32_t* elem_block, int32_t* grid_mult) {
     if (!b) return MPS_ERR_ARG;
     (void)hipSetDevice(b->device);
@@ -686,46 +644,42 @@ extern "C" int mps_batch_autotune(mps_batch b, int32_t* elem_block, int32_t* gri
         }
     };
     snapshot(true);
-    const int bs0 = b->bs, gm0 = b->grid_mult;
+    const int gm0 = b->grid_mult;
     float best = 1e30f;
-    int best_bs = bs0, best_gm = gm0;
-    const int bss[3] = {64, 128, 256};
+    int best_gm = gm0;
+    b->grid_rule = false;
     const int gms[5] = {1, 2, 4, 8, 16};
-    for (int bs : bss)
-        for (int gm : gms) {
-            if (bs * gm > 4096) continue;  // more resident threads per CU than the hardware holds
-            b->bs = bs;
-            b->grid_mult = gm;
-            b->dirty = true;
-            for (auto& t : b->tab)
-                if (t.exec) {
-                    (void)hipGraphExecDestroy(t.exec);
-                    t.exec = nullptr;
-                }
-            rc = flush_tables(b);
-            if (rc == MPS_OK) rc = enqueue(b, 1);  // warm-up launch
-            float ms = 0.f;
-            if (rc == MPS_OK) {
-                (void)hipEventRecord(e0, b->stream);
-                rc = enqueue(b, 2);
-                (void)hipEventRecord(e1, b->stream);
-                (void)hipEventSynchronize(e1);
-                (void)hipEventElapsedTime(&ms, e0, e1);
+    b->bs = MPS_PATCH;
+    for (int gm : gms) {
+        b->grid_mult = gm;
+        b->dirty = true;
+        for (auto& t : b->tab)
+            if (t.exec) {
+                (void)hipGraphExecDestroy(t.exec);
+                t.exec = nullptr;
             }
-            snapshot(false);
-            if (rc != MPS_OK) break;
-            if (ms < best) {
-                best = ms;
-                best_bs = bs;
-                best_gm = gm;
-            }
+        rc = flush_tables(b);
+        if (rc == MPS_OK) rc = enqueue(b, 1);  // warm-up launch
+        float ms = 0.f;
+        if (rc == MPS_OK) {
+            (void)hipEventRecord(e0, b->stream);
+            rc = enqueue(b, 2);
+            (void)hipEventRecord(e1, b->stream);
+            (void)hipEventSynchronize(e1);
+            (void)hipEventElapsedTime(&ms, e0, e1);
         }
+        snapshot(false);
+        if (rc != MPS_OK) break;
+        if (ms < best) {
+            best = ms;
+            best_gm = gm;
+        }
+    }
     (void)hipStreamSynchronize(b->stream);
     (void)hipFree(backup);
     (void)hipFree(ctl_bk);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    b->bs = best_bs;
     b->grid_mult = best_gm;
     b->dirty = true;
     for (auto& t : b->tab)
@@ -737,7 +691,7 @@ extern "C" int mps_batch_autotune(mps_batch b, int32_t* elem_block, int32_t* gri
     rc = flush_tables(b);
     if (rc) return rc;
     rc = refresh(b);
-    if (elem_block) *elem_block = best_bs;
+    if (elem_block) *elem_block = b->bs;
     if (grid_mult) *grid_mult = best_gm;
     return rc;
 }

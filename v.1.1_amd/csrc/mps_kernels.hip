@@ -70,13 +70,24 @@ struct PatchList {
 template <typename T>
 __device__ __forceinline__ void node_sum(const MpsInst& I, int g, int q0, int q1, int nen, const T* __restrict__ sf,
                                          const uint16_t* __restrict__ pc) {
+    // four entries at a time: their list and force reads are all issued before the ordered additions.  Entries past the
+    // end repeat the last one and add 0.0, which changes no sum (a sum that starts at 0.0 is never -0.0).
     double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-    for (int q = q0; q < q1; q++) {
-        const int c = pc[q];
-        const int i = c / nen, a = c % nen;
-        s0 += (double)sf[(a * 3 + 0) * MPS_PATCH + i];
-        s1 += (double)sf[(a * 3 + 1) * MPS_PATCH + i];
-        s2 += (double)sf[(a * 3 + 2) * MPS_PATCH + i];
+    for (int q = q0; q < q1; q += 4) {
+        T f[4][3];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int c = pc[min(q + r, q1 - 1)], i = c / nen, a = c % nen;
+#pragma unroll
+            for (int d = 0; d < 3; d++) f[r][d] = sf[(a * 3 + d) * MPS_PATCH + i];
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const bool in = q + r < q1;
+            s0 += in ? (double)f[r][0] : 0.0;
+            s1 += in ? (double)f[r][1] : 0.0;
+            s2 += in ? (double)f[r][2] : 0.0;
+        }
     }
     if (sizeof(T) == 4) {  // precision form: partials rounded once to FP32, summed in FP64 by the node kernel
         float* dst = reinterpret_cast<float*>(I.part) + 3 * (size_t)g;
@@ -416,10 +427,18 @@ __device__ __forceinline__ int batch_stride() { return (gridDim.x & 7) ? gridDim
 // first element); BS work-items share the patch's elements.  At least 2 waves per SIMD: the FP64 hex
 // instantiations otherwise take more than 256 registers and run one wave per SIMD (10% slower for
 // a batch of FP64 cubes, against a small spill).
+// FP32 with one work-item per element (BS = MPS_PATCH, the choice unless the caller names another): the patch's lists
+// are loaded ahead of the element work, as in k_elem (8-entry pieces end inside the instance's block: prow and pcol are
+// followed by other arrays); 20 cubes of 6..40 elements a side 41.8 -> 39.3 us.  In FP64 the lists' registers cost more
+// than their latency (9 cubes of 6..24: 15.6 -> 16.3 us).  Nodes are gathered by 32-bit offsets: a mesh has fewer than
+// MPS_OFF32_NODES nodes.
 template <typename T, int NEN, int LAW, int BS>
 __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) void k_elem_batch(const MpsInst* __restrict__ insts,
                                                     const MpsWork* __restrict__ work, const int* __restrict__ nwork_p) {
+    constexpr bool PRE = BS == MPS_PATCH && sizeof(T) == 4;
     __shared__ T sf[NEN * 3 * MPS_PATCH];
+    __shared__ __align__(16) uint16_t spc[PRE ? NEN * MPS_PATCH : 1];
+    __shared__ __align__(16) uint16_t spr[PRE ? PatchList<NEN>::SPR : 1];
     __shared__ unsigned long long sh[BS / 64 + 1];
     const int nwork = *nwork_p;
     for (int w = batch_first(nwork); w < batch_end(nwork); w += batch_stride()) {
@@ -428,7 +447,8 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) void k_
         const long long k = I.ctl->A;
         if (W.first && threadIdx.x == 0) I.ctl->B = k;
         if (I.ctl->slot[k & 1].go) {
-            unsigned long long m = patch_forces<T, NEN, LAW, BS>(I, W.begin / MPS_PATCH, true, sf, nullptr, nullptr);
+            unsigned long long m =
+                patch_forces<T, NEN, LAW, BS, false, PRE, false, true>(I, W.begin / MPS_PATCH, true, sf, spc, spr);
             m = block_min_u64(m, sh);
             if (threadIdx.x == 0) atomicMin(dt_slot(I, dt_parity(k + 1), w & (MPS_DT_SLOTS - 1)), m);
         }
