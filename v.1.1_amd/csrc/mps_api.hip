@@ -423,10 +423,12 @@ int prepare(const mps_mesh* mesh, const mps_material* mat, const mps_bcs* bcs, c
 }
 
 // Meshes up to this many elements step in the spread form: hex8 FP64 29,800 elements 16.4 us per step against 19.9, 64,000
-// 29.4 against 21.0; tet4 FP32 form 48,000 10.2 against 11.3, 93,800 16.7 against 12.0.  MPS_SPREAD=0 in the environment keeps the patch form,
+// 29.4 against 21.0; tet4 FP32 form 48,000 10.2 against 11.3, 93,800 16.7 against 12.0.  With energies every step the patch
+// form gives up more (its energy kernels and sums): hex8 35,800 28.6 against 31.4, 50,700 38.1 against 31.4; tet4 55,600 14.3
+// against 22.1.  Loads and viscosity come after creation: at 31,700 elements with both 24.5 against 29.1.  MPS_SPREAD=0 in the environment keeps the patch form,
 // MPS_SPREAD=1 takes the spread form at any size; so do the switches of the patch kernels (MPS_GATHER32, MPS_DT_SKIP,
 // MPS_TET_STAGING), which have no meaning in the spread form.  Both forms give the same bits.
-static const int64_t kSpreadMaxHex = 32768, kSpreadMaxTet = 60000;
+static const int64_t kSpreadMaxHex = 32768, kSpreadMaxTet = 60000, kSpreadMaxHexEnergy = 40960, kSpreadMaxTetEnergy = 80000;
 
 void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const int64_t N = hp.N, Ne = hp.Ne, nen = hp.nen;
@@ -434,7 +436,9 @@ void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const char* env = getenv("MPS_SPREAD");
     const bool force = env && strcmp(env, "1") == 0;
     if (env && !force && strcmp(env, "0") == 0) return;
-    if (!force && (Ne > (nen == 8 ? kSpreadMaxHex : kSpreadMaxTet) || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") ||
+    const bool en = hp.cfg.energy_every > 0 && hp.cfg.precision == MPS_PREC_FP64;
+    const int64_t most = nen == 8 ? (en ? kSpreadMaxHexEnergy : kSpreadMaxHex) : (en ? kSpreadMaxTetEnergy : kSpreadMaxTet);
+    if (!force && (Ne > most || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") ||
                    getenv("MPS_TET_STAGING")))
         return;
     const int64_t EB = nen == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET, nb = (Ne + EB - 1) / EB, S = Ne * nen;
@@ -522,6 +526,7 @@ struct mps_solver_s {
     double* fint_part = nullptr;     // partial forces of mps_internal_force (allocated on first use, in allocs)
     bool part_valid = false;         // I.part holds the forces of the current u (false: set-up scratch)
     bool spread_forces = false;      // the last step ran in the spread form: its forces are in I.sp_f
+    bool pressure_loads = false;     // the loads hold a pressure block
     bool primed = false;       // prologue (first dt) done
     long long next_step = 1;   // host mirror of ctl->A
     bool step_begun = false;   // step next_step already predicted on the device
@@ -574,13 +579,18 @@ static hipError_t dalloc(mps_solver_s* h, P** p, size_t bytes) {
     return e;
 }
 
+// Captured chunks hold the kernels' arguments: they go when a call changes the instance.
+static void drop_graphs(mps_solver_s* h) {
+    for (auto& g : h->graphs) (void)hipGraphExecDestroy(g.exec);
+    h->graphs.clear();
+}
+
 static void release(mps_solver_s* h) {
     if (!h) return;
     for (hipEvent_t e : h->evpool) (void)hipEventDestroy(e);
     h->evpool.clear();
     if (h->device >= 0) (void)hipSetDevice(h->device);
-    for (auto& g : h->graphs) (void)hipGraphExecDestroy(g.exec);
-    h->graphs.clear();
+    drop_graphs(h);
     if (h->stream) (void)hipStreamSynchronize(h->stream);
     for (void* p : h->allocs) (void)hipFree(p);
     h->allocs.clear();
@@ -774,6 +784,8 @@ static int upload_instance(mps_solver_s* h, const HostPrep& hp) {
         I.sp_own = spo;
         I.sp_nb = sp.nb;
         I.sp_stride = sp.stride;
+        I.n_patch = hp.n_patch;
+        if (I.energy_every > 0 && I.precision == MPS_PREC_FP64) HCHK(h, dalloc(h, &I.sp_ep, mpsk::spread_energy_doubles(I) * 8));
     }
     HCHK(h, hipMemcpyAsync(bcval, hp.bcval.data(), hp.bcval.size() * 8, hipMemcpyHostToDevice, h->stream));
     HCHK(h, hipMemsetAsync(hist, 0xFF, MPS_HIST_COLS * (size_t)cap * 8, h->stream));  // NaN
@@ -913,6 +925,7 @@ extern "C" int mps_set_viscosity(mps_handle h, int32_t type, double c1, double c
     if (!std::isfinite(c1) || !std::isfinite(cl) || !std::isfinite(elem_size) || !std::isfinite(c0))
         return h->fail(MPS_ERR_ARG, "mps_set_viscosity: parameters must be finite");
     MpsInst& I = h->I;
+    drop_graphs(h);
     if (type != MPS_VISC_BULK) {  // the deviatoric variant adds no force
         I.uprev = nullptr;
         return MPS_OK;
@@ -1122,6 +1135,7 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
     const int64_t N = I.N, Ne = I.Ne;
     const int nen = I.nen;
     int n_grav = 0, grav_block = -1;
+    bool pressure = false;
     double grav = 0.0;
     int64_t n_force = 0, n_face = 0;
     for (int b = 0; b < n_loads; b++) {
@@ -1147,6 +1161,7 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
         } else if (L.type >= MPS_LOAD_PRESSURE_RAMP && L.type <= MPS_LOAD_TRACTION_INST) {
             const bool ramp = L.type == MPS_LOAD_PRESSURE_RAMP || L.type == MPS_LOAD_TRACTION_RAMP;
             const bool trac = L.type >= MPS_LOAD_TRACTION_RAMP;
+            pressure = pressure || (!trac && L.n > 0);
             if (L.n > 0 && (!L.index || !L.face)) return h->fail(MPS_ERR_ARG, at + "surface load needs index and face");
             if (trac && (!L.force || !std::isfinite(L.force[0]) || !std::isfinite(L.force[1]) || !std::isfinite(L.force[2])))
                 return h->fail(MPS_ERR_ARG, at + "TRACTION needs a finite traction vector in force[0..2]");
@@ -1242,6 +1257,7 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
         lrow.back()++;
     }
     HCHK(h, hipStreamSynchronize(h->stream));
+    drop_graphs(h);
     for (void* q : h->load_allocs) (void)hipFree(q);
     h->load_allocs.clear();
     I.n_lnode = 0;
@@ -1265,7 +1281,7 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
         I.lrow = (const int32_t*)p;
         HCHK(h, upload(lcode.data(), lcode.size() * 4, &p));
         I.lcode = (const int32_t*)p;
-        HCHK(h, upload(nullptr, lnn.size() * 24, &p));
+        HCHK(h, upload(nullptr, lnn.size() * 2 * 24, &p));
         I.lf = (double*)p;
         I.n_lnode = (int32_t)lnn.size();
         if (I.energy_every > 0) {  // previous step's external force of the flagged nodes (work of the loads)
@@ -1291,6 +1307,7 @@ extern "C" int mps_set_loads(mps_handle h, int32_t n_loads, const mps_load* load
         I.sblk = (const double*)p;
         I.n_sgp = (int32_t)sge.size();
     }
+    h->pressure_loads = pressure;
     HCHK(h, hipMemcpy((void*)I.ninfo, ninfo.data(), (size_t)N * 4, hipMemcpyHostToDevice));
     if (grav_block >= 0 && grav != 0.0) {
         HCHK(h, upload(nullptr, (size_t)N * 8, &p));
@@ -1480,10 +1497,13 @@ static void collect_times(mps_solver_s* h, const std::vector<int>& kinds) {
 // still holds it before the node pass (when (k-1) % every == 0 and k-1 is in this chunk), in the element kernel
 // (FP64 inviscid form) or in the standalone pass before the node kernel; after the last node pass, the pass for
 // the KIN_ENERGY of the chunk's last step.  The node kernels accumulate the work sums every step.
-// True when the steps run in the spread form: set up at creation, and nothing in the step that only the patch form has.
+// True when the steps run in the spread form: set up at creation, and nothing in the step that only the patch form has
+// (DOF series, pressure loads, which need the step's displacement, energies with FP32 forces or with viscosity, viscous
+// tet4 elements).
 static bool use_spread(const mps_solver_s* h) {
     const MpsInst& I = h->I;
-    return I.sp_nb > 0 && !h->step_begun && I.energy_every == 0 && I.uprev == nullptr && I.n_series == 0 && I.n_lnode == 0;
+    return I.sp_nb > 0 && !h->step_begun && I.n_series == 0 && !h->pressure_loads &&
+           (I.energy_every == 0 || mpsk::elem_fuses_energy(I)) && (I.uprev == nullptr || I.nen == 8);
 }
 
 // Spread form of enqueue_steps: one launch per step, and the end of the sequence.
@@ -1491,7 +1511,9 @@ static hipError_t enqueue_spread(mps_solver_s* h, long long count, std::vector<i
     hipError_t e = hipSuccess;
     for (long long i = 0; i < count && e == hipSuccess; i++) {
         TimedLaunch t(h, 0);
-        e = mpsk::launch_spread(h->I, (int)i, h->stream);
+        const long long k = h->next_step + i, every = h->I.energy_every;
+        const bool kin = every > 0 && i >= 1 && k >= 2 && (k - 1) % every == 0;
+        e = mpsk::launch_spread(h->I, (int)i, kin ? MPS_E_KIN : 0u, h->stream);
         t.done();
         if (t.a) kinds->push_back(0);
     }
@@ -1500,6 +1522,13 @@ static hipError_t enqueue_spread(mps_solver_s* h, long long count, std::vector<i
     e = mpsk::launch_spread_end(h->I, h->stream);
     t.done();
     if (t.a) kinds->push_back(1);
+    if (h->I.energy_every > 0) {
+        TimedLaunch te(h, 3);
+        if (e == hipSuccess) e = mpsk::launch_energy(h->I, MPS_E_KIN_NOW, h->stream);
+        if (e == hipSuccess) e = mpsk::launch_energy_tail(h->I, h->stream);
+        te.done();
+        if (te.a) kinds->push_back(3);
+    }
     h->next_step += count;
     return e;
 }
@@ -1815,8 +1844,7 @@ extern "C" int mps_set_dof_series(mps_handle h, int64_t n, const int32_t* which,
     if (n > INT32_MAX) return h->fail(MPS_ERR_ARG, "mps_set_dof_series: too many entries");
     (void)hipSetDevice(h->device);
     HCHK(h, hipStreamSynchronize(h->stream));
-    for (auto& g : h->graphs) (void)hipGraphExecDestroy(g.exec);  // the captured steps launch the series kernel
-    h->graphs.clear();
+    drop_graphs(h);  // the captured steps launch the series kernel
     for (void* p : h->series_allocs) (void)hipFree(p);
     h->series_allocs.clear();
     MpsInst& I = h->I;

@@ -31,7 +31,8 @@
 //     lidx          int32[N]         compact index of a flagged node (read only for flagged nodes)
 //     lnn, lrow     int32[n_lnode], [n_lnode+1]  node id; CSR into lcode
 //     lcode         int32[items]     kind (bits 30-31: MPS_ITEM_*) | index
-//     lf            double[3*n_lnode]  the step's external force of each flagged node
+//     lf            double[2*3*n_lnode]  the step's external force of each flagged node (the spread form: two sets by
+//                                    the parity of the step's index)
 //     lm, lwin      double[3*n_f], [2*n_f]  nodal force entry: F/(tf-t0) (classNodes.cpp:85-96); t0, tf
 //     fgrav         double[N]      gravity load along z (NULL: no gravity)
 //     sge, sgb      int32[n_sgp]   pressure surface Gauss point: bulk element, block
@@ -200,6 +201,7 @@ struct MpsInst {
     const int32_t* sp_own;    // [N] entry of sp_node that owns the node
     void* sp_f;               // [2][3*nen*Ne] element forces in node order, by the parity of the step's index
     double* sp_uw;            // [6*N] alternate u and w
+    double* sp_ep;            // energies (solves with energies): node sums by wave and group, element sums by element and patch
     // per-step DOF series (mps_set_dof_series): n_series entries, recorded into ser_ring[(k-1)%hist_cap][i]
     int32_t n_series;
     const int32_t* ser_dof;   // node + N*dir

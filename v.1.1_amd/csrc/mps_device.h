@@ -379,6 +379,7 @@ __device__ __forceinline__ void pk1(const float* H, float pa, float pb, float* P
 // St-Venant-Kirchhoff 0.5 S:E (hyperElasticStVenantKirchhoff.cpp:251-274); linear elastic
 // 0.5 (P:F - P:I) (linearElastic.cpp:97-110).
 __device__ __forceinline__ double defo_energy(int law, const double* F, double lambda, double mu) {
+#pragma clang fp contract(off)
     if (law == 1) return 0.0;
     if (law >= 2) {
         double H[9], P[9];
@@ -763,9 +764,10 @@ __device__ __forceinline__ void elem_mat(const MpsInst& I, int e, double& pa, do
 // ---------------------------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ void add_bulk_visc(const T* H, T trD, T qa, T qb, T* P) {
+#pragma clang fp contract(off)
     const T J = T(1) + detIpH_m1(H);
     const T mn = trD < T(0) ? trD : T(0);
-    const T q = (qa * fabs(trD) * mn + qb * trD) / J;
+    const T q = fma_t(qa * fabs(trD), mn, qb * trD) / J;
     T F[9], cF[9];
 #pragma unroll
     for (int i = 0; i < 9; i++) F[i] = H[i];
@@ -774,7 +776,7 @@ __device__ __forceinline__ void add_bulk_visc(const T* H, T trD, T qa, T qb, T* 
     F[8] += T(1);
     cof3(F, cF);
 #pragma unroll
-    for (int i = 0; i < 9; i++) P[i] += q * cF[i];
+    for (int i = 0; i < 9; i++) P[i] = fma_t(q, cF[i], P[i]);
 }
 
 // Viscosity coefficients of element e (qa, qb of add_bulk_visc); element size and sound speed are the
@@ -819,6 +821,26 @@ __device__ __forceinline__ void gather_nodes(size_t N, const int* nd, const doub
     }
 }
 
+// rho/2 |v|^2 at a Gauss point from the sums vs and the (unscaled) butterfly coefficients Cv of the nodal velocities.
+__device__ __forceinline__ double hex_point_kinetic(const double* vs, const double (*Cv)[3], const GpSigns<double>& s,
+                                                    double rho) {
+#pragma clang fp contract(off)
+    const double g = MPS_GP, g2 = MPS_GP * MPS_GP, g3 = MPS_GP * MPS_GP * MPS_GP;
+    double kv = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        double v = fma(s.x * g, Cv[0][j], vs[j]);
+        v = fma(s.y * g, Cv[1][j], v);
+        v = fma(s.z * g, Cv[2][j], v);
+        v = fma(s.xy * g2, Cv[3][j], v);
+        v = fma(s.yz * g2, Cv[4][j], v);
+        v = fma(s.xz * g2, Cv[5][j], v);
+        v = 0.125 * fma(s.xy * s.z * g3, Cv[6][j], v);
+        kv = fma(0.5 * rho * v, v, kv);
+    }
+    return kv;
+}
+
 // Consistent kinetic energy of hex8 element e (KIN_ENERGY, dataExtraction.cpp:631-707): sum over the GPs of
 // wJ[gp] rho/2 |v(gp)|^2, v(gp) = sum_a phi_a(gp) v_a evaluated from the butterfly coefficients of the nodal
 // velocities, (sum_a v_a + sum_m s_m(gp) g^|m| C_m) / 8.
@@ -835,20 +857,12 @@ __device__ __forceinline__ double hex_kinetic(const MpsInst& I, const int* nd, d
         for (int a = 0; a < 8; a++) t += x[a][d];
         vs[d] = t;
     }
-    const double g = MPS_GP, g2 = MPS_GP * MPS_GP, g3 = MPS_GP * MPS_GP * MPS_GP;
     double ek = 0.0;
 #pragma unroll
     for (int gp = 0; gp < 8; gp++) {
-        const int sx = sxi(gp), sy = seta(gp), sz = szeta(gp);
-        double kv = 0.0;
-#pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const double vel = 0.125 * (vs[j] + (sx * g) * Cv[0][j] + (sy * g) * Cv[1][j] + (sz * g) * Cv[2][j] +
-                                        (sx * sy * g2) * Cv[3][j] + (sy * sz * g2) * Cv[4][j] +
-                                        (sx * sz * g2) * Cv[5][j] + (sx * sy * sz * g3) * Cv[6][j]);
-            kv += 0.5 * rho * vel * vel;
-        }
-        ek += kv * wJ[gp];
+        const GpSigns<double> sg = {(double)sxi(gp),           (double)seta(gp),           (double)szeta(gp),
+                                    (double)(seta(gp) * szeta(gp)), (double)(sxi(gp) * szeta(gp)), (double)(sxi(gp) * seta(gp))};
+        ek = fma(hex_point_kinetic(vs, Cv, sg, rho), wJ[gp], ek);
     }
     return ek;
 }
@@ -881,6 +895,16 @@ __device__ __forceinline__ void hex_grad(const T* Jm, const T* Du, T* cJ, T* H, 
             H[i * 3 + j] = m * *rJ;
             if (i == j) Fd[i] = fma_t(m, *rJ, T(1));
         }
+}
+
+// Row i of tr(D cof(J)^T) for the gradient D of the displacement increment, from its coefficients a[m] (component i).
+template <typename T>
+__device__ __forceinline__ T hex_visc_trace(const T* a, const GpSigns<T>& s, const T* cJ) {
+#pragma clang fp contract(off)
+    const T d0 = fma_t(s.yz, a[6], fma_t(s.z, a[5], fma_t(s.y, a[3], a[0])));
+    const T d1 = fma_t(s.xz, a[6], fma_t(s.z, a[4], fma_t(s.x, a[3], a[1])));
+    const T d2 = fma_t(s.xy, a[6], fma_t(s.y, a[4], fma_t(s.x, a[5], a[2])));
+    return dot3(d0, cJ[0], d1, cJ[1], d2, cJ[2]);
 }
 
 // Stress at a hex8 Gauss point from hex_grad's H and Fd.
@@ -1019,9 +1043,8 @@ __device__ __forceinline__ double hex8_element(const MpsInst& I, int e, const do
                 const T a0 = vs[(0 * 3 + i) * MPS_PATCH], a1 = vs[(1 * 3 + i) * MPS_PATCH], a2 = vs[(2 * 3 + i) * MPS_PATCH];
                 const T a3 = vs[(3 * 3 + i) * MPS_PATCH], a4 = vs[(4 * 3 + i) * MPS_PATCH], a5 = vs[(5 * 3 + i) * MPS_PATCH];
                 const T a6 = vs[(6 * 3 + i) * MPS_PATCH];
-                tr += (a0 + s.y * a3 + s.z * a5 + s.yz * a6) * cJ[i * 3 + 0] +
-                      (a1 + s.x * a3 + s.z * a4 + s.xz * a6) * cJ[i * 3 + 1] +
-                      (a2 + s.x * a5 + s.y * a4 + s.xy * a6) * cJ[i * 3 + 2];
+                const T a[7] = {a0, a1, a2, a3, a4, a5, a6};
+                tr += hex_visc_trace(a, s, cJ + 3 * i);
             }
             add_bulk_visc<T>(H, tr * rJ * trs, qa, qb, P);
         }
@@ -1205,17 +1228,24 @@ __device__ __forceinline__ double tet_dt(const double (*x)[3], const double (*uu
 
 // Kinetic energy of tet4 element e at its Gauss point (dataExtraction.cpp:631-707): wJ rho/2 |v(gp)|^2 with
 // v(gp) = sum_a v_a / 4 (the shape values at (1/4, 1/4, 1/4)).
+__device__ __forceinline__ double tet_point_kinetic(const double (*v)[3], double rho, double wJ) {
+#pragma clang fp contract(off)
+    double kv = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        const double vel = 0.25 * (((v[0][j] + v[1][j]) + v[2][j]) + v[3][j]);
+        kv = fma(0.5 * rho * vel, vel, kv);
+    }
+    return kv * wJ;
+}
 __device__ __forceinline__ double tet_kinetic(const MpsInst& I, const int* nd, double rho, double wJ) {
     const size_t N = (size_t)I.N;
-    double vel[3] = {0.0, 0.0, 0.0};
+    double v[4][3];
 #pragma unroll
     for (int a = 0; a < 4; a++)
 #pragma unroll
-        for (int j = 0; j < 3; j++) vel[j] += 0.25 * I.v[j * N + nd[a]];
-    double kv = 0.0;
-#pragma unroll
-    for (int j = 0; j < 3; j++) kv += 0.5 * rho * vel[j] * vel[j];
-    return kv * wJ;
+        for (int j = 0; j < 3; j++) v[a][j] = I.v[j * N + nd[a]];
+    return tet_point_kinetic(v, rho, wJ);
 }
 
 template <typename T, int LAW, bool VISC = false, bool EN = false, bool O32 = false>
@@ -1339,8 +1369,8 @@ __device__ __forceinline__ void node_fext(const MpsInst& I, int n, uint32_t info
     }
 }
 
-__device__ __forceinline__ double node_fext1(const MpsInst& I, int n, uint32_t info, int i) {
-    if (info & MPS_NODE_LOADED) return I.lf[3 * (size_t)I.lidx[n] + i];
+__device__ __forceinline__ double node_fext1(const MpsInst& I, const double* __restrict__ lf, int n, uint32_t info, int i) {
+    if (info & MPS_NODE_LOADED) return lf[3 * (size_t)I.lidx[n] + i];
     return (i == 2 && I.fgrav) ? I.fgrav[n] : 0.0;
 }
 
@@ -1426,15 +1456,15 @@ __device__ __forceinline__ void load_item(const MpsInst& I, int n, uint32_t code
     }
 }
 
-// External force of the flagged nodes lb*MPS_LOAD_NODES .. +MPS_LOAD_NODES-1 at time t into lf, by one workgroup of 256
-// (NeumannBCManagement, boundaryConditions.cpp:75-140: zero, then the node's load items in input order).  32 lanes per
-// node take one item each and three of them add the items up in order, from sh (256*3 doubles): a node on a loaded face
-// has 16 items and more, whose dependent loads one work-item would walk through one after the other.  No barrier: a
-// node's lanes are half a wave.
-#define MPS_LOAD_NODES 8
+// External force at time t of the flagged nodes of workgroup lb, one per 32 work-items, into lf (NeumannBCManagement,
+// boundaryConditions.cpp:75-140: zero, then the node's load items in input order).  32 lanes per node take one item each
+// and three of them add the items up in order, from sh (3 doubles per work-item): a node on a loaded face has 16 items
+// and more, whose dependent loads one work-item would walk through one after the other.  No barrier: a node's lanes are
+// half a wave.
+#define MPS_LOAD_NODES 8  // per workgroup of 256
 __device__ __forceinline__ void loads_block(const MpsInst& I, int lb, double t, double* sh, double* lf) {
 #pragma clang fp contract(off)
-    const int l = threadIdx.x & 31, j = lb * MPS_LOAD_NODES + (int)(threadIdx.x >> 5);
+    const int l = threadIdx.x & 31, j = lb * (int)(blockDim.x >> 5) + (int)(threadIdx.x >> 5);
     const bool on = j < I.n_lnode;
     const int q0 = on ? I.lrow[j] : 0, q1 = on ? I.lrow[j + 1] : 0, n = on ? I.lnn[j] : 0;
     double* s = sh + (threadIdx.x & ~31) * 3;

@@ -17,9 +17,11 @@ bool elem_fuses_energy(const MpsInst& I);
 // (MPS_E_DEF, MPS_E_KIN) and MPS_N_PREV when the previous step ran in this launch.
 hipError_t launch_node(const MpsInst& I, int fuse, hipStream_t st, unsigned nflags);
 hipError_t launch_begin(const MpsInst& I, hipStream_t st);
-// Spread form (mps_spread.hip): step with index ci in a launch sequence that starts from u, v, a; the end of the
-// sequence (u, v, a of its last step); internal force at DOFs after it.
-hipError_t launch_spread(const MpsInst& I, int ci, hipStream_t st);
+// Spread form (mps_spread.hip): step with index ci in a launch sequence that starts from u, v, a (eflags: MPS_E_KIN when
+// the previous step is an energy step of this sequence); the end of the sequence (u, v, a of its last step); internal
+// force at DOFs after it; size of MpsInst::sp_ep.
+size_t spread_energy_doubles(const MpsInst& I);
+hipError_t launch_spread(const MpsInst& I, int ci, unsigned eflags, hipStream_t st);
 hipError_t launch_spread_end(const MpsInst& I, hipStream_t st);
 hipError_t launch_spread_pick(const MpsInst& I, const int32_t* idx, int64_t n, double* out, hipStream_t st);
 hipError_t launch_dt(const MpsInst& I, const double* u, unsigned long long* out, hipStream_t st);

@@ -20,6 +20,12 @@
 // 750 13.6 / 6.8, 10,400 12.9 / 6.8, 48,000 13.8 / 10.0, 93,800 14.6 / 18.0; FP32 form: 10,400 10.5 / 6.8, 48,000 11.3 /
 // 10.2, 93,800 12.0 / 16.7.  Every node is updated by all the workgroups that hold it (4.5 per 8 hex8 elements where the
 // patch form has 1.03 per element), so past the size where the lanes are no longer idle the patch form is the better one.
+// With energies every step and loads (hex8 FP64): 512 elements 29.8 / 7.7, 12,200 30.7 / 13.4, 35,800 31.4 / 28.6; tet4 750
+// 22.1 / 7.7, 55,600 22.1 / 14.3; with viscosity and loads (FP64 Belytschko): 512 24.0 / 7.0, 12,200 25.3 / 12.5, 31,700 29.1 /
+// 24.5.  The patch form takes three launches for these steps; here the external forces and the energy sums are extra
+// workgroups of the step's launch.
+// Tried: one wave per workgroup, which takes the dt and the forces in turn (half the waves): 2 us more at 1,000 elements and
+// the same above 30,000, where the issue of 1,380 vector instructions per 8 elements is the bound, not the waves in flight.
 // Tried: 16 and 32 hex8 elements per workgroup: fewer shared nodes, but 0.4 to 1.8 us more up to 2,000 elements and
 // nothing gained above.
 #include "../../include/mps_gpu.h"
@@ -167,17 +173,14 @@ __device__ __forceinline__ void lds_read(const T* __restrict__ p, T* v) {
 // Forces of a hex8 element by its eight lanes: lane j takes component j of the butterflies (j < 6), Gauss point j, its
 // share of the moment sums and node j.  sn: staged node values [9][ss] (X, u, X + u); lx: the element's local node indices.
 template <typename T>
-__device__ __forceinline__ void hex_coefficients(const double* __restrict__ sn, int ss, const uint16_t* __restrict__ lx,
-                                                 T* __restrict__ sc, int j) {
+__device__ __forceinline__ void hex_coefficients1(const double* __restrict__ s, const uint16_t* __restrict__ lx, T* __restrict__ c) {
 #pragma clang fp contract(off)
-    if (j < 6) {
-        const double* s = sn + j * ss;
+    {
         double x[8], A[7];
 #pragma unroll
         for (int a = 0; a < 8; a++) x[a] = s[lx[a]];
         hex_butterfly1(x, A);
         const double g = MPS_GP;
-        T* c = sc + (j < 3 ? j : 18 + j);
         c[0] = (T)(0.125 * A[0]);
         c[3] = (T)(0.125 * A[1]);
         c[6] = (T)(0.125 * A[2]);
@@ -187,8 +190,25 @@ __device__ __forceinline__ void hex_coefficients(const double* __restrict__ sn, 
         c[18] = (T)((0.125 * g * g) * A[6]);
     }
 }
-template <typename T, int LAW>
-__device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restrict__ sq, int j, double pa, double pb, T* f) {
+template <typename T>
+__device__ __forceinline__ void hex_coefficients(const double* __restrict__ sn, int ss, const uint16_t* __restrict__ lx,
+                                                 T* __restrict__ sc, int j) {
+    if (j < 6) hex_coefficients1<T>(sn + j * ss, lx, sc + (j < 3 ? j : 18 + j));
+}
+
+// What the element phase adds to the forces (step modes): bulk viscosity from the displacement increments of the step
+// (coefficients sv of the element, qa and qb of visc_coeffs, rdt = 1/dt), or the step's energies (en: W(F), det F and wJ
+// of the lane's Gauss point).
+enum { kPlain = 0, kVisc = 1, kEnergy = 2 };
+template <typename T>
+struct StepExtra {
+    const T* sv;
+    T qa, qb, rdt;
+    double en[3];
+};
+template <typename T, int LAW, int MODE>
+__device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restrict__ sq, int j, double pa, double pb, T* f,
+                                                 StepExtra<T>& ex) {
 #pragma clang fp contract(off)
     {  // Gauss point j
         T A[44];
@@ -200,7 +220,26 @@ __device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restri
         hex_jac<T>(Ax, s, Jm);
         hex_jac<T>(Au, s, Du);
         hex_grad<T>(Jm, Du, cJ, H, Fd, &dJ, &rJ);
-        hex_pk1<LAW>(H, Fd, (T)pa, (T)pb, P);
+        if constexpr (MODE == kEnergy) {  // weight 1: wJ = |det J|
+            double Wg, Jg;
+            hex_pk1<LAW>(H, Fd, pa, pb, P, &Wg, &Jg);
+            ex.en[0] = Wg;
+            ex.en[1] = Jg;
+            ex.en[2] = fabs(dJ);
+        } else {
+            hex_pk1<LAW>(H, Fd, (T)pa, (T)pb, P);
+        }
+        if constexpr (MODE == kVisc) {
+            T tr = T(0);
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                T a[7];
+#pragma unroll
+                for (int m = 0; m < 7; m++) a[m] = ex.sv[m * 3 + i];
+                tr += hex_visc_trace(a, s, cJ + 3 * i);
+            }
+            add_bulk_visc<T>(H, tr * rJ * ex.rdt, ex.qa, ex.qb, P);
+        }
         hex_stress_columns<T>(P, cJ, dJ, Q);
 #pragma unroll
         for (int k = 0; k < 3; k++)
@@ -346,27 +385,224 @@ template <typename T, int NEN>
 constexpr size_t fixed_lds() {
     return NEN == 8 ? sizeof(T) * MPS_SPREAD_HEX * (kCol + kCoef + kArea + (sizeof(T) == 4 ? kPos : 0)) : 0;
 }
-// Bytes of dynamic LDS: staged node values (hex8 X, u, X + u; tet4 X, u), then the element phase's arrays.
-template <int NEN>
+// Bytes of dynamic LDS: staged node values (hex8 X, u, X + u; tet4 X, u; with viscosity the increments, with energies the
+// velocities), then the element phase's arrays.
+template <int NEN, int MODE>
 __host__ __device__ size_t stage_lds(int ss) {
-    return ((size_t)(NEN == 8 ? 9 : 6) * ss * 8 + 15) / 16 * 16;
+    return ((size_t)((NEN == 8 ? 9 : 6) + (MODE != kPlain ? 3 : 0)) * ss * 8 + 15) / 16 * 16;
+}
+constexpr int kVisc21 = 22, kKin = 26;  // per element: viscosity coefficients; velocity sums and coefficients
+template <typename T, int NEN, int MODE>
+size_t spread_lds(const MpsInst& I) {
+    size_t b = stage_lds<NEN, MODE>(I.sp_stride) + fixed_lds<T, NEN>() + (MODE == kVisc ? sizeof(T) * MPS_SPREAD_HEX * kVisc21 : 0) +
+               (MODE == kEnergy && NEN == 8 ? 8 * MPS_SPREAD_HEX * kKin : 0);
+    const size_t loads = I.n_lnode > 0 ? 3 * 8 * (size_t)spread_threads<NEN>() : 0;
+    return b > loads ? b : loads;
+}
+
+// ---------------------------------------------------------------------------
+// Energies.  A step's sums are added up while later steps run: the kernel with index ci leaves the energies of each element
+// (DEFO_ENERGY and VOLUME of step k, KIN_ENERGY of step k-1) and the node sums of each of its waves (step k-1); a few
+// workgroups of the next kernel add the elements of a patch or 256 workgroups' node sums, and one of the kernel after that
+// adds those and writes the history.  One workgroup for all of them took as long as the step itself.  The elements are
+// added in the patch form's order (block_sum of a patch, reduce_parts of the patches), the node sums in one of their own;
+// neither depends on where the launch sequences end.
+// ---------------------------------------------------------------------------
+constexpr int kRows = 256;
+__host__ __device__ __forceinline__ int ep_groups(int nb) { return (nb + kRows - 1) / kRows; }
+template <int NEN>
+constexpr int ep_width() {  // node sums of a workgroup
+    return MPS_NODE_PARTS * (spread_threads<NEN>() / 64);
+}
+// Sets 0 and 1 by the parity of the kernel's index; set 2 of the node sums: the end of a sequence (its last step).
+template <int NEN>
+__device__ __forceinline__ double* ep_rows(const MpsInst& I, int set) {
+    return I.sp_ep + (size_t)set * I.sp_nb * ep_width<NEN>();
+}
+template <int NEN>
+__device__ __forceinline__ double* ep_sums(const MpsInst& I, int set) {  // of the groups
+    return ep_rows<NEN>(I, 3) + (size_t)set * ep_groups(I.sp_nb) * MPS_NODE_PARTS;
+}
+template <int NEN>
+__device__ __forceinline__ double* ep_patches(const MpsInst& I, int set) {  // element sums of the patches
+    return ep_sums<NEN>(I, 3) + (size_t)set * 3 * I.n_patch;
+}
+template <int NEN>
+__device__ __forceinline__ double* ep_elems(const MpsInst& I, int set) {  // [3][Ne]
+    return ep_patches<NEN>(I, 2) + (size_t)set * 3 * I.Ne;
+}
+
+// Sum over the lanes of a wave of NV values, in every lane.
+template <int NV>
+__device__ __forceinline__ void wave_sum(double* v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+        for (int j = 0; j < NV; j++) v[j] += __shfl_xor(v[j], off, 64);
+}
+// block_sum of 256 work-items by a workgroup of fewer waves: get(i, v) gives the values of work-item i.
+template <int NV, typename F>
+__device__ __forceinline__ void sum256(F get, double* out, double* sh) {
+    const int lane = threadIdx.x & 63;
+    __syncthreads();  // an earlier call may still be reading sh
+    for (int w = threadIdx.x >> 6; w < 4; w += blockDim.x >> 6) {
+        double v[NV];
+        get(w * 64 + lane, v);
+        wave_sum<NV>(v);
+        if (lane == 0)
+#pragma unroll
+            for (int j = 0; j < NV; j++) sh[w * NV + j] = v[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NV; j++) out[j] = ((sh[j] + sh[NV + j]) + sh[2 * NV + j]) + sh[3 * NV + j];
+}
+// The nb entries of NV values at part: work-item i takes i, i + 256, ... (reduce_parts of a workgroup of 256).
+template <int NV>
+__device__ __forceinline__ void sum_parts(const double* __restrict__ part, int nb, double* out, double* sh) {
+    sum256<NV>([&](int i, double* v) {
+#pragma unroll
+        for (int j = 0; j < NV; j++) v[j] = 0.0;
+        for (int b = i; b < nb; b += 256)
+#pragma unroll
+            for (int j = 0; j < NV; j++) v[j] += part[(size_t)b * NV + j];
+    }, out, sh);
+}
+// Element sums of entry x (the patch that workgroup x of the patch form computes), and node sums of group x, of a set, by
+// the calling workgroup.
+template <int NEN>
+__device__ __forceinline__ void ep_add_patch(const MpsInst& I, int set, int x, double* sh) {
+    const double* ee = ep_elems<NEN>(I, set);
+    const int p = xcd_tile(x, I.n_patch);
+    double t[3];
+    sum256<3>([&](int i, double* v) {
+        const int e = p * MPS_PATCH + i;
+#pragma unroll
+        for (int j = 0; j < 3; j++) v[j] = e < I.Ne ? ee[(size_t)j * I.Ne + e] : 0.0;
+    }, t, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int j = 0; j < 3; j++) ep_patches<NEN>(I, set)[3 * x + j] = t[j];
+}
+template <int NEN>
+__device__ __forceinline__ void ep_add_group(const MpsInst& I, int set, int x, double* sh) {
+    constexpr int NW = spread_threads<NEN>() / 64;
+    const double* rows = ep_rows<NEN>(I, set);
+    double t[MPS_NODE_PARTS];
+    sum256<MPS_NODE_PARTS>([&](int i, double* v) {
+        const int b = x * kRows + i;
+#pragma unroll
+        for (int j = 0; j < MPS_NODE_PARTS; j++) {
+            v[j] = 0.0;
+#pragma unroll
+            for (int w = 0; w < NW; w++) v[j] += b < I.sp_nb ? rows[(size_t)b * ep_width<NEN>() + w * MPS_NODE_PARTS + j] : 0.0;
+        }
+    }, t, sh);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int j = 0; j < MPS_NODE_PARTS; j++) ep_sums<NEN>(I, set)[x * MPS_NODE_PARTS + j] = t[j];
+}
+// Node sums t of step j into the running works and the history (by one work-item).
+__device__ __forceinline__ void node_history(const MpsInst& I, long long j, const double* t) {
+    MpsCtl* ctl = I.ctl;
+    ctl->w_ext += t[0];
+    ctl->w_react += t[1];
+    *hist_at(I, MPS_H_WEXT, j) = ctl->w_ext;
+    *hist_at(I, MPS_H_WREACT, j) = ctl->w_react;
+    if (j % I.energy_every == 0) {
+        *hist_at(I, MPS_H_EKL, j) = t[2];
+        *hist_at(I, MPS_H_EEXT, j) = t[3];
+    }
+    ctl->wred = j;
+}
+// Sums of the kernel with index s of the sequence that starts at step A into the history, by the calling workgroup.
+template <int NEN>
+__device__ __forceinline__ void spread_history(const MpsInst& I, long long A, int s, double* sh) {
+    double el[3], nd[MPS_NODE_PARTS];
+    sum_parts<3>(ep_patches<NEN>(I, s & 1), I.n_patch, el, sh);
+    sum_parts<MPS_NODE_PARTS>(ep_sums<NEN>(I, s & 1), ep_groups(I.sp_nb), nd, sh);
+    if (threadIdx.x != 0 || I.hist_cap <= 0) return;
+    const long long k = A + s;
+    if (k % I.energy_every == 0) {
+        *hist_at(I, MPS_H_EDEF, k) = el[0];
+        *hist_at(I, MPS_H_VOL, k) = el[1];
+    }
+    if (s == 0) return;
+    if ((k - 1) % I.energy_every == 0) *hist_at(I, MPS_H_EKIN, k - 1) = el[2];
+    node_history(I, k - 1, nd);
+}
+// Energy terms of DOF (n, d) at step k, by the owner of the node (node_energy_forces and node_energy_motion for one
+// direction): u the step's displacement, incr its increment, fi and fe the forces, m, v and wkin as the update leaves them.
+__device__ __forceinline__ void dof_energy(const MpsInst& I, int n, uint32_t info, int d, long long k, double u, double incr,
+                                           double fi, double fe, double m, double v, double wkin, double* red) {
+    double fp = fe;
+    if (info & MPS_NODE_LOADED) {
+        double* lp = I.lfprev + 3 * (size_t)I.lidx[n] + d;
+        fp = *lp;
+        *lp = fe;
+    }
+    double wr = wkin;
+    if ((info >> d) & 1u) {
+        double* rp = I.rprev + 3 * (size_t)((info & MPS_REC_MASK) >> 3) + d;
+        const double r = fi - fe;
+        wr += 0.5 * (*rp + r) * incr;
+        *rp = r;
+    }
+    if (k >= 2) {
+        red[0] += 0.5 * (fp + fe) * incr;
+        red[1] += wr;
+    }
+    red[2] += 0.5 * m * v * v;
+    red[3] += u * fe;
+}
+
+// External force of the step with index ci (its flagged nodes, two sets by parity).
+__device__ __forceinline__ double* spread_lf(const MpsInst& I, int ci) {
+    return I.lf + (ci & 1 ? 3 * (size_t)I.n_lnode : 0);
+}
+
+// The workgroups of a step kernel before its element workgroups: with energies the patches, the groups and the history,
+// then the external forces of the step.
+template <int NEN, int MODE>
+__device__ __forceinline__ void spread_side(const MpsInst& I, int ci, int x, long long A, double time, double* sh) {
+    if constexpr (MODE == kEnergy) {
+        const int G = ep_groups(I.sp_nb), P = I.n_patch;
+        if (x <= P + G) {
+            if (x < P + G && ci >= 1) {
+                if (x < P) ep_add_patch<NEN>(I, (ci - 1) & 1, x, sh);
+                else ep_add_group<NEN>(I, (ci - 1) & 1, x - P, sh);
+            } else if (x == P + G && ci >= 2) {
+                spread_history<NEN>(I, A, ci - 2, sh);
+            }
+            return;
+        }
+        x -= P + G + 1;
+    }
+    loads_block(I, x, time, sh, spread_lf(I, ci));
+}
+template <int NEN, int MODE>
+unsigned side_blocks(const MpsInst& I) {
+    constexpr int per = spread_threads<NEN>() / 32;
+    return (MODE == kEnergy ? (unsigned)(I.n_patch + ep_groups(I.sp_nb)) + 1 : 0u) + (unsigned)((I.n_lnode + per - 1) / per);
 }
 
 }  // namespace
 
 // Step k = A + ci, ci its index in the launch sequence: solve of step k-1 (ci > 0), begin of step k, its element forces
-// and the stable dt for step k+1 (the file's head).
-template <typename T, int NEN, int LAW>
-__global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int ci) {
+// and the stable dt for step k+1 (the file's head).  eflags (energies): MPS_E_KIN.
+template <typename T, int NEN, int LAW, int MODE>
+__global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int ci, unsigned eflags) {
     extern __shared__ __align__(16) double smem[];
     constexpr int EB = NEN == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET;  // elements of a workgroup
     __shared__ uint16_t slx[NEN == 8 ? EB * 8 : 1];
     constexpr int NT = spread_threads<NEN>(), FLIGHT = NEN == 8 ? 8 : 16;
-    const int b = xcd_tile(blockIdx.x, gridDim.x), t = threadIdx.x, ss = I.sp_stride;
+    const int nside = (int)gridDim.x - I.sp_nb, bx = (int)blockIdx.x - nside;  // workgroups of spread_side come first
+    const bool side = bx < 0;
+    const int b = side ? 0 : xcd_tile(bx, I.sp_nb), t = threadIdx.x, ss = I.sp_stride;
     // tables first: their addresses depend on nothing.  Work item it: direction it % 3 of the workgroup's node it / 3.
     const int4* tab = I.sp_node + (size_t)b * ss;
     int4 E = make_int4(-1, 0, 0, 0);
-    if (t < 3 * ss) E = tab[t / 3];
+    if (t < 3 * ss && !side) E = tab[t / 3];
     // role in the element phase: wave of forces or of stable dt
     const bool force = t < 64;
     const int lane = t & 63, j = t & 7;
@@ -407,7 +643,7 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
     if (E.x != -1) L.load(I, E, t - 3 * (t / 3), ci == 0, ur, wr, fr);
     MpsStepSlot nx;
     const int st = begin_scalars(I, k, prev, row_min(m16), &nx);
-    if (blockIdx.x == 0 && t == 0) {
+    if (bx == 0 && t == 0) {
         ctl->sslot[ci & 1] = nx;
         if (st != MPSD_RUNNING) ctl->status = st;
         if (nx.go) {
@@ -421,6 +657,13 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
         spread_reset(I, (ci + 2) % 3);
     }
     if (!nx.go) return;
+    if (side) {
+        spread_side<NEN, MODE>(I, ci, (int)blockIdx.x, A, nx.time, smem);
+        return;
+    }
+    const double* lf = spread_lf(I, ci + 1);  // step k-1
+    double red[MPS_NODE_PARTS] = {0.0, 0.0, 0.0, 0.0};
+    double* se = smem + (NEN == 8 ? 9 : 6) * ss;  // staged increments or velocities: se[d*ss + q]
     for (int it = t; it < 3 * ss; it += NT) {
         const int q = it / 3, d = it - 3 * q;
         if (it != t) {
@@ -433,13 +676,20 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
         if (ci == 0) {
             w = half_velocity(nx.dt, L.w, L.m);
         } else {
-            double v, acc;
-            const double fi = L.force(E, fr, d);
-            node_update1(I, L.info, d, k - 1, prev.dt, L.m, -fi + node_fext1(I, n, L.info, d), L.w, &v, &acc);
+            double v, acc, wkin = 0.0;
+            const double fi = L.force(E, fr, d), fe = node_fext1(I, lf, n, L.info, d);
+            node_update1(I, L.info, d, k - 1, prev.dt, L.m, -fi + fe, L.w, &v, &acc, MODE == kEnergy ? &wkin : nullptr);
             if (E.x < 0) check_finite(I, n, d, k - 1, u);
+            if constexpr (MODE == kEnergy) {
+                se[d * ss + q] = v;
+                if (E.x < 0)
+                    dof_energy(I, n, L.info, d, k - 1, u, step_increment(I, L.info, d, k - 1, prev.dt, L.w), fi, fe, L.m, v,
+                               wkin, red);
+            }
             w = half_velocity(nx.dt, v, acc);
         }
         u += step_increment(I, L.info, d, k, nx.dt, w);
+        if constexpr (MODE == kVisc) se[d * ss + q] = u - L.u;
         if (E.x < 0) {
             uo[d * N + n] = u;
             wo[d * N + n] = w;
@@ -454,21 +704,80 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
         }
     }
     __syncthreads();
+    StepExtra<T> ex;
+    double* sums = ep_rows<NEN>(I, ci & 1) + (size_t)b * ep_width<NEN>();
+    const auto node_row = [&]() {  // the wave's node sums of step k-1
+        wave_sum<MPS_NODE_PARTS>(red);
+        if (lane == 0)
+#pragma unroll
+            for (int j = 0; j < MPS_NODE_PARTS; j++) sums[(t >> 6) * MPS_NODE_PARTS + j] = red[j];
+    };
+    double* ee = ep_elems<NEN>(I, ci & 1);  // the elements' energies
     T* fo = spread_forces<T>(I, ci);
     unsigned long long dmin = 0x7FF0000000000000ull;
     if constexpr (NEN == 8) {
-        T* base = reinterpret_cast<T*>(reinterpret_cast<char*>(smem) + stage_lds<8>(ss));
+        T* base = reinterpret_cast<T*>(reinterpret_cast<char*>(smem) + stage_lds<8, MODE>(ss));
         T* sc = base + EB * kCol;  // the elements' coefficients
         if (force) hex_coefficients<T>(smem, ss, slx + el * 8, sc + el * kCoef, j);
+        double* sk = reinterpret_cast<double*>(reinterpret_cast<char*>(base) + fixed_lds<T, 8>());
+        if constexpr (MODE == kEnergy) {  // sums and coefficients of the nodal velocities (hex_kinetic)
+            if ((eflags & MPS_E_KIN) && force && j < 3) {
+                double x[8], A[7], sum = 0.0;
+#pragma unroll
+                for (int a = 0; a < 8; a++) {
+                    x[a] = se[j * ss + slx[el * 8 + a]];
+                    sum += x[a];
+                }
+                hex_butterfly1(x, A);
+                double* c = sk + el * kKin + j;
+                c[0] = sum;
+#pragma unroll
+                for (int m = 0; m < 7; m++) c[3 * (m + 1)] = A[m];
+            }
+        }
+        if constexpr (MODE == kVisc) {
+            T* sv = reinterpret_cast<T*>(reinterpret_cast<char*>(base) + fixed_lds<T, 8>()) + el * kVisc21;
+            if (force && j < 3) hex_coefficients1<T>(se + j * ss, slx + el * 8, sv + j);
+            double da, db;
+            visc_coeffs(I, ec, kc.c, &da, &db);
+            ex.sv = sv;
+            ex.qa = (T)da;
+            ex.qb = (T)db;
+            ex.rdt = (T)(nx.dt == 0.0 ? 0.0 : 1 / nx.dt);
+        }
         if constexpr (sizeof(T) == 4) __syncthreads();  // the FP32 lengths are taken from the coefficients
         else wave_sync();
         if (force) {
             T f[3];
-            hex_spread_force<T, LAW>(sc + el * kCoef, base + el * kCol, j, kc.pa, kc.pb, f);
+            hex_spread_force<T, LAW, MODE>(sc + el * kCoef, base + el * kCol, j, kc.pa, kc.pb, f, ex);
             if (mine) {
                 T* dst = fo + 3 * (size_t)pos[0];
 #pragma unroll
                 for (int i = 0; i < 3; i++) dst[i] = f[i];
+            }
+            if constexpr (MODE == kEnergy) {
+                // the points' values to LDS (over the columns), where three lanes of an element add them in order
+                double* sp = reinterpret_cast<double*>(base + el * kCol);
+                double kv = 0.0;
+                if (eflags & MPS_E_KIN) {
+                    const double* c = sk + el * kKin;
+                    double vc[24];
+                    lds_read<24>(c, vc);
+                    kv = hex_point_kinetic(vc, reinterpret_cast<const double(*)[3]>(vc + 3), gp_signs<double>(j),
+                                           I.rho ? I.rho[ec] : I.rho0);
+                }
+                sp[j * 4] = ex.en[0];
+                sp[j * 4 + 1] = ex.en[1];
+                sp[j * 4 + 2] = kv;
+                sp[j * 4 + 3] = ex.en[2];
+                wave_sync();
+                if (j < 3 && mine) {
+                    double sum = 0.0;
+#pragma unroll
+                    for (int gp = 0; gp < 8; gp++) sum = fma(sp[gp * 4 + j], sp[gp * 4 + 3], sum);
+                    ee[(size_t)j * I.Ne + e] = sum;
+                }
+                node_row();
             }
             return;
         }
@@ -476,20 +785,40 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
                                             lane, kc.c, kc.l0);
         if (lane < 8 && mine) dmin = d2bits(dte);
     } else {
-        if (t >= 128) return;
+        if (t >= 128) {
+            if constexpr (MODE == kEnergy) node_row();
+            return;
+        }
         const int l[4] = {(int)(l4.x & 0xffffu), (int)(l4.x >> 16), (int)(l4.y & 0xffffu), (int)(l4.y >> 16)};
         double x[4][3], uu[4][3];
 #pragma unroll
         for (int a = 0; a < 4; a++) staged_node(smem, l[a], x[a], uu[a]);
         if (force) {
             T f[4][3];
-            tet4_core<T, LAW, false>(I, e, nullptr, x, uu, kc, f, false, 0.0);
-            if (!mine) return;
+            double r[4];
+            tet4_core<T, LAW, false, MODE == kEnergy>(I, e, nullptr, x, uu, kc, f, false, 0.0, r);
+            if (mine) {
 #pragma unroll
-            for (int a = 0; a < 4; a++) {
-                T* dst = fo + 3 * (size_t)pos[a];
+                for (int a = 0; a < 4; a++) {
+                    T* dst = fo + 3 * (size_t)pos[a];
 #pragma unroll
-                for (int i = 0; i < 3; i++) dst[i] = f[a][i];
+                    for (int i = 0; i < 3; i++) dst[i] = f[a][i];
+                }
+            }
+            if constexpr (MODE == kEnergy) {
+                if (mine) {
+                    ee[e] = r[0];
+                    ee[(size_t)I.Ne + e] = r[1];
+                    if (eflags & MPS_E_KIN) {
+                        double v[4][3];
+#pragma unroll
+                        for (int a = 0; a < 4; a++)
+#pragma unroll
+                            for (int d = 0; d < 3; d++) v[a][d] = se[d * ss + l[a]];
+                        ee[2 * (size_t)I.Ne + e] = tet_point_kinetic(v, I.rho ? I.rho[e] : I.rho0, r[3]);
+                    }
+                }
+                node_row();
             }
             return;
         }
@@ -500,11 +829,13 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
 #pragma unroll
     for (int off = NEN == 8 ? 4 : 32; off > 0; off >>= 1) dmin = umin64(dmin, (unsigned long long)__shfl_xor((long long)dmin, off, 64));
     if (lane == 0) atomicMin(dt_spread(I, (ci + 1) % 3, b & (MPS_DT_SLOTS - 1)), dmin);
+    if constexpr (MODE == kEnergy) node_row();
 }
 
 // After a launch sequence: solve of its last step (B), from the buffer that step wrote, into u, v and a.
-template <typename T>
-__global__ __launch_bounds__(256) void k_spread_end(MpsInst I) {
+template <typename T, int NEN, int MODE>
+__global__ __launch_bounds__(spread_threads<NEN>()) void k_spread_end(MpsInst I) {
+    constexpr int NT = spread_threads<NEN>();
     const MpsCtl* ctl = I.ctl;
     const long long A = ctl->A, k = ctl->B;
     if (k < A) return;  // no step was begun
@@ -514,32 +845,66 @@ __global__ __launch_bounds__(256) void k_spread_end(MpsInst I) {
     double *ur, *wr;
     uw_buffers(I, (int)((k - A) & 1) ^ 1, &ur, &wr);
     const T* fr = spread_forces<T>(I, (int)(k - A));
-    for (int it = threadIdx.x; it < 3 * ss; it += 256) {
+    const double* lf = spread_lf(I, (int)(k - A));
+    double red[MPS_NODE_PARTS] = {0.0, 0.0, 0.0, 0.0};
+    const int b = xcd_tile(blockIdx.x, gridDim.x);
+    for (int it = threadIdx.x; it < 3 * ss; it += NT) {
         const int q = it / 3, d = it - 3 * q;
-        const int4 E = I.sp_node[(size_t)xcd_tile(blockIdx.x, gridDim.x) * ss + q];
+        const int4 E = I.sp_node[(size_t)b * ss + q];
         if (E.x == -1) break;
         if (E.x >= 0) continue;  // another workgroup owns the node
         const int n = E.x & 0x7FFFFFFF;
         const size_t i = d * N + n;
         NodeLoads<T, 8> L;
         L.load(I, E, d, false, ur, wr, fr);
-        double v, a;
-        const double u = L.u, fi = L.force(E, fr, d);
-        node_update1(I, L.info, d, k, dt, L.m, -fi + node_fext1(I, n, L.info, d), L.w, &v, &a);
+        double v, a, wkin = 0.0;
+        const double u = L.u, fi = L.force(E, fr, d), fe = node_fext1(I, lf, n, L.info, d);
+        node_update1(I, L.info, d, k, dt, L.m, -fi + fe, L.w, &v, &a, MODE == kEnergy ? &wkin : nullptr);
         check_finite(I, n, d, k, u);
+        if constexpr (MODE == kEnergy)
+            dof_energy(I, n, L.info, d, k, u, step_increment(I, L.info, d, k, dt, L.w), fi, fe, L.m, v, wkin, red);
         I.u[i] = u;
         I.v[i] = v;
         I.a[i] = a;
     }
+    if constexpr (MODE == kEnergy) {
+        wave_sum<MPS_NODE_PARTS>(red);
+        double* sums = ep_rows<NEN>(I, 2) + (size_t)b * ep_width<NEN>();
+        if ((threadIdx.x & 63) == 0)
+#pragma unroll
+            for (int j = 0; j < MPS_NODE_PARTS; j++) sums[(threadIdx.x >> 6) * MPS_NODE_PARTS + j] = red[j];
+    }
+}
+
+// Sums that no step kernel has added up yet: the patches and groups of the last step kernel, the groups of the end.
+template <int NEN>
+__global__ __launch_bounds__(spread_threads<NEN>()) void k_spread_groups(MpsInst I) {
+    __shared__ double sh[MPS_NODE_PARTS * 4];
+    const long long A = I.ctl->A, k = I.ctl->B;
+    if (k < A) return;
+    const int G = ep_groups(I.sp_nb), P = I.n_patch, x = blockIdx.x, set = (int)(k - A) & 1;
+    if (x < P) ep_add_patch<NEN>(I, set, x, sh);
+    else if (x < P + G) ep_add_group<NEN>(I, set, x - P, sh);
+    else ep_add_group<NEN>(I, 2, x - P - G, sh);
 }
 
 // Closes a launch sequence: its steps count as done, and the scalars and the pending min go where the patch form and the
-// next sequence find them.
-__global__ __launch_bounds__(64) void k_spread_close(MpsInst I) {
+// next sequence find them.  Energies: KIN_ENERGY of the last step is left to the standalone pass.
+template <int NEN, int MODE>
+__global__ __launch_bounds__(MODE == kEnergy ? spread_threads<NEN>() : 64) void k_spread_close(MpsInst I) {
     MpsCtl* ctl = I.ctl;
     const long long A = ctl->A, k = ctl->B;
     if (k < A) return;
     const int ci = (int)(k - A);
+    if constexpr (MODE == kEnergy) {  // the sums that no step kernel has added up yet, in order
+        __shared__ double sh[MPS_NODE_PARTS * 4];
+        if (ci >= 1) spread_history<NEN>(I, A, ci - 1, sh);
+        spread_history<NEN>(I, A, ci, sh);
+        double t[MPS_NODE_PARTS];
+        sum_parts<MPS_NODE_PARTS>(ep_sums<NEN>(I, 2), ep_groups(I.sp_nb), t, sh);
+        if (threadIdx.x == 0 && I.hist_cap > 0) node_history(I, k, t);
+        __syncthreads();  // every thread has read the control block
+    }
     const unsigned long long mb = row_min(*dt_spread(I, (ci + 1) % 3, threadIdx.x & (MPS_DT_SLOTS - 1)));
     if (threadIdx.x != 0) return;
     MpsStepSlot s = ctl->sslot[ci & 1];
@@ -569,21 +934,41 @@ __global__ void k_spread_pick(MpsInst I, const int32_t* __restrict__ idx, int64_
 
 namespace mpsk {
 
-hipError_t launch_spread(const MpsInst& I, int ci, hipStream_t st) {
+static int spread_mode(const MpsInst& I) { return I.energy_every > 0 ? kEnergy : I.uprev != nullptr ? kVisc : kPlain; }
+
+size_t spread_energy_doubles(const MpsInst& I) {
+    const size_t nb = (size_t)I.sp_nb, w = (size_t)(I.nen == 8 ? ep_width<8>() : ep_width<4>());
+    return 3 * (nb * w + (size_t)ep_groups(I.sp_nb) * MPS_NODE_PARTS) + 2 * 3 * ((size_t)I.n_patch + (size_t)I.Ne);
+}
+
+hipError_t launch_spread(const MpsInst& I, int ci, unsigned eflags, hipStream_t st) {
     const unsigned nb = (unsigned)I.sp_nb;
-#define MPS_SPREAD(T, NEN, LAW) \
-    k_spread<T, NEN, LAW><<<nb, spread_threads<NEN>(), stage_lds<NEN>(I.sp_stride) + fixed_lds<T, NEN>(), st>>>(I, ci)
-#define MPS_SPREAD_LAW(T, NEN)                       \
-    switch (I.law) {                                 \
-        case 0: MPS_SPREAD(T, NEN, 0); break;        \
-        case 1: MPS_SPREAD(T, NEN, 1); break;        \
-        case 2: MPS_SPREAD(T, NEN, 2); break;        \
-        default: MPS_SPREAD(T, NEN, 3); break;       \
+#define MPS_SPREAD(T, NEN, LAW, M) \
+    k_spread<T, NEN, LAW, M><<<nb + side_blocks<NEN, M>(I), spread_threads<NEN>(), spread_lds<T, NEN, M>(I), st>>>(I, ci, eflags)
+#define MPS_SPREAD_LAW(T, NEN, M)                       \
+    switch (I.law) {                                    \
+        case 0: MPS_SPREAD(T, NEN, 0, M); break;        \
+        case 1: MPS_SPREAD(T, NEN, 1, M); break;        \
+        case 2: MPS_SPREAD(T, NEN, 2, M); break;        \
+        default: MPS_SPREAD(T, NEN, 3, M); break;       \
     }
+    const int mode = spread_mode(I);
     if (I.nen == 8) {
-        if (I.precision == 1) { MPS_SPREAD_LAW(float, 8) } else { MPS_SPREAD_LAW(double, 8) }
+        if (I.precision == 1) {
+            if (mode == kVisc) { MPS_SPREAD_LAW(float, 8, kVisc) } else { MPS_SPREAD_LAW(float, 8, kPlain) }
+        } else if (mode == kVisc) {
+            MPS_SPREAD_LAW(double, 8, kVisc)
+        } else if (mode == kEnergy) {
+            MPS_SPREAD_LAW(double, 8, kEnergy)
+        } else {
+            MPS_SPREAD_LAW(double, 8, kPlain)
+        }
+    } else if (I.precision == 1) {
+        MPS_SPREAD_LAW(float, 4, kPlain)
+    } else if (mode == kEnergy) {
+        MPS_SPREAD_LAW(double, 4, kEnergy)
     } else {
-        if (I.precision == 1) { MPS_SPREAD_LAW(float, 4) } else { MPS_SPREAD_LAW(double, 4) }
+        MPS_SPREAD_LAW(double, 4, kPlain)
     }
 #undef MPS_SPREAD_LAW
 #undef MPS_SPREAD
@@ -592,11 +977,30 @@ hipError_t launch_spread(const MpsInst& I, int ci, hipStream_t st) {
 
 hipError_t launch_spread_end(const MpsInst& I, hipStream_t st) {
     const unsigned nb = (unsigned)I.sp_nb;
-    if (I.precision == 1) k_spread_end<float><<<nb, 256, 0, st>>>(I);
-    else k_spread_end<double><<<nb, 256, 0, st>>>(I);
+    const bool en = spread_mode(I) == kEnergy;
+#define MPS_SPREAD_END(T, NEN, M) k_spread_end<T, NEN, M><<<nb, spread_threads<NEN>(), 0, st>>>(I)
+    if (I.nen == 8) {
+        if (I.precision == 1) MPS_SPREAD_END(float, 8, kPlain);
+        else if (en) MPS_SPREAD_END(double, 8, kEnergy);
+        else MPS_SPREAD_END(double, 8, kPlain);
+    } else {
+        if (I.precision == 1) MPS_SPREAD_END(float, 4, kPlain);
+        else if (en) MPS_SPREAD_END(double, 4, kEnergy);
+        else MPS_SPREAD_END(double, 4, kPlain);
+    }
+#undef MPS_SPREAD_END
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    k_spread_close<<<1, 64, 0, st>>>(I);
+    const unsigned groups = (unsigned)I.n_patch + 2 * (unsigned)ep_groups(I.sp_nb);
+    if (!en) {
+        k_spread_close<8, kPlain><<<1, 64, 0, st>>>(I);
+    } else if (I.nen == 8) {
+        k_spread_groups<8><<<groups, spread_threads<8>(), 0, st>>>(I);
+        k_spread_close<8, kEnergy><<<1, spread_threads<8>(), 0, st>>>(I);
+    } else {
+        k_spread_groups<4><<<groups, spread_threads<4>(), 0, st>>>(I);
+        k_spread_close<4, kEnergy><<<1, spread_threads<4>(), 0, st>>>(I);
+    }
     return hipGetLastError();
 }
 
