@@ -949,18 +949,18 @@ __device__ __forceinline__ void hex_stress_columns(T* P, const T* cJ, T dJ, T (*
 // GPs' wJ go to vs[gp*MPS_PATCH] (an LDS array apart from the force slots), for the kinetic energy, which the
 // element kernel computes after the force phase (hex_kinetic).
 // ---------------------------------------------------------------------------
+// cpre: the element's connectivity, loaded ahead.
 // dtsk (FP64): the element kernel's dt skip threshold (MpsCtl::dt_skip; +inf: none).  A wave whose elements all
 // have hex_dt_above(dtsk) returns +inf as their dt and skips the strict length.
 template <typename T, int LAW, bool VISC = false, bool EN = false, bool O32 = false>
 __device__ __forceinline__ double hex8_element(const MpsInst& I, int e, const double* __restrict__ u, T (*f)[3],
                                                bool want_dt, T* vs = nullptr, double rdt = 0.0,
                                                unsigned eflags = 0u, double* en = nullptr,
-                                               double dtsk = __builtin_inf()) {
+                                               double dtsk = __builtin_inf(), const int4* cpre = nullptr) {
     static_assert(!EN || (sizeof(T) == 8 && !VISC), "fused energies: FP64 inviscid element kernels");
     double e_def = 0.0, e_vol = 0.0;
-    const int32_t* cn = I.conn + (size_t)e * 8;
-    int4 q0 = *reinterpret_cast<const int4*>(cn);
-    int4 q1 = *reinterpret_cast<const int4*>(cn + 4);
+    const int4* cn = reinterpret_cast<const int4*>(I.conn + (size_t)e * 8);
+    const int4 q0 = cpre ? cpre[0] : cn[0], q1 = cpre ? cpre[1] : cn[1];
     const int nd[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
     const size_t N = (size_t)I.N;
     double pa, pb, c;
@@ -1251,8 +1251,8 @@ __device__ __forceinline__ double tet_kinetic(const MpsInst& I, const int* nd, d
 template <typename T, int LAW, bool VISC = false, bool EN = false, bool O32 = false>
 __device__ __forceinline__ double tet4_element(const MpsInst& I, int e, const double* __restrict__ u, T (*f)[3],
                                                bool want_dt, double rdt = 0.0, unsigned eflags = 0u,
-                                               double* en = nullptr) {
-    const int4 q = *reinterpret_cast<const int4*>(I.conn + (size_t)e * 4);
+                                               double* en = nullptr, const int4* cpre = nullptr) {
+    const int4 q = cpre ? cpre[0] : *reinterpret_cast<const int4*>(I.conn + (size_t)e * 4);
     const int nd[4] = {q.x, q.y, q.z, q.w};
     const size_t N = (size_t)I.N;
     double x[4][3], uu[4][3];
@@ -1344,12 +1344,11 @@ __device__ __forceinline__ double step_increment(const MpsInst& I, uint32_t info
     return U;
 }
 
-// Prediction + Dirichlet displacement of node n for step k (nonlinearSystem.cpp:1186-1201,
+// Prediction + Dirichlet displacement of a node (info: its Dirichlet bits) for step k (nonlinearSystem.cpp:1186-1201,
 // solverExplicit.cpp:545-575), from the half-step velocity w.  The prescribed velocity and the zero
 // acceleration of the constrained DOFs are set by the solve of the same step (node_update).
-__device__ __forceinline__ void predict_node(const MpsInst& I, int n, long long k, double dt, double* u,
+__device__ __forceinline__ void predict_node(const MpsInst& I, uint32_t info, long long k, double dt, double* u,
                                              const double* w) {
-    const uint32_t info = I.ninfo[n];
 #pragma unroll
     for (int i = 0; i < 3; i++) u[i] += step_increment(I, info, i, k, dt, w[i]);
 }
@@ -1499,49 +1498,34 @@ __device__ __forceinline__ void load_partial(const MpsInst& I, int g, double* c)
     }
 }
 
-// Internal force of node n: the sum of its patch partials in ascending patch order, in FP64 (the precision
-// form's FP32 partials widened first).
-__device__ __forceinline__ void node_partial_sum(const MpsInst& I, int n, double* f) {
-    int q = I.nrow[n];
-    const int q1 = I.nrow[n + 1];
-    double f0 = 0.0, f1 = 0.0, f2 = 0.0;
-    if (I.precision == 1) {  // FP32 partials of the precision form, summed in FP64
-        const float* __restrict__ part = reinterpret_cast<const float*>(I.part);
-        for (; q + 2 <= q1; q += 2) {
-            const float* c0 = part + 3 * (size_t)I.ncol[q];
-            const float* c1 = part + 3 * (size_t)I.ncol[q + 1];
-            const double a0 = c0[0], b0 = c0[1], d0 = c0[2];
-            const double a1 = c1[0], b1 = c1[1], d1 = c1[2];
-            f0 += a0; f1 += b0; f2 += d0;
-            f0 += a1; f1 += b1; f2 += d1;
-        }
-        if (q < q1) {
-            const float* c = part + 3 * (size_t)I.ncol[q];
-            f0 += (double)c[0];
-            f1 += (double)c[1];
-            f2 += (double)c[2];
-        }
-    } else {
-        const double* __restrict__ part = I.part;
-        // 2 entries per iteration: both loads issue before the (ordered) additions
-        for (; q + 2 <= q1; q += 2) {
-            const double* c0 = part + 3 * (size_t)I.ncol[q];
-            const double* c1 = part + 3 * (size_t)I.ncol[q + 1];
-            const double a0 = c0[0], b0 = c0[1], d0 = c0[2];
-            const double a1 = c1[0], b1 = c1[1], d1 = c1[2];
-            f0 += a0; f1 += b0; f2 += d0;
-            f0 += a1; f1 += b1; f2 += d1;
-        }
-        if (q < q1) {
-            const double* c = part + 3 * (size_t)I.ncol[q];
-            f0 += c[0];
-            f1 += c[1];
-            f2 += c[2];
-        }
+// Internal force of a node: the sum of its patch partials (entries q .. q1-1 of ncol) in ascending patch order, in FP64
+// (the precision form's FP32 partials widened first).  g0, g1: its first two entries, loaded ahead (node_first_partials);
+// two partials are in flight at a time, with the next two entries behind them.
+__device__ __forceinline__ void node_first_partials(const MpsInst& I, int q, int q1, int* g0, int* g1) {
+    *g0 = q < q1 ? I.ncol[q] : 0;
+    *g1 = q + 1 < q1 ? I.ncol[q + 1] : 0;
+}
+__device__ __forceinline__ void node_partial_sum(const MpsInst& I, int q, int q1, int g0, int g1, double* f) {
+    f[0] = f[1] = f[2] = 0.0;
+    while (q < q1) {
+        double c0[3], c1[3];
+        load_partial(I, g0, c0);
+        const bool two = q + 1 < q1;
+        if (two) load_partial(I, g1, c1);
+        q += 2;
+        node_first_partials(I, q, q1, &g0, &g1);
+#pragma unroll
+        for (int d = 0; d < 3; d++) f[d] += c0[d];
+        if (two)
+#pragma unroll
+            for (int d = 0; d < 3; d++) f[d] += c1[d];
     }
-    f[0] = f0;
-    f[1] = f1;
-    f[2] = f2;
+}
+__device__ __forceinline__ void node_partial_sum(const MpsInst& I, int n, double* f) {
+    const int q = I.nrow[n], q1 = I.nrow[n + 1];
+    int g0, g1;
+    node_first_partials(I, q, q1, &g0, &g1);
+    node_partial_sum(I, q, q1, g0, g1, f);
 }
 
 // rhs = -fint + fext (nonlinearSystem.cpp:1096-1107).
@@ -1679,13 +1663,25 @@ __device__ __forceinline__ unsigned long long* dt_slot(const MpsInst& I, int par
 __device__ __forceinline__ unsigned int* dt_count(const MpsInst& I, int s) {
     return reinterpret_cast<unsigned int*>(I.dtred + MPS_DT_WORDS + (size_t)s * MPS_DT_STRIDE);
 }
-// Min over the slots of one parity, returned in every lane; all 64 lanes of the wave must call it.
-__device__ __forceinline__ unsigned long long dt_read_min(const MpsInst& I, int parity) {
-    unsigned long long v = *dt_slot(I, parity, threadIdx.x & (MPS_DT_SLOTS - 1));
+// Min over the slots of one parity, returned in every lane; all 64 lanes of the wave must call it.  (dt_min_of: from the
+// lane's slot value.)
+__device__ __forceinline__ unsigned long long dt_min_of(unsigned long long v) {
 #pragma unroll
     for (int off = MPS_DT_SLOTS / 2; off > 0; off >>= 1)
         v = umin64(v, (unsigned long long)__shfl_xor((long long)v, off, 64));
     return v;
+}
+__device__ __forceinline__ unsigned long long dt_read_min(const MpsInst& I, int parity) {
+    return dt_min_of(*dt_slot(I, parity, threadIdx.x & (MPS_DT_SLOTS - 1)));
+}
+// Scalars of step k: both records are read, so that their address does not wait for k.
+__device__ __forceinline__ MpsStepSlot step_slot(const MpsStepSlot& s0, const MpsStepSlot& s1, long long k) {
+    const bool odd = k & 1;
+    MpsStepSlot s;
+    s.time = odd ? s1.time : s0.time;
+    s.dt = odd ? s1.dt : s0.dt;
+    s.go = odd ? s1.go : s0.go;
+    return s;
 }
 // dt_read_min for a reader in the kernel whose workgroups are still adding to the slots (device-scope loads).
 __device__ __forceinline__ unsigned long long dt_read_min_now(const MpsInst& I, int parity) {

@@ -62,6 +62,20 @@ struct PatchList {
     }
 };
 
+// What a work-item of a patch loads before the step control has arrived: its lists and its element's connectivity.
+template <int NEN>
+struct PatchPre {
+    PatchList<NEN> list;
+    int4 conn[NEN / 4];
+    __device__ __forceinline__ void load(const MpsInst& I, int p) {
+        const int e0 = p * MPS_PATCH, ne = min(MPS_PATCH, I.Ne - e0);
+        const int4* cn = reinterpret_cast<const int4*>(I.conn + (size_t)(e0 + min((int)threadIdx.x, ne - 1)) * NEN);
+#pragma unroll
+        for (int r = 0; r < NEN / 4; r++) conn[r] = cn[r];
+        list.load(I, p, e0, ne * NEN, I.poff[p + 1] - I.poff[p]);
+    }
+};
+
 // Second half of a patch: after the barrier that follows the LDS force writes, the block sums, per
 // distinct node of the patch, its contributions in ascending (element, slot) order in FP64 and writes
 // one partial force per node.  With PRE (one work-item per element, BS = MPS_PATCH) the contribution
@@ -131,19 +145,18 @@ __device__ __forceinline__ unsigned long long patch_forces(const MpsInst& I, int
                                                            uint16_t* __restrict__ spc, uint16_t* __restrict__ spr,
                                                            double rdt = 0.0, unsigned eflags = 0u,
                                                            double* env = nullptr, double* swj = nullptr,
-                                                           double dtsk = __builtin_inf()) {
+                                                           double dtsk = __builtin_inf(), PatchPre<NEN>* pre = nullptr) {
     const int e0 = p * MPS_PATCH;
     const int ne = min(MPS_PATCH, I.Ne - e0);
-    PatchList<NEN> pl;
-    if constexpr (PRE) pl.load(I, p, e0, ne * NEN, I.poff[p + 1] - I.poff[p]);
     unsigned long long dmin = INF_BITS;
     for (int i = threadIdx.x; i < ne; i += BS) {
         T f[NEN][3];
         double en[3] = {0.0, 0.0, 0.0};
         const double dte =
-            (NEN == 8) ? hex8_element<T, LAW, VISC, EN, O32>(I, e0 + i, I.u, (T(*)[3])f, want_dt,
-                                                              EN ? (T*)(swj + i) : sf + i, rdt, eflags, en, dtsk)
-                       : tet4_element<T, LAW, VISC, EN, O32>(I, e0 + i, I.u, (T(*)[3])f, want_dt, rdt, eflags, en);
+            (NEN == 8) ? hex8_element<T, LAW, VISC, EN, O32>(I, e0 + i, I.u, (T(*)[3])f, want_dt, EN ? (T*)(swj + i) : sf + i,
+                                                              rdt, eflags, en, dtsk, PRE ? pre->conn : nullptr)
+                       : tet4_element<T, LAW, VISC, EN, O32>(I, e0 + i, I.u, (T(*)[3])f, want_dt, rdt, eflags, en,
+                                                             PRE ? pre->conn : nullptr);
         if constexpr (EN) {
 #pragma unroll
             for (int j = 0; j < 3; j++) env[j] += en[j];
@@ -154,9 +167,9 @@ __device__ __forceinline__ unsigned long long patch_forces(const MpsInst& I, int
             for (int d = 0; d < 3; d++) sf[(a * 3 + d) * MPS_PATCH + i] = f[a][d];
         dmin = umin64(dmin, d2bits(dte));
     }
-    if constexpr (PRE) pl.store(spc, spr, ne * NEN);
+    if constexpr (PRE) pre->list.store(spc, spr, ne * NEN);
     __syncthreads();
-    patch_sums<T, NEN, BS, PRE>(I, p, sf, spc, spr + (PRE ? pl.off : 0));
+    patch_sums<T, NEN, BS, PRE>(I, p, sf, spc, spr + (PRE ? pre->list.off : 0));
     return dmin;
 }
 
@@ -252,18 +265,25 @@ __global__ __launch_bounds__(MPS_PATCH) __attribute__((amdgpu_waves_per_eu(VISC 
     constexpr bool SKIP = sizeof(T) == 8 && NEN == 8 && !VISC;
     long long k = 0;
     double rdt = 0.0, dtsk = __builtin_inf();
+    const int p = xcd_tile(blockIdx.x, gridDim.x);
+    PatchPre<NEN> pre;
     if (mode == 0) {
+        // the control block, the lists and the connectivity travel together: one after the other they were 2,400 of
+        // 27,800 cycles of a workgroup that has its CU for itself
         k = I.ctl->A;
+        const MpsStepSlot s0 = I.ctl->slot[0], s1 = I.ctl->slot[1];
+        if (SKIP) dtsk = I.ctl->dt_skip;
+        pre.load(I, p);
         if (blockIdx.x == 0 && threadIdx.x == 0) I.ctl->B = k;
-        const MpsStepSlot s = I.ctl->slot[k & 1];
+        const MpsStepSlot s = step_slot(s0, s1, k);
         if (!s.go) return;
         if (VISC) rdt = (s.dt == 0.0) ? 0.0 : 1 / s.dt;
-        if (SKIP) dtsk = I.ctl->dt_skip;
+    } else {
+        pre.load(I, p);
     }
-    const int p = xcd_tile(blockIdx.x, gridDim.x);
     double env[3] = {0.0, 0.0, 0.0};
     unsigned long long m = patch_forces<T, NEN, LAW, MPS_PATCH, VISC, true, EN, O32>(I, p, mode == 0, sf, spc, spr,
-                                                                                    rdt, eflags, env, swj, dtsk);
+                                                                                    rdt, eflags, env, swj, dtsk, &pre);
     if (mode == 0) {
         m = block_min_u64(m, sh);
         if (threadIdx.x == 0) atomicMin(dt_slot(I, dt_parity(k + 1), blockIdx.x & (MPS_DT_SLOTS - 1)), m);
@@ -316,12 +336,12 @@ __global__ __launch_bounds__(MPS_PATCH) __attribute__((amdgpu_waves_per_eu(sizeo
     constexpr bool SKIP = sizeof(T) == 8;  // stable-dt skip (dt_certify)
     long long k = 0;
     double dtsk = __builtin_inf();
-    if (mode == 0) {
+    int go = 1;
+    if (mode == 0) {  // used once the nodes are on their way (k_elem)
         k = I.ctl->A;
-        if (blockIdx.x == 0 && threadIdx.x == 0) I.ctl->B = k;
-        const MpsStepSlot s = I.ctl->slot[k & 1];
-        if (!s.go) return;
+        const MpsStepSlot s0 = I.ctl->slot[0], s1 = I.ctl->slot[1];
         if (SKIP) dtsk = I.ctl->dt_skip;
+        go = step_slot(s0, s1, k).go;
     }
     const int p = xcd_tile(blockIdx.x, gridDim.x);
     const int e0 = p * MPS_PATCH;
@@ -346,6 +366,8 @@ __global__ __launch_bounds__(MPS_PATCH) __attribute__((amdgpu_waves_per_eu(sizeo
         s[2] = make_double2(u1, u2);
     }
     pl.store(spc, nullptr, ne * 4);  // the list arrives with the nodes; stored now, it holds no registers below
+    if (mode == 0 && blockIdx.x == 0 && threadIdx.x == 0) I.ctl->B = k;
+    if (!go) return;
     __syncthreads();
     unsigned long long dmin = INF_BITS;
     double env[3] = {0.0, 0.0, 0.0};
@@ -445,10 +467,13 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(2))) void k_
         const MpsWork W = work[w];
         const MpsInst& I = insts[W.inst];
         const long long k = I.ctl->A;
+        const MpsStepSlot s0 = I.ctl->slot[0], s1 = I.ctl->slot[1];
+        PatchPre<NEN> pre;
+        if constexpr (PRE) pre.load(I, W.begin / MPS_PATCH);
         if (W.first && threadIdx.x == 0) I.ctl->B = k;
-        if (I.ctl->slot[k & 1].go) {
-            unsigned long long m =
-                patch_forces<T, NEN, LAW, BS, false, PRE, false, true>(I, W.begin / MPS_PATCH, true, sf, spc, spr);
+        if (step_slot(s0, s1, k).go) {
+            unsigned long long m = patch_forces<T, NEN, LAW, BS, false, PRE, false, true>(
+                I, W.begin / MPS_PATCH, true, sf, spc, spr, 0.0, 0u, nullptr, nullptr, __builtin_inf(), &pre);
             m = block_min_u64(m, sh);
             if (threadIdx.x == 0) atomicMin(dt_slot(I, dt_parity(k + 1), w & (MPS_DT_SLOTS - 1)), m);
         }
@@ -491,13 +516,37 @@ template <bool EN = false>
 __device__ __forceinline__ bool node_item(const MpsInst& I, int n, bool first, int fuse, unsigned nflags,
                                           double* red = nullptr) {
     MpsCtl* ctl = I.ctl;
+    const size_t N = (size_t)I.N;
+    // everything whose address is known is loaded before any of it is used: read when needed, the control block, the
+    // slots, the state and the node's lists were five dependent loads, nearly all of the 6 us of a mesh that fits the caches
+    const int i0 = n < 0 ? 0 : n;
     const long long k = ctl->B;
-    const MpsStepSlot s = ctl->slot[k & 1];
+    const MpsStepSlot s0 = ctl->slot[0], s1 = ctl->slot[1];
+    unsigned long long m0 = 0ull, m1 = 0ull;
+    if (fuse) {
+        m0 = *dt_slot(I, 0, threadIdx.x & (MPS_DT_SLOTS - 1));
+        m1 = *dt_slot(I, 1, threadIdx.x & (MPS_DT_SLOTS - 1));
+    }
+    const int q0 = I.nrow[i0], q1 = I.nrow[i0 + 1];
+    double u[3], w[3], v[3], a[3];
+    {
+        const double* src = (nflags & (MPS_N_IN_VA | MPS_N_IN_WA)) == MPS_N_IN_WA ? I.a : I.v;
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            u[i] = I.u[i * N + i0];
+            w[i] = src[i * N + i0];
+        }
+    }
+    const uint32_t info = I.ninfo[i0];
+    const double m = I.mass[i0];
+    int g0, g1;
+    node_first_partials(I, q0, q1, &g0, &g1);
+    const MpsStepSlot s = step_slot(s0, s1, k);
     if (!s.go) return false;
     MpsStepSlot nx;
     nx.go = 0;
     int st = MPSD_RUNNING;
-    const unsigned long long mb = fuse ? dt_read_min(I, dt_parity(k + 1)) : 0ull;
+    const unsigned long long mb = fuse ? dt_min_of(dt_parity(k + 1) ? m1 : m0) : 0ull;
     if (fuse) st = begin_scalars(I, k + 1, s, mb, &nx);
     if (first) {
         ctl->A = k + 1;
@@ -510,31 +559,35 @@ __device__ __forceinline__ bool node_item(const MpsInst& I, int n, bool first, i
         }
     }
     if (n < 0) return true;
-    const size_t N = (size_t)I.N;
-    double u[3], w[3], v[3], a[3];
+    if (nflags & MPS_N_IN_VA) {
 #pragma unroll
-    for (int i = 0; i < 3; i++) u[i] = I.u[i * N + n];
-    load_half_velocity(I, n, nflags, s.dt, w);
+        for (int i = 0; i < 3; i++) w[i] = half_velocity(s.dt, w[i], I.a[i * N + n]);
+    }
+    double fi[3];
+    if (EN || (info & 7u) != 7u) node_partial_sum(I, q0, q1, g0, g1, fi);
     if (EN) {
         // the forces first (also of a fully constrained node, for the work of the supports), then the step's
         // increments from w: nothing extra is held through the partial sums
-        const uint32_t info = I.ninfo[n];
         double rhs[3];
         {
-            double fi[3], fe[3], incr[3];
-            node_partial_sum(I, n, fi);
+            double fe[3], incr[3];
             node_fext(I, n, info, fe);
 #pragma unroll
             for (int i = 0; i < 3; i++) incr[i] = step_increment(I, info, i, k, s.dt, w[i]);
             node_energy_forces(I, n, info, k, u, incr, fi, fe, red);
             node_rhs(fi, fe, rhs);
         }
-        const double m = I.mass[n];
         double wkin = -0.0;
         node_update(I, info, k, s.dt, m, rhs, w, v, a, &wkin);
         node_energy_motion(m, k, wkin, v, red);
     } else {
-        solve_node(I, n, k, s.dt, w, v, a);
+        double rhs[3] = {0.0, 0.0, 0.0};
+        if ((info & 7u) != 7u) {
+            double fe[3];
+            node_fext(I, n, info, fe);
+            node_rhs(fi, fe, rhs);
+        }
+        node_update(I, info, k, s.dt, m, rhs, w, v, a);
     }
     if (n == I.dof1_node) {
         double x = u[I.dof1_dir];
@@ -551,7 +604,7 @@ __device__ __forceinline__ bool node_item(const MpsInst& I, int n, bool first, i
         }
 #pragma unroll
         for (int i = 0; i < 3; i++) w[i] = half_velocity(nx.dt, v[i], a[i]);
-        predict_node(I, n, k + 1, nx.dt, u, w);
+        predict_node(I, info, k + 1, nx.dt, u, w);
     }
 #pragma unroll
     for (int i = 0; i < 3; i++) I.u[i * N + n] = u[i];
@@ -711,7 +764,7 @@ __device__ __forceinline__ void begin_item(const MpsInst& I, int n, bool first) 
 #pragma unroll
         for (int i = 0; i < 3; i++) I.uprev[i * N + n] = u[i];
     }
-    predict_node(I, n, k, nx.dt, u, w);
+    predict_node(I, I.ninfo[n], k, nx.dt, u, w);
 #pragma unroll
     for (int i = 0; i < 3; i++) I.u[i * N + n] = u[i];
 }
