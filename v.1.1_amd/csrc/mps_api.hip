@@ -422,13 +422,15 @@ int prepare(const mps_mesh* mesh, const mps_material* mat, const mps_bcs* bcs, c
     return MPS_OK;
 }
 
-// Meshes up to this many elements step in the spread form: hex8 FP64 29,800 elements 16.4 us per step against 19.9, 64,000
-// 29.4 against 21.0; tet4 FP32 form 48,000 10.2 against 11.3, 93,800 16.7 against 12.0.  With energies every step the patch
-// form gives up more (its energy kernels and sums): hex8 35,800 28.6 against 31.4, 50,700 38.1 against 31.4; tet4 55,600 14.3
-// against 22.1.  Loads and viscosity come after creation: at 31,700 elements with both 24.5 against 29.1.  MPS_SPREAD=0 in the environment keeps the patch form,
-// MPS_SPREAD=1 takes the spread form at any size; so do the switches of the patch kernels (MPS_GATHER32, MPS_DT_SKIP,
-// MPS_TET_STAGING), which have no meaning in the spread form.  Both forms give the same bits.
-static const int64_t kSpreadMaxHex = 32768, kSpreadMaxTet = 60000, kSpreadMaxHexEnergy = 40960, kSpreadMaxTetEnergy = 80000;
+// Meshes up to this many elements step in the spread form.  us per step, spread / patch form: hex8 FP64 29,800 elements
+// 16.8 / 19.2, 35,900 18.9 / 20.4, 46,700 23.2 / 19.4, FP32 form 35,900 16.0 / 17.4, 46,700 18.6 / 16.7; tet4 FP64 63,900 11.6 /
+// 12.3, 93,800 16.8 / 13.6, FP32 form 35,000 9.8 / 9.9, 48,000 10.3 / 10.0.  With energies every step the patch form gives up
+// more (its energy kernels and sums): hex8 35,800 24.5 / 30.9, 50,700 32.2 / 31.1; tet4 55,600 13.4 / 21.6.  Loads and viscosity
+// come after creation: at 31,700 elements with both 22.8 / 29.2, at 46,700 30.3 / 27.3.  MPS_SPREAD=0 in the environment
+// keeps the patch form, MPS_SPREAD=1 takes the spread form at any size; so do the switches of the patch kernels
+// (MPS_GATHER32, MPS_DT_SKIP, MPS_TET_STAGING), which have no meaning in the spread form.  Both forms give the same bits.
+static const int64_t kSpreadMaxHex = 36864, kSpreadMaxTet = 64000, kSpreadMaxTet32 = 40000;
+static const int64_t kSpreadMaxHexEnergy = 49152, kSpreadMaxTetEnergy = 80000;
 
 void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const int64_t N = hp.N, Ne = hp.Ne, nen = hp.nen;
@@ -436,8 +438,10 @@ void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const char* env = getenv("MPS_SPREAD");
     const bool force = env && strcmp(env, "1") == 0;
     if (env && !force && strcmp(env, "0") == 0) return;
-    const bool en = hp.cfg.energy_every > 0 && hp.cfg.precision == MPS_PREC_FP64;
-    const int64_t most = nen == 8 ? (en ? kSpreadMaxHexEnergy : kSpreadMaxHex) : (en ? kSpreadMaxTetEnergy : kSpreadMaxTet);
+    const bool fp64 = hp.cfg.precision == MPS_PREC_FP64, en = hp.cfg.energy_every > 0 && fp64;
+    const int64_t most = nen == 8 ? (en ? kSpreadMaxHexEnergy : kSpreadMaxHex)
+                                  : (en ? kSpreadMaxTetEnergy : fp64 ? kSpreadMaxTet : kSpreadMaxTet32);
+    if (hp.bcval.size() / 3 > (1u << 23)) return;  // Dirichlet records of an entry
     if (!force && (Ne > most || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") ||
                    getenv("MPS_TET_STAGING")))
         return;
@@ -492,8 +496,9 @@ void build_spread(const HostPrep& hp, SpreadTables* sp) {
             const int64_t g = b * stride + (i - off[(size_t)b]);
             const bool own = sp->own[(size_t)n] < 0;
             if (own) sp->own[(size_t)n] = (int32_t)g;
-            sp->node[(size_t)g] = make_int4(own ? (int32_t)((uint32_t)n | 0x80000000u) : n, first[(size_t)n],
-                                            first[(size_t)n + 1] - first[(size_t)n], (int32_t)ends[(size_t)n]);
+            const uint32_t z = (uint32_t)(first[(size_t)n + 1] - first[(size_t)n]) | hp.ninfo[(size_t)n] << 6;
+            sp->node[(size_t)g] = make_int4(own ? (int32_t)((uint32_t)n | 0x80000000u) : n, first[(size_t)n], (int32_t)z,
+                                            (int32_t)ends[(size_t)n]);
         }
     sp->nb = (int32_t)nb;
     sp->stride = (int32_t)stride;

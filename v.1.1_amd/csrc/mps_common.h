@@ -194,8 +194,9 @@ struct MpsInst {
     // spread form (mps_spread.hip; sp_nb = 0: not set up): sp_nb workgroups of consecutive elements, each with up to
     // sp_stride distinct nodes
     int32_t sp_nb, sp_stride;
-    const int4* sp_node;      // [sp_nb*sp_stride] {node (bit 31: owned by this workgroup), first position, count, end bits
-                              // of the patches among its positions}; x = -1: padding
+    const int4* sp_node;      // [sp_nb*sp_stride] {node (bit 31: owned by this workgroup), first position, count (6 bits),
+                              // Dirichlet bits (3) and record (23), end bits of the patches among its positions}; x = -1:
+                              // padding
     const uint16_t* sp_lx;    // [nen*Ne] index of each element slot's node among its workgroup's nodes
     const int32_t* sp_pos;    // [nen*Ne] position of each element slot in node order
     const int32_t* sp_own;    // [N] entry of sp_node that owns the node

@@ -1273,29 +1273,20 @@ __device__ __forceinline__ double tet4_element(const MpsInst& I, int e, const do
 // Step control (begin of step k): lagged time update, termination, stable dt.
 // solverExplicit.cpp:217-273.
 // ---------------------------------------------------------------------------
+// Without branches: the arguments it reads are then requested together.
 __device__ __forceinline__ int begin_scalars(const MpsInst& I, long long k, const MpsStepSlot& prev,
                                              unsigned long long dtmin_bits, MpsStepSlot* out) {
 #pragma clang fp contract(off)
-    out->go = 0;
-    out->time = prev.time;
-    out->dt = prev.dt;
-    if (!prev.go) return MPSD_RUNNING;
-    double time;
-    if (I.time_mode == MPS_TIME_FIXED) {
-        if (k > I.n_steps) return MPSD_DONE;
-        time = prev.time + prev.dt;
-    } else {
-        if (!(prev.time < I.tf - 1E-12)) return MPSD_DONE;
-        if (prev.time + prev.dt > I.tf) time = I.tf;
-        else time = prev.time + prev.dt;
-    }
-    double dt = bits2d(dtmin_bits);
-    dt = dt * I.scale;
-    if (dt < 1E-20) return MPSD_ERR_DT;
-    out->time = time;
-    out->dt = dt;
-    out->go = 1;
-    return MPSD_RUNNING;
+    const bool fixed = I.time_mode == MPS_TIME_FIXED;
+    const double next = prev.time + prev.dt, tf = I.tf;
+    const bool done = fixed ? k > I.n_steps : !(prev.time < tf - 1E-12);
+    const double time = !fixed && next > tf ? tf : next;
+    const double dt = bits2d(dtmin_bits) * I.scale;
+    const bool small = dt < 1E-20, go = prev.go && !done && !small;
+    out->go = go;
+    out->time = go ? time : prev.time;
+    out->dt = go ? dt : prev.dt;
+    return !prev.go ? MPSD_RUNNING : done ? MPSD_DONE : small ? MPSD_ERR_DT : MPSD_RUNNING;
 }
 
 // Stable-dt skip threshold for the element kernel of step k, from the min dt of step k-1 (bit pattern mb, before
@@ -1333,15 +1324,22 @@ __device__ __forceinline__ void bc_motion(const MpsInst& I, double val, long lon
 // and a).  Constrained DOFs hold a = 0, so there w = v.
 __device__ __forceinline__ double half_velocity(double dt, double v, double a) { return __builtin_fma(0.5 * dt, a, v); }
 
-// Increment of DOF i of node n at the begin of step k: the prediction dt w on active DOFs (w the half-step
-// velocity above), the prescribed U on constrained ones.
+// Increment of a DOF at the begin of step k: the prediction dt w on active DOFs (w the half-step velocity above), the
+// prescribed U on constrained ones (fixed, BC value val).
+__device__ __forceinline__ double dof_increment(const MpsInst& I, bool fixed, double val, long long k, double dt, double w) {
+#pragma clang fp contract(off)
+    if (!fixed) return dt * w;
+    double U, V;
+    bc_motion(I, val, k, dt, &U, &V);
+    return U;
+}
+// The same of DOF i of a node with Dirichlet bits and record info.
+__device__ __forceinline__ double bc_value(const MpsInst& I, uint32_t info, int i) {
+    return ((info >> i) & 1u) ? I.bcval[3 * (size_t)((info & MPS_REC_MASK) >> 3) + i] : 0.0;
+}
 __device__ __forceinline__ double step_increment(const MpsInst& I, uint32_t info, int i, long long k, double dt,
                                                  double w) {
-#pragma clang fp contract(off)
-    if (!((info >> i) & 1u)) return dt * w;
-    double U, V;
-    bc_motion(I, I.bcval[3 * (size_t)((info & MPS_REC_MASK) >> 3) + i], k, dt, &U, &V);
-    return U;
+    return dof_increment(I, (info >> i) & 1u, bc_value(I, info, i), k, dt, w);
 }
 
 // Prediction + Dirichlet displacement of a node (info: its Dirichlet bits) for step k (nonlinearSystem.cpp:1186-1201,
@@ -1368,23 +1366,20 @@ __device__ __forceinline__ void node_fext(const MpsInst& I, int n, uint32_t info
     }
 }
 
-__device__ __forceinline__ double node_fext1(const MpsInst& I, const double* __restrict__ lf, int n, uint32_t info, int i) {
-    if (info & MPS_NODE_LOADED) return lf[3 * (size_t)I.lidx[n] + i];
-    return (i == 2 && I.fgrav) ? I.fgrav[n] : 0.0;
-}
-
 // Force of scatter node a at surface Gauss point q at time t.  Pressure (BCsPressureRamp / BCsPressureInst,
 // boundaryConditions.cpp:370-496): F of the bulk element at the point (classSpatialPoint::getF,
 // classSpatialPoint.cpp:41-68: node terms first, then the identity), J = det F, n = F^-T n0, and
 // w|J_s| phi_a J P(t) n_i.  Traction (BCsTractionRamp / Inst, :218-271): w|J_s| phi_a T_i(t).  FP64, reference operation
 // order; everything it reads is loaded before it is used.
+// PRESSURE = false: the loads hold no pressure block (whose force takes the step's displacement, and most of the registers).
+template <bool PRESSURE = true>
 __device__ __forceinline__ void surface_force(const MpsInst& I, int q, int a, double t, double* out) {
 #pragma clang fp contract(off)
     const double* D = I.sgd + (size_t)q * MPS_SGP_STRIDE;
     const double* B = I.sblk + MPS_SBLK_STRIDE * (size_t)I.sgb[q];
     const double ws = D[27], ph = D[28 + a];
     const bool in = t >= B[2] && t <= B[3];
-    if (B[0] >= 4.0) {
+    if (!PRESSURE || B[0] >= 4.0) {
         for (int i = 0; i < 3; i++) {
             const double T = in ? (B[0] == 4.0 ? B[4 + i] / (B[3] - B[2]) * (t - B[2]) : B[4 + i]) : 0.;
             out[i] = ws * ph * T;
@@ -1440,12 +1435,13 @@ __device__ __forceinline__ void surface_force(const MpsInst& I, int q, int a, do
 // One load item of node n at time t: a nodal force entry (BCsNodalForces, boundaryConditions.cpp:1120-1134 with
 // classNeumann::getTracAmount, classNodes.h:101-108: F/(tf-t0) * t for t0 <= t <= tf, else 0), a surface force, or the
 // node's gravity load (BCsGravity :1146-1172, constant, summed over the Gauss points at set-up).
+template <bool PRESSURE = true>
 __device__ __forceinline__ void load_item(const MpsInst& I, int n, uint32_t code, double t, double* c) {
 #pragma clang fp contract(off)
     const uint32_t kind = code >> 30;
     const size_t idx = code & MPS_ITEM_INDEX;
     if (kind == MPS_ITEM_PRESSURE) {
-        surface_force(I, (int)(idx >> 3), (int)(idx & 7), t, c);
+        surface_force<PRESSURE>(I, (int)(idx >> 3), (int)(idx & 7), t, c);
     } else if (kind == MPS_ITEM_FORCE) {
         const bool in = t >= I.lwin[2 * idx] && t <= I.lwin[2 * idx + 1];
         for (int d = 0; d < 3; d++) c[d] = in ? I.lm[3 * idx + d] * t : 0.0;
@@ -1461,6 +1457,7 @@ __device__ __forceinline__ void load_item(const MpsInst& I, int n, uint32_t code
 // and more, whose dependent loads one work-item would walk through one after the other.  No barrier: a node's lanes are
 // half a wave.
 #define MPS_LOAD_NODES 8  // per workgroup of 256
+template <bool PRESSURE = true>
 __device__ __forceinline__ void loads_block(const MpsInst& I, int lb, double t, double* sh, double* lf) {
 #pragma clang fp contract(off)
     const int l = threadIdx.x & 31, j = lb * (int)(blockDim.x >> 5) + (int)(threadIdx.x >> 5);
@@ -1470,7 +1467,7 @@ __device__ __forceinline__ void loads_block(const MpsInst& I, int lb, double t, 
     double fe = 0.0;
     for (int q = q0; __any(q < q1); q += 32) {
         double c[3] = {0.0, 0.0, 0.0};
-        if (q + l < q1) load_item(I, n, (uint32_t)I.lcode[q + l], t, c);
+        if (q + l < q1) load_item<PRESSURE>(I, n, (uint32_t)I.lcode[q + l], t, c);
 #pragma unroll
         for (int d = 0; d < 3; d++) s[l * 3 + d] = c[d];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1540,12 +1537,12 @@ __device__ __forceinline__ void node_rhs(const double* fi, const double* fe, dou
 // the previous step (its velocity on constrained DOFs); rhs = -fint + fext of the node (read for free DOFs
 // only).  With wkin, 1/2 m (V^2 - w^2) of each constrained DOF, whose velocity the prescribed V replaces, is
 // added to *wkin.
-__device__ __forceinline__ void node_update1(const MpsInst& I, uint32_t info, int i, long long k, double dt, double m,
-                                             double rhs, double w, double* v, double* a, double* wkin = nullptr) {
+__device__ __forceinline__ void dof_update(const MpsInst& I, bool fixed, double val, long long k, double dt, double m,
+                                           double rhs, double w, double* v, double* a, double* wkin = nullptr) {
 #pragma clang fp contract(off)
-    if ((info >> i) & 1u) {
+    if (fixed) {
         double U, V;
-        bc_motion(I, I.bcval[3 * (size_t)((info & MPS_REC_MASK) >> 3) + i], k, dt, &U, &V);
+        bc_motion(I, val, k, dt, &U, &V);
         if (wkin) *wkin += 0.5 * m * (V * V - w * w);
         *v = V;
         *a = 0.;
@@ -1559,7 +1556,8 @@ __device__ __forceinline__ void node_update(const MpsInst& I, uint32_t info, lon
                                             const double* rhs, const double* w, double* v, double* a,
                                             double* wkin = nullptr) {
 #pragma unroll
-    for (int i = 0; i < 3; i++) node_update1(I, info, i, k, dt, m, rhs[i], w[i], v + i, a + i, wkin);
+    for (int i = 0; i < 3; i++)
+        dof_update(I, (info >> i) & 1u, bc_value(I, info, i), k, dt, m, rhs[i], w[i], v + i, a + i, wkin);
 }
 
 // Gather + lumped-mass solve of node n at step k (node_partial_sum, node_fext, node_update): v, a of the step

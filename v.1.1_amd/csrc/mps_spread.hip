@@ -15,15 +15,17 @@
 // work.  Every sum keeps the patch form's order -- the forces of a node are added per patch of MPS_PATCH elements and then
 // over the patches -- and an element's arithmetic is the same function by function, so both forms give the same bits.
 //
-// Measured, us per step, patch form / here.  hex8 FP64: 1,000 elements 19.0 / 5.6, 8,000 19.4 / 7.2, 15,600 19.9 / 9.9,
-// 29,800 19.9 / 16.4, 64,000 21.0 / 29.4; FP32 form: 1,000 15.9 / 5.6, 15,600 16.7 / 9.1, 29,800 16.9 / 14.3; tet4 FP64:
-// 750 13.6 / 6.8, 10,400 12.9 / 6.8, 48,000 13.8 / 10.0, 93,800 14.6 / 18.0; FP32 form: 10,400 10.5 / 6.8, 48,000 11.3 /
-// 10.2, 93,800 12.0 / 16.7.  Every node is updated by all the workgroups that hold it (4.5 per 8 hex8 elements where the
-// patch form has 1.03 per element), so past the size where the lanes are no longer idle the patch form is the better one.
-// With energies every step and loads (hex8 FP64): 512 elements 29.8 / 7.7, 12,200 30.7 / 13.4, 35,800 31.4 / 28.6; tet4 750
-// 22.1 / 7.7, 55,600 22.1 / 14.3; with viscosity and loads (FP64 Belytschko): 512 24.0 / 7.0, 12,200 25.3 / 12.5, 31,700 29.1 /
-// 24.5.  The patch form takes three launches for these steps; here the external forces and the energy sums are extra
-// workgroups of the step's launch.
+// Measured, us per step, patch form / here.  hex8 FP64: 1,000 elements 17.7 / 5.6, 8,000 18.4 / 7.4, 15,600 19.1 / 10.2,
+// 29,800 19.2 / 16.8, 46,700 19.4 / 23.2; FP32 form: 1,000 14.6 / 5.6, 15,600 16.2 / 9.3, 29,800 16.5 / 14.2; tet4 FP64: 750
+// 12.3 / 6.6, 10,400 12.2 / 6.7, 48,000 12.2 / 10.2, 93,800 13.6 / 16.8; FP32 form: 10,400 9.7 / 6.4, 48,000 10.0 / 10.3.
+// Every node is updated by all the workgroups that hold it (4.5 per 8 hex8 elements where the patch form has 1.03 per
+// element), so past the size where the lanes are no longer idle the patch form is the better one.
+// With energies every step and loads (hex8 FP64): 512 elements 29.3 / 7.3, 12,200 30.2 / 12.1, 35,800 30.9 / 24.5; tet4 750
+// 22.0 / 7.2, 55,600 21.6 / 13.4; with viscosity and loads (FP64 Belytschko): 512 23.4 / 6.6, 12,200 25.2 / 11.6, 31,700 29.2 /
+// 22.8.  The patch form takes three launches for these steps; here the external forces and the energy sums are extra
+// workgroups of the step's launch, on a path of their own from the first instruction, and without the pressure loads'
+// code: sharing the element workgroups' prologue, with that code, cost 48 registers, two of five waves per SIMD, and 18.7
+// instead of 16.8 us at 29,800 elements.
 // Tried: one wave per workgroup, which takes the dt and the forces in turn (half the waves): 2 us more at 1,000 elements and
 // the same above 30,000, where the issue of 1,380 vector instructions per 8 elements is the bound, not the waves in flight.
 // Tried: 16 and 32 hex8 elements per workgroup: fewer shared nodes, but 0.4 to 1.8 us more up to 2,000 elements and
@@ -61,41 +63,58 @@ __device__ __forceinline__ T* spread_forces(const MpsInst& I, int ci) {
     return reinterpret_cast<T*>(I.sp_f) + (ci & 1 ? 3 * (size_t)I.nen * I.Ne : 0);
 }
 
-// What the update of one node in one direction reads, loaded before any of it is used.  At index 0 of a sequence w and m
-// are v and a, and the forces are not used.
+// Entry E of sp_node: count, Dirichlet bits and record of the node.
+__device__ __forceinline__ int entry_count(const int4& E) { return E.z & 63; }
+__device__ __forceinline__ bool entry_fixed(const int4& E, int d) { return ((uint32_t)E.z >> (6 + d)) & 1u; }
+__device__ __forceinline__ uint32_t entry_record(const int4& E) { return (uint32_t)E.z >> 9; }
+
+// What the update of one node in one direction reads, loaded before any of it is used (the Dirichlet value and the load
+// index among it: read when needed they were a third dependent load, in the workgroups of every supported face).  At index
+// 0 of a sequence w and m are v and a, and the forces are not used.
 template <typename T, int FLIGHT>
 struct NodeLoads {
-    double X, u, w, m;
-    uint32_t info;
+    double X, u, w, m, bc, fg;
+    int li;       // index of the node's external force, -1: none
     T c[FLIGHT];  // the first element forces
     __device__ __forceinline__ void load(const MpsInst& I, const int4& E, int d, bool first, const double* __restrict__ ur,
                                          const double* __restrict__ wr, const T* __restrict__ f) {
-        const int n = E.x & 0x7FFFFFFF;
+        const int n = E.x & 0x7FFFFFFF, last = entry_count(E) - 1;
         const size_t i = (size_t)d * I.N + n;
+        li = -1;
+        fg = 0.0;
+        if (I.n_lnode > 0) li = I.lidx[n];  // uniform branches; the others load in every lane, used or not
+        if (I.fgrav) {
+            const double g = I.fgrav[n];
+            fg = d == 2 ? g : 0.0;
+        }
+        bc = I.bcval[3 * (size_t)entry_record(E) + d];
         X = I.X[i];
         u = ur[i];
         w = wr[i];  // (at index 0 the buffer is v)
         m = *(first ? I.a + i : I.mass + n);
-        info = I.ninfo[n];
         const T* p = f + 3 * (size_t)E.y + d;
 #pragma unroll
-        for (int q = 0; q < FLIGHT; q++) c[q] = p[3 * min(q, E.z - 1)];
+        for (int q = 0; q < FLIGHT; q++) c[q] = p[3 * min(q, last)];
+    }
+    __device__ __forceinline__ double fext(const double* __restrict__ lf, int d) const {
+        return li >= 0 ? lf[3 * (size_t)li + d] : fg;
     }
     // Internal force of the node in direction d: its entries added per patch (end bits E.w), then over the patches --
     // the order and the roundings of patch_sums and node_partial_sum.  Without branches: entries past the end add 0.0 to
     // sums that are never -0.0.
     __device__ __forceinline__ double force(const int4& E, const T* __restrict__ f, int d) {
 #pragma clang fp contract(off)
+        const int count = entry_count(E);
         double fi = 0.0, s = 0.0;
-        for (int q0 = 0; q0 < E.z; q0 += FLIGHT) {
+        for (int q0 = 0; q0 < count; q0 += FLIGHT) {
             if (q0 > 0) {
                 const T* p = f + 3 * (size_t)E.y + d;
 #pragma unroll
-                for (int q = 0; q < FLIGHT; q++) c[q] = p[3 * min(q0 + q, E.z - 1)];
+                for (int q = 0; q < FLIGHT; q++) c[q] = p[3 * min(q0 + q, count - 1)];
             }
 #pragma unroll
             for (int q = 0; q < FLIGHT; q++) {
-                s += q0 + q < E.z ? (double)c[q] : 0.0;
+                s += q0 + q < count ? (double)c[q] : 0.0;
                 const bool end = ((uint32_t)E.w >> (q0 + q)) & 1u;  // q0 + q <= 31
                 fi += end ? (sizeof(T) == 4 ? (double)(float)s : s) : 0.0;
                 s = end ? 0.0 : s;
@@ -531,19 +550,19 @@ __device__ __forceinline__ void spread_history(const MpsInst& I, long long A, in
     if ((k - 1) % I.energy_every == 0) *hist_at(I, MPS_H_EKIN, k - 1) = el[2];
     node_history(I, k - 1, nd);
 }
-// Energy terms of DOF (n, d) at step k, by the owner of the node (node_energy_forces and node_energy_motion for one
+// Energy terms of DOF d of a node (entry E, load index li) at step k, by the node's owner (node_energy_forces and node_energy_motion for one
 // direction): u the step's displacement, incr its increment, fi and fe the forces, m, v and wkin as the update leaves them.
-__device__ __forceinline__ void dof_energy(const MpsInst& I, int n, uint32_t info, int d, long long k, double u, double incr,
+__device__ __forceinline__ void dof_energy(const MpsInst& I, const int4& E, int li, int d, long long k, double u, double incr,
                                            double fi, double fe, double m, double v, double wkin, double* red) {
     double fp = fe;
-    if (info & MPS_NODE_LOADED) {
-        double* lp = I.lfprev + 3 * (size_t)I.lidx[n] + d;
+    if (li >= 0) {
+        double* lp = I.lfprev + 3 * (size_t)li + d;
         fp = *lp;
         *lp = fe;
     }
     double wr = wkin;
-    if ((info >> d) & 1u) {
-        double* rp = I.rprev + 3 * (size_t)((info & MPS_REC_MASK) >> 3) + d;
+    if (entry_fixed(E, d)) {
+        double* rp = I.rprev + 3 * (size_t)entry_record(E) + d;
         const double r = fi - fe;
         wr += 0.5 * (*rp + r) * incr;
         *rp = r;
@@ -578,7 +597,7 @@ __device__ __forceinline__ void spread_side(const MpsInst& I, int ci, int x, lon
         }
         x -= P + G + 1;
     }
-    loads_block(I, x, time, sh, spread_lf(I, ci));
+    loads_block<false>(I, x, time, sh, spread_lf(I, ci));
 }
 template <int NEN, int MODE>
 unsigned side_blocks(const MpsInst& I) {
@@ -588,21 +607,47 @@ unsigned side_blocks(const MpsInst& I) {
 
 }  // namespace
 
+// Step control of the kernel with index ci, the same in every workgroup: requested by load (the lane's dt slot with it),
+// evaluated by begin.
+struct StepControl {
+    long long A, k;
+    MpsStepSlot prev, nx;
+    unsigned long long m16;
+    __device__ __forceinline__ void load(const MpsInst& I, int ci) {
+        const MpsCtl* ctl = I.ctl;
+        A = ctl->A;
+        k = A + ci;
+        const MpsStepSlot* pp = ci == 0 ? ctl->slot + ((A - 1) & 1) : ctl->sslot + ((ci - 1) & 1);
+        prev.time = pp->time;
+        prev.dt = pp->dt;
+        prev.go = pp->go;
+        const int row = threadIdx.x & (MPS_DT_SLOTS - 1);
+        m16 = *(ci == 0 ? dt_slot(I, dt_parity(A), row) : dt_spread(I, ci % 3, row));
+    }
+    __device__ __forceinline__ int begin(const MpsInst& I) { return begin_scalars(I, k, prev, row_min(m16), &nx); }
+};
+
 // Step k = A + ci, ci its index in the launch sequence: solve of step k-1 (ci > 0), begin of step k, its element forces
 // and the stable dt for step k+1 (the file's head).  eflags (energies): MPS_E_KIN.
 template <typename T, int NEN, int LAW, int MODE>
-__global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int ci, unsigned eflags) {
+__global__ __launch_bounds__(spread_threads<NEN>()) __attribute__((amdgpu_waves_per_eu(NEN == 8 ? (MODE == kPlain && sizeof(T) == 4 ? 5 : 4) : MODE == kPlain && sizeof(T) == 4 ? 4 : 3))) void k_spread(MpsInst I, int ci, unsigned eflags) {
     extern __shared__ __align__(16) double smem[];
     constexpr int EB = NEN == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET;  // elements of a workgroup
     __shared__ uint16_t slx[NEN == 8 ? EB * 8 : 1];
     constexpr int NT = spread_threads<NEN>(), FLIGHT = NEN == 8 ? 8 : 16;
     const int nside = (int)gridDim.x - I.sp_nb, bx = (int)blockIdx.x - nside;  // workgroups of spread_side come first
-    const bool side = bx < 0;
-    const int b = side ? 0 : xcd_tile(bx, I.sp_nb), t = threadIdx.x, ss = I.sp_stride;
+    if (bx < 0) {
+        StepControl c;
+        c.load(I, ci);
+        (void)c.begin(I);
+        if (c.nx.go) spread_side<NEN, MODE>(I, ci, (int)blockIdx.x, c.A, c.nx.time, smem);
+        return;
+    }
+    const int b = xcd_tile(bx, I.sp_nb), t = threadIdx.x, ss = I.sp_stride;
     // tables first: their addresses depend on nothing.  Work item it: direction it % 3 of the workgroup's node it / 3.
     const int4* tab = I.sp_node + (size_t)b * ss;
     int4 E = make_int4(-1, 0, 0, 0);
-    if (t < 3 * ss && !side) E = tab[t / 3];
+    if (t < 3 * ss) E = tab[t / 3];
     // role in the element phase: wave of forces or of stable dt
     const bool force = t < 64;
     const int lane = t & 63, j = t & 7;
@@ -624,16 +669,11 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
         l4 = *reinterpret_cast<const uint2*>(I.sp_lx + (size_t)ec * 4);
     }
     const TetConsts kc = tet_consts(I, ec, true);
-    // step control, the same in every workgroup: read now, used once the nodes' loads are on their way
+    StepControl sc0;  // read now, used once the nodes' loads are on their way
+    sc0.load(I, ci);
+    const long long k = sc0.k;
     MpsCtl* ctl = I.ctl;
-    const long long A = ctl->A, k = A + ci;
-    const MpsStepSlot* pp = ci == 0 ? ctl->slot + ((A - 1) & 1) : ctl->sslot + ((ci - 1) & 1);
-    MpsStepSlot prev;
-    prev.time = pp->time;
-    prev.dt = pp->dt;
-    prev.go = pp->go;
-    const int row = t & (MPS_DT_SLOTS - 1);
-    const unsigned long long m16 = *(ci == 0 ? dt_slot(I, dt_parity(A), row) : dt_spread(I, ci % 3, row));
+    const MpsStepSlot prev = sc0.prev;
     const size_t N = (size_t)I.N;
     double *ur, *wr, *uo, *wo;
     uw_buffers(I, ci & 1, &ur, &wr);
@@ -641,8 +681,8 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
     const T* fr = spread_forces<T>(I, ci + 1);  // step k-1
     NodeLoads<T, FLIGHT> L;
     if (E.x != -1) L.load(I, E, t - 3 * (t / 3), ci == 0, ur, wr, fr);
-    MpsStepSlot nx;
-    const int st = begin_scalars(I, k, prev, row_min(m16), &nx);
+    const int st = sc0.begin(I);
+    const MpsStepSlot nx = sc0.nx;
     if (bx == 0 && t == 0) {
         ctl->sslot[ci & 1] = nx;
         if (st != MPSD_RUNNING) ctl->status = st;
@@ -657,10 +697,6 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
         spread_reset(I, (ci + 2) % 3);
     }
     if (!nx.go) return;
-    if (side) {
-        spread_side<NEN, MODE>(I, ci, (int)blockIdx.x, A, nx.time, smem);
-        return;
-    }
     const double* lf = spread_lf(I, ci + 1);  // step k-1
     double red[MPS_NODE_PARTS] = {0.0, 0.0, 0.0, 0.0};
     double* se = smem + (NEN == 8 ? 9 : 6) * ss;  // staged increments or velocities: se[d*ss + q]
@@ -672,23 +708,24 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread(MpsInst I, int
         }
         if (E.x == -1) break;  // the rest is padding
         const int n = E.x & 0x7FFFFFFF;
+        const bool fixed = entry_fixed(E, d);
         double u = L.u, w;
         if (ci == 0) {
             w = half_velocity(nx.dt, L.w, L.m);
         } else {
             double v, acc, wkin = 0.0;
-            const double fi = L.force(E, fr, d), fe = node_fext1(I, lf, n, L.info, d);
-            node_update1(I, L.info, d, k - 1, prev.dt, L.m, -fi + fe, L.w, &v, &acc, MODE == kEnergy ? &wkin : nullptr);
+            const double fi = L.force(E, fr, d), fe = L.fext(lf, d);
+            dof_update(I, fixed, L.bc, k - 1, prev.dt, L.m, -fi + fe, L.w, &v, &acc, MODE == kEnergy ? &wkin : nullptr);
             if (E.x < 0) check_finite(I, n, d, k - 1, u);
             if constexpr (MODE == kEnergy) {
                 se[d * ss + q] = v;
                 if (E.x < 0)
-                    dof_energy(I, n, L.info, d, k - 1, u, step_increment(I, L.info, d, k - 1, prev.dt, L.w), fi, fe, L.m, v,
-                               wkin, red);
+                    dof_energy(I, E, L.li, d, k - 1, u, dof_increment(I, fixed, L.bc, k - 1, prev.dt, L.w), fi, fe, L.m, v, wkin,
+                               red);
             }
             w = half_velocity(nx.dt, v, acc);
         }
-        u += step_increment(I, L.info, d, k, nx.dt, w);
+        u += dof_increment(I, fixed, L.bc, k, nx.dt, w);
         if constexpr (MODE == kVisc) se[d * ss + q] = u - L.u;
         if (E.x < 0) {
             uo[d * N + n] = u;
@@ -858,11 +895,12 @@ __global__ __launch_bounds__(spread_threads<NEN>()) void k_spread_end(MpsInst I)
         NodeLoads<T, 8> L;
         L.load(I, E, d, false, ur, wr, fr);
         double v, a, wkin = 0.0;
-        const double u = L.u, fi = L.force(E, fr, d), fe = node_fext1(I, lf, n, L.info, d);
-        node_update1(I, L.info, d, k, dt, L.m, -fi + fe, L.w, &v, &a, MODE == kEnergy ? &wkin : nullptr);
+        const double u = L.u, fi = L.force(E, fr, d), fe = L.fext(lf, d);
+        const bool fixed = entry_fixed(E, d);
+        dof_update(I, fixed, L.bc, k, dt, L.m, -fi + fe, L.w, &v, &a, MODE == kEnergy ? &wkin : nullptr);
         check_finite(I, n, d, k, u);
         if constexpr (MODE == kEnergy)
-            dof_energy(I, n, L.info, d, k, u, step_increment(I, L.info, d, k, dt, L.w), fi, fe, L.m, v, wkin, red);
+            dof_energy(I, E, L.li, d, k, u, dof_increment(I, fixed, L.bc, k, dt, L.w), fi, fe, L.m, v, wkin, red);
         I.u[i] = u;
         I.v[i] = v;
         I.a[i] = a;
@@ -928,7 +966,7 @@ __global__ void k_spread_pick(MpsInst I, const int32_t* __restrict__ idx, int64_
     const T* f = spread_forces<T>(I, I.ctl->spread_last);
     NodeLoads<T, 8> L;
 #pragma unroll
-    for (int q = 0; q < 8; q++) L.c[q] = f[3 * ((size_t)E.y + min(q, E.z - 1)) + d];
+    for (int q = 0; q < 8; q++) L.c[q] = f[3 * ((size_t)E.y + min(q, entry_count(E) - 1)) + d];
     out[i] = L.force(E, f, d);
 }
 
