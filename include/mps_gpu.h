@@ -296,8 +296,8 @@ int mps_destroy(mps_handle h);
 
 /* Graph replay of step chunks (default on): when enabled and kernel timing is off, mps_run
  * replays each chunk of steps from a captured hipGraph (one per chunk length and, with energies,
- * per first step modulo energy_every) instead of launching its kernels one by one.  No reference
- * counterpart. */
+ * per first step modulo energy_every) from its second use on, instead of launching its kernels one
+ * by one.  No reference counterpart. */
 int mps_set_graphs(mps_handle h, int32_t enable);
 
 /* Capture and instantiate, without running anything, the graphs that mps_run(h, max_steps) would
