@@ -62,6 +62,25 @@ def test_energies(shape, tet, every, law, monkeypatch):
     same(perturb(box(*shape, tet=tet), 0.1, 7), monkeypatch, energies=every, law=law)
 
 
+@pytest.mark.parametrize("law", [0, 1, 2, 3])
+@pytest.mark.parametrize("shape,tet,every", [((1, 1, 1), False, 1), ((16, 16, 1), False, 3), ((21, 11, 9), False, 2),
+                                             ((11, 1, 1), True, 1), ((9, 7, 6), True, 2)])
+def test_energies_fp32(shape, tet, every, law, monkeypatch):
+    """FP32 forces: the energies stay FP64, in the patch form by a pass of its own with other intermediates.  F's diagonal
+    is rounded at 2^-53; the strains of the state are 1e-4 and more, so energies of the strain agree to some 1e-12 (1e-11
+    here), the volume to 1e-13."""
+    m = perturb(box(*shape, tet=tet), 0.1, 7)
+    kw = dict(energies=every, law=law, precision=G.PREC_FP32_ELEM)
+    (a, ha), (b, hb) = (solve(m, f, monkeypatch, **kw) for f in ("0", "1"))
+    for x, y in zip(a, b):
+        assert np.array_equal(x, y)
+    for key, rtol in (("time", 0), ("dt", 0), ("e_def", 1e-11), ("volume", 1e-13), ("e_kin", 1e-13)):
+        np.testing.assert_allclose(ha[key], hb[key], rtol=rtol, equal_nan=True, err_msg=key)
+    for key in SUMS:
+        scale = np.nanmax(np.abs(ha[key])) if not np.isnan(ha[key]).all() else 0.0
+        np.testing.assert_allclose(ha[key], hb[key], rtol=0, atol=8 * 3 * m["n_nodes"] * 2.0 ** -53 * scale, equal_nan=True)
+
+
 @pytest.mark.parametrize("precision", [G.PREC_FP64, G.PREC_FP32_ELEM])
 @pytest.mark.parametrize("shape", [(1, 1, 1), (3, 3, 1), (16, 16, 1), (257, 1, 1), (11, 9, 7)])
 def test_viscosity(shape, precision, monkeypatch):

@@ -423,14 +423,14 @@ int prepare(const mps_mesh* mesh, const mps_material* mat, const mps_bcs* bcs, c
 }
 
 // Meshes up to this many elements step in the spread form.  us per step, spread / patch form: hex8 FP64 29,800 elements
-// 16.8 / 19.2, 35,900 18.9 / 20.4, 46,700 23.2 / 19.4, FP32 form 35,900 16.0 / 17.4, 46,700 18.6 / 16.7; tet4 FP64 63,900 11.6 /
-// 12.3, 93,800 16.8 / 13.6, FP32 form 35,000 9.8 / 9.9, 48,000 10.3 / 10.0.  With energies every step the patch form gives up
-// more (its energy kernels and sums): hex8 35,800 24.5 / 30.9, 50,700 32.2 / 31.1; tet4 55,600 13.4 / 21.6.  Loads and viscosity
-// come after creation: at 31,700 elements with both 22.8 / 29.2, at 46,700 30.3 / 27.3.  MPS_SPREAD=0 in the environment
-// keeps the patch form, MPS_SPREAD=1 takes the spread form at any size; so do the switches of the patch kernels
-// (MPS_GATHER32, MPS_DT_SKIP, MPS_TET_STAGING), which have no meaning in the spread form.  Both forms give the same bits.
+// 16.8 / 19.2, 35,900 18.9 / 20.4, 46,700 23.2 / 19.4; tet4 FP64 63,900 11.6 / 12.3, 93,800 16.8 / 13.6, FP32 form 35,000
+// 9.8 / 9.9, 48,000 10.3 / 10.0.  With energies every step the patch form gives up more (its energy kernels and sums): hex8
+// 35,800 24.5 / 30.9, 50,700 32.2 / 31.1; tet4 55,600 13.4 / 21.6, 82,900 (FP32 form) 18.1 / 24.6.  Loads and viscosity come
+// after creation: at 31,700 elements with both 22.8 / 29.2, at 46,700 30.3 / 27.3.  MPS_SPREAD=0 in the environment keeps
+// the patch form, MPS_SPREAD=1 takes the spread form at any size; so do the switches of the patch kernels (MPS_GATHER32,
+// MPS_DT_SKIP, MPS_TET_STAGING), which have no meaning in the spread form.  Both forms give the same bits.
 static const int64_t kSpreadMaxHex = 36864, kSpreadMaxTet = 64000, kSpreadMaxTet32 = 40000;
-static const int64_t kSpreadMaxHexEnergy = 49152, kSpreadMaxTetEnergy = 80000;
+static const int64_t kSpreadMaxHexEnergy = 49152, kSpreadMaxTetEnergy = 96000;
 
 void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const int64_t N = hp.N, Ne = hp.Ne, nen = hp.nen;
@@ -438,10 +438,11 @@ void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const char* env = getenv("MPS_SPREAD");
     const bool force = env && strcmp(env, "1") == 0;
     if (env && !force && strcmp(env, "0") == 0) return;
-    const bool fp64 = hp.cfg.precision == MPS_PREC_FP64, en = hp.cfg.energy_every > 0 && fp64;
+    const bool fp64 = hp.cfg.precision == MPS_PREC_FP64, en = hp.cfg.energy_every > 0;
     const int64_t most = nen == 8 ? (en ? kSpreadMaxHexEnergy : kSpreadMaxHex)
                                   : (en ? kSpreadMaxTetEnergy : fp64 ? kSpreadMaxTet : kSpreadMaxTet32);
     if (hp.bcval.size() / 3 > (1u << 23)) return;  // Dirichlet records of an entry
+    if (nen == 8 && hp.cfg.precision != MPS_PREC_FP64) return;  // its roundings are those of the patch kernels (mps_device.h)
     if (!force && (Ne > most || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") ||
                    getenv("MPS_TET_STAGING")))
         return;
@@ -791,7 +792,7 @@ static int upload_instance(mps_solver_s* h, const HostPrep& hp) {
         I.sp_nb = sp.nb;
         I.sp_stride = sp.stride;
         I.n_patch = hp.n_patch;
-        if (I.energy_every > 0 && I.precision == MPS_PREC_FP64) HCHK(h, dalloc(h, &I.sp_ep, mpsk::spread_energy_doubles(I) * 8));
+        if (I.energy_every > 0) HCHK(h, dalloc(h, &I.sp_ep, mpsk::spread_energy_doubles(I) * 8));
     }
     HCHK(h, hipMemcpyAsync(bcval, hp.bcval.data(), hp.bcval.size() * 8, hipMemcpyHostToDevice, h->stream));
     HCHK(h, hipMemsetAsync(hist, 0xFF, MPS_HIST_COLS * (size_t)cap * 8, h->stream));  // NaN
@@ -1504,12 +1505,11 @@ static void collect_times(mps_solver_s* h, const std::vector<int>& kinds) {
 // (FP64 inviscid form) or in the standalone pass before the node kernel; after the last node pass, the pass for
 // the KIN_ENERGY of the chunk's last step.  The node kernels accumulate the work sums every step.
 // True when the steps run in the spread form: set up at creation, and nothing in the step that only the patch form has
-// (DOF series, pressure loads, which need the step's displacement, energies with FP32 forces or with viscosity, viscous
-// tet4 elements).
+// (DOF series, pressure loads, which need the step's displacement, energies with viscosity, viscous tet4 elements).
 static bool use_spread(const mps_solver_s* h) {
     const MpsInst& I = h->I;
     return I.sp_nb > 0 && !h->step_begun && I.n_series == 0 && !h->pressure_loads &&
-           (I.energy_every == 0 || mpsk::elem_fuses_energy(I)) && (I.uprev == nullptr || I.nen == 8);
+           (I.uprev == nullptr || (I.energy_every == 0 && I.nen == 8));
 }
 
 // Spread form of enqueue_steps: one launch per step, and the end of the sequence.

@@ -151,6 +151,31 @@ __device__ __forceinline__ void cof3(const T* A, T* C) {
     C[8] = diff2(A[0], A[4], A[1], A[3]);
 }
 
+// FP32 hex8 (functions _c, hex_grad, hex_char_length_pf, add_bulk_visc): the compiler chooses the FMAs, across these
+// functions.  Single roundings of the stresses are what an FP32 solve from rest sees in its accelerations (2e-4 of them),
+// so that this form keeps the choice it has always had, and hex8 meshes in it stay in the patch form.
+__device__ __forceinline__ void cof3_c(const float* A, float* C) {
+    C[0] = A[4] * A[8] - A[5] * A[7];
+    C[1] = A[5] * A[6] - A[3] * A[8];
+    C[2] = A[3] * A[7] - A[4] * A[6];
+    C[3] = A[2] * A[7] - A[1] * A[8];
+    C[4] = A[0] * A[8] - A[2] * A[6];
+    C[5] = A[1] * A[6] - A[0] * A[7];
+    C[6] = A[1] * A[5] - A[2] * A[4];
+    C[7] = A[2] * A[3] - A[0] * A[5];
+    C[8] = A[0] * A[4] - A[1] * A[3];
+}
+
+__device__ __forceinline__ float det3_c(const float* A) {
+    return A[0] * (A[4] * A[8] - A[7] * A[5]) - A[1] * (A[3] * A[8] - A[6] * A[5]) +
+           A[2] * (A[3] * A[7] - A[6] * A[4]);
+}
+__device__ __forceinline__ float detIpH_m1_c(const float* H) {
+    float tr = H[0] + H[4] + H[8];
+    float i2 = H[0] * H[4] + H[4] * H[8] + H[0] * H[8] - H[1] * H[3] - H[5] * H[7] - H[2] * H[6];
+    return tr + i2 + det3_c(H);
+}
+
 // Reciprocal: hardware estimate refined by Newton steps (<= 1 ulp for FP64).
 __device__ __forceinline__ double rcp(double x) {
 #pragma clang fp contract(off)
@@ -184,7 +209,6 @@ __device__ __forceinline__ double log_near1(double J) {
 // log(1+x) (FP32): Taylor series to x^9 for |x| < 0.05 (truncation < 2e-13 relative);
 // otherwise Goldberg's form log(u) * x / (u - 1), u = 1 + x.
 __device__ __forceinline__ float log1p_fast(float x) {
-#pragma clang fp contract(off)
     if (fabsf(x) < 0.05f) {
         float p = 1.f / 9.f;
         p = fmaf(p, x, -1.f / 8.f);
@@ -238,6 +262,37 @@ __device__ __forceinline__ void pk1_svk_lin(const T* H, T lam, T mu, T* P) {
 #pragma unroll
         for (int j = 0; j < 3; j++)
             P[i * 3 + j] = fma_t(H[i * 3 + 2], S[6 + j], fma_t(H[i * 3 + 1], S[3 + j], fma_t(H[i * 3], S[j], S[i * 3 + j])));
+}
+
+template <int LAW>
+__device__ __forceinline__ void pk1_svk_lin_c(const float* H, float lam, float mu, float* P) {
+    float E[9];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            float e = 0.5f * (H[i * 3 + j] + H[j * 3 + i]);
+            if (LAW == 2) e += 0.5f * (H[i] * H[j] + H[3 + i] * H[3 + j] + H[6 + i] * H[6 + j]);
+            E[i * 3 + j] = e;
+        }
+    const float ltr = lam * (E[0] + E[4] + E[8]);
+    const float mu2 = 2.f * mu;
+    float S[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) S[i] = mu2 * E[i];
+    S[0] += ltr;
+    S[4] += ltr;
+    S[8] += ltr;
+    if (LAW == 3) {
+#pragma unroll
+        for (int i = 0; i < 9; i++) P[i] = S[i];
+        return;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            P[i * 3 + j] = S[i * 3 + j] + H[i * 3] * S[j] + H[i * 3 + 1] * S[3 + j] + H[i * 3 + 2] * S[6 + j];
 }
 
 __device__ __forceinline__ double defo_energy(int law, const double* F, double lambda, double mu);
@@ -371,6 +426,68 @@ __device__ __forceinline__ void pk1(const float* H, float pa, float pb, float* P
 #pragma unroll
             for (int j = 0; j < 3; j++)
                 P[i * 3 + j] = dot3(sg[i * 3], cF[j], sg[i * 3 + 1], cF[3 + j], sg[i * 3 + 2], cF[6 + j]);
+    }
+}
+// The same for hex8 elements, contracted by the compiler (cof3_c).
+template <int LAW>
+__device__ __forceinline__ void pk1_c(const float* H, float pa, float pb, float* P) {
+    if (LAW >= 2) {
+        pk1_svk_lin_c<LAW>(H, pa, pb, P);
+        return;
+    }
+    if (LAW == 0) {  // pa = lambda, pb = mu
+        float cH[9];
+        cof3_c(H, cH);
+        const float tr = H[0] + H[4] + H[8];
+        const float sv = (cH[0] + cH[4] + cH[8]) + (H[0] * cH[0] + H[1] * cH[1] + H[2] * cH[2]);
+        const float Jm1 = tr + sv;
+        const float lt = pa * log1p_fast(Jm1);
+        const float rJ = rcp(1.f + Jm1);
+        const float a = (pb - lt) * rJ;
+        const float b = (pb * sv + lt * (1.f + tr)) * rJ;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++) P[i * 3 + j] = pb * H[i * 3 + j] + a * (H[j * 3 + i] - cH[i * 3 + j]);
+        P[0] += b;
+        P[4] += b;
+        P[8] += b;
+        return;
+    }
+    const float Jm1 = detIpH_m1_c(H);
+    const float lnJ = log1p_fast(Jm1);
+    float F[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) F[i] = H[i];
+    F[0] += 1.f;
+    F[4] += 1.f;
+    F[8] += 1.f;
+    float cF[9];
+    cof3_c(F, cF);
+    {  // Belytschko (pa = mu, pb = K1): sigma = mu J^{-5/3} dev(B - I) + K (J-1) I ; P = sigma cof(F)
+        float Bm[9];
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = i; j < 3; j++) {
+                Bm[i * 3 + j] = H[i * 3 + j] + H[j * 3 + i] + H[i * 3] * H[j * 3] + H[i * 3 + 1] * H[j * 3 + 1] +
+                                H[i * 3 + 2] * H[j * 3 + 2];
+                Bm[j * 3 + i] = Bm[i * 3 + j];
+            }
+        const float tr3 = (Bm[0] + Bm[4] + Bm[8]) * (1.f / 3.f);
+        const float f2 = pa * __expf(-(5.f / 3.f) * lnJ);
+        const float vol = pb * Jm1 - f2 * tr3;
+        float sg[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) sg[i] = f2 * Bm[i];
+        sg[0] += vol;
+        sg[4] += vol;
+        sg[8] += vol;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                P[i * 3 + j] = sg[i * 3] * cF[j] + sg[i * 3 + 1] * cF[3 + j] + sg[i * 3 + 2] * cF[6 + j];
     }
 }
 
@@ -560,35 +677,25 @@ __device__ __forceinline__ bool tet_dt_above(const double (*x)[3], double l0, do
 // FP32 characteristic lengths for the precision form (the reference formulas with FP32 areas, volume and
 // ratio, hardware square root and reciprocal).  Tet: edge vectors differenced in FP64, so there is no
 // cancellation against the absolute coordinates; hex: from node positions relative to their centroid.
-// Norm of the cross product, twice the triangle's area.
-__device__ __forceinline__ float norm_tri_pf(const float* p, const float* q, const float* r) {
-#pragma clang fp contract(off)
+__device__ __forceinline__ float area_tri_pf(const float* p, const float* q, const float* r) {
     const float A0 = p[0] - r[0], A1 = p[1] - r[1], A2 = p[2] - r[2];
     const float B0 = q[0] - r[0], B1 = q[1] - r[1], B2 = q[2] - r[2];
-    const float C0 = diff2(A1, B2, A2, B1), C1 = diff2(A2, B0, A0, B2), C2 = diff2(A0, B1, A1, B0);
-    return __builtin_amdgcn_sqrtf(dot3(C0, C0, C1, C1, C2, C2));  // hardware sqrt, 1 ulp
-}
-
-// Twice the inscribed-sphere radius from the area sum A and the corner edges M (rows 0-1, 0-3, 0-4).
-__device__ __forceinline__ float hex_length_pf(const float* M, float A) {
-#pragma clang fp contract(off)
-    return 6.0f * fabsf(det3(M)) * __builtin_amdgcn_rcpf(A);
+    const float C0 = A1 * B2 - A2 * B1, C1 = A2 * B0 - A0 * B2, C2 = A0 * B1 - A1 * B0;
+    return 0.5f * __builtin_amdgcn_sqrtf(C0 * C0 + C1 * C1 + C2 * C2);  // hardware sqrt, 1 ulp
 }
 __device__ __forceinline__ float hex_char_length_pf(const float (*x)[3]) {
-#pragma clang fp contract(off)
     const int fc[6][4] = {{0, 1, 2, 3}, {4, 5, 6, 7}, {0, 1, 5, 4}, {1, 2, 6, 5}, {2, 3, 7, 6}, {0, 3, 7, 4}};
     float A = 0.0f;
 #pragma unroll
     for (int f = 0; f < 6; f++)
-        A += fma_t(0.5f, norm_tri_pf(x[fc[f][0]], x[fc[f][1]], x[fc[f][2]]),
-                   0.5f * norm_tri_pf(x[fc[f][0]], x[fc[f][2]], x[fc[f][3]]));
+        A += area_tri_pf(x[fc[f][0]], x[fc[f][1]], x[fc[f][2]]) + area_tri_pf(x[fc[f][0]], x[fc[f][2]], x[fc[f][3]]);
     float M[9];
     const int c[3] = {1, 3, 4};
 #pragma unroll
     for (int j = 0; j < 3; j++)
 #pragma unroll
         for (int d = 0; d < 3; d++) M[j * 3 + d] = x[c[j]][d] - x[0][d];
-    return hex_length_pf(M, A);
+    return 6.0f * fabsf(det3_c(M)) * __builtin_amdgcn_rcpf(A);
 }
 
 // Tet: from the deformed edge vectors e_j = x_{j+1} - x_0 = Jm(:,j) + Du(:,j), whose parts the element already
@@ -779,6 +886,21 @@ __device__ __forceinline__ void add_bulk_visc(const T* H, T trD, T qa, T qb, T* 
     for (int i = 0; i < 9; i++) P[i] = fma_t(q, cF[i], P[i]);
 }
 
+__device__ __forceinline__ void add_bulk_visc(const float* H, float trD, float qa, float qb, float* P) {
+    const float J = 1.f + detIpH_m1_c(H);
+    const float mn = trD < 0.f ? trD : 0.f;
+    const float q = (qa * fabs(trD) * mn + qb * trD) / J;
+    float F[9], cF[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) F[i] = H[i];
+    F[0] += 1.f;
+    F[4] += 1.f;
+    F[8] += 1.f;
+    cof3_c(F, cF);
+#pragma unroll
+    for (int i = 0; i < 9; i++) P[i] += q * cF[i];
+}
+
 // Viscosity coefficients of element e (qa, qb of add_bulk_visc); element size and sound speed are the
 // element's undeformed length and sound speed unless given.
 __device__ __forceinline__ void visc_coeffs(const MpsInst& I, int e, double c, double* qa, double* qb) {
@@ -897,6 +1019,18 @@ __device__ __forceinline__ void hex_grad(const T* Jm, const T* Du, T* cJ, T* H, 
         }
 }
 
+__device__ __forceinline__ void hex_grad(const float* Jm, const float* Du, float* cJ, float* H, float*, float* dJ, float* rJ) {
+    cof3_c(Jm, cJ);
+    const float d = Jm[0] * cJ[0] + Jm[1] * cJ[1] + Jm[2] * cJ[2], r = rcp(d);
+    *dJ = d;
+    *rJ = r;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            H[i * 3 + j] = (Du[i * 3] * cJ[j * 3] + Du[i * 3 + 1] * cJ[j * 3 + 1] + Du[i * 3 + 2] * cJ[j * 3 + 2]) * r;
+}
+
 // Row i of tr(D cof(J)^T) for the gradient D of the displacement increment, from its coefficients a[m] (component i).
 template <typename T>
 __device__ __forceinline__ T hex_visc_trace(const T* a, const GpSigns<T>& s, const T* cJ) {
@@ -905,6 +1039,11 @@ __device__ __forceinline__ T hex_visc_trace(const T* a, const GpSigns<T>& s, con
     const T d1 = fma_t(s.xz, a[6], fma_t(s.z, a[4], fma_t(s.x, a[3], a[1])));
     const T d2 = fma_t(s.xy, a[6], fma_t(s.y, a[4], fma_t(s.x, a[5], a[2])));
     return dot3(d0, cJ[0], d1, cJ[1], d2, cJ[2]);
+}
+
+__device__ __forceinline__ float hex_visc_trace(const float* a, const GpSigns<float>& s, const float* cJ) {
+    return (a[0] + s.y * a[3] + s.z * a[5] + s.yz * a[6]) * cJ[0] + (a[1] + s.x * a[3] + s.z * a[4] + s.xz * a[6]) * cJ[1] +
+           (a[2] + s.x * a[5] + s.y * a[4] + s.xy * a[6]) * cJ[2];
 }
 
 // Stress at a hex8 Gauss point from hex_grad's H and Fd.
@@ -920,7 +1059,7 @@ __device__ __forceinline__ void hex_pk1(const double* H, const double* Fd, doubl
 }
 template <int LAW>
 __device__ __forceinline__ void hex_pk1(const float* H, const float*, float pa, float pb, float* P) {
-    pk1<LAW>(H, pa, pb, P);
+    pk1_c<LAW>(H, pa, pb, P);
 }
 
 // Columns Q[k][i] of wJ P J^-T: weight 1 (GPsDistribution.cpp:392-432), so wJ J^-T = sign(det J) cof(J) and
@@ -1021,7 +1160,7 @@ __device__ __forceinline__ double hex8_element(const MpsInst& I, int e, const do
         T Jm[9], Du[9], H[9], Fd[3];
         hex_jac<T>(Ax, s, Jm);
         hex_jac<T>(Au, s, Du);
-        hex_grad<T>(Jm, Du, cJ, H, Fd, &dJ, &rJ);
+        hex_grad(Jm, Du, cJ, H, Fd, &dJ, &rJ);
         if constexpr (EN) {  // weight 1: wJ = |det J| (classGPs.cpp:26-27)
             double Wg, Jg;
             hex_pk1<LAW>(H, Fd, tpa, tpb, P, &Wg, &Jg);
@@ -1046,7 +1185,7 @@ __device__ __forceinline__ double hex8_element(const MpsInst& I, int e, const do
                 const T a[7] = {a0, a1, a2, a3, a4, a5, a6};
                 tr += hex_visc_trace(a, s, cJ + 3 * i);
             }
-            add_bulk_visc<T>(H, tr * rJ * trs, qa, qb, P);
+            add_bulk_visc(H, tr * rJ * trs, qa, qb, P);
         }
         hex_stress_columns<T>(P, cJ, dJ, Q);
         // moment sums, one FMA per (moment, column) pair: a +-1 factor makes each product exact
@@ -1182,7 +1321,7 @@ __device__ __forceinline__ double tet4_core(const MpsInst& I, int e, const int* 
         for (int i = 0; i < 3; i++) tr += Dd[i * 3] * iJ[i] + Dd[i * 3 + 1] * iJ[3 + i] + Dd[i * 3 + 2] * iJ[6 + i];
         double da, db;
         visc_coeffs(I, e, c, &da, &db);
-        add_bulk_visc<T>(H, tr * (T)rdt, (T)da, (T)db, P);
+        add_bulk_visc(H, tr * (T)rdt, (T)da, (T)db, P);
     }
     T dphi[4][3];
 #pragma unroll

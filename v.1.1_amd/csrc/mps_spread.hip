@@ -16,16 +16,17 @@
 // over the patches -- and an element's arithmetic is the same function by function, so both forms give the same bits.
 //
 // Measured, us per step, patch form / here.  hex8 FP64: 1,000 elements 17.7 / 5.6, 8,000 18.4 / 7.4, 15,600 19.1 / 10.2,
-// 29,800 19.2 / 16.8, 46,700 19.4 / 23.2; FP32 form: 1,000 14.6 / 5.6, 15,600 16.2 / 9.3, 29,800 16.5 / 14.2; tet4 FP64: 750
-// 12.3 / 6.6, 10,400 12.2 / 6.7, 48,000 12.2 / 10.2, 93,800 13.6 / 16.8; FP32 form: 10,400 9.7 / 6.4, 48,000 10.0 / 10.3.
+// 29,800 19.2 / 16.8, 46,700 19.4 / 23.2; tet4 FP64: 750 12.3 / 6.6, 10,400 12.2 / 6.7, 48,000 12.2 / 10.2, 93,800 13.6 /
+// 16.8; FP32 form: 10,400 9.7 / 6.4, 48,000 10.0 / 10.3.  Hex8 meshes in the FP32 form keep the patch kernels, whose FMAs the
+// compiler chooses (cof3_c in mps_device.h).
 // Every node is updated by all the workgroups that hold it (4.5 per 8 hex8 elements where the patch form has 1.03 per
 // element), so past the size where the lanes are no longer idle the patch form is the better one.
 // With energies every step and loads (hex8 FP64): 512 elements 29.3 / 7.3, 12,200 30.2 / 12.1, 35,800 30.9 / 24.5; tet4 750
-// 22.0 / 7.2, 55,600 21.6 / 13.4; with viscosity and loads (FP64 Belytschko): 512 23.4 / 6.6, 12,200 25.2 / 11.6, 31,700 29.2 /
-// 22.8.  The patch form takes three launches for these steps; here the external forces and the energy sums are extra
-// workgroups of the step's launch, on a path of their own from the first instruction, and without the pressure loads'
-// code: sharing the element workgroups' prologue, with that code, cost 48 registers, two of five waves per SIMD, and 18.7
-// instead of 16.8 us at 29,800 elements.
+// 22.0 / 7.2, 55,600 21.6 / 13.4, FP32 form 55,600 22.6 / 12.9; with viscosity and loads (FP64 Belytschko): 512 23.4 / 6.6,
+// 12,200 25.2 / 11.6, 31,700 29.2 / 22.8.  The patch form takes three launches for these steps; here the external forces
+// and the energy sums are extra workgroups of the step's launch, on a path of their own from the first instruction, and
+// without the pressure loads' code: sharing the element workgroups' prologue, with that code, cost 48 registers, two of
+// five waves per SIMD, and 18.7 instead of 16.8 us at 29,800 elements.
 // Tried: one wave per workgroup, which takes the dt and the forces in turn (half the waves): 2 us more at 1,000 elements and
 // the same above 30,000, where the issue of 1,380 vector instructions per 8 elements is the bound, not the waves in flight.
 // Tried: 16 and 32 hex8 elements per workgroup: fewer shared nodes, but 0.4 to 1.8 us more up to 2,000 elements and
@@ -38,10 +39,10 @@ using namespace mpsd;
 
 namespace {
 
-// LDS of the hex8 element phase, in values of T per element: butterfly coefficients of X and u (42), later the moment
-// sums (21); stress columns of the eight points (72); face triangle areas (12); FP32 node positions (24).  Coefficients
+// LDS of the hex8 element phase, in values per element: butterfly coefficients of X and u (42), later the moment
+// sums (21); stress columns of the eight points (72); face triangle areas (12).  Coefficients
 // and columns are read in 16-byte pieces; with these strides the eight elements of a wave fall into different banks.
-constexpr int kCoef = 44, kCol = 76, kArea = 12, kPos = 24;
+constexpr int kCoef = 44, kCol = 76, kArea = 12;
 
 // LDS exchange between the lanes of one wavefront: LDS operations of a wave stay in order, so only the compiler has to
 // be kept from moving them.
@@ -238,7 +239,7 @@ __device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restri
         T Jm[9], Du[9], cJ[9], H[9], Fd[3], P[9], Q[3][3], dJ, rJ;
         hex_jac<T>(Ax, s, Jm);
         hex_jac<T>(Au, s, Du);
-        hex_grad<T>(Jm, Du, cJ, H, Fd, &dJ, &rJ);
+        hex_grad(Jm, Du, cJ, H, Fd, &dJ, &rJ);
         if constexpr (MODE == kEnergy) {  // weight 1: wJ = |det J|
             double Wg, Jg;
             hex_pk1<LAW>(H, Fd, pa, pb, P, &Wg, &Jg);
@@ -257,7 +258,7 @@ __device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restri
                 for (int m = 0; m < 7; m++) a[m] = ex.sv[m * 3 + i];
                 tr += hex_visc_trace(a, s, cJ + 3 * i);
             }
-            add_bulk_visc<T>(H, tr * rJ * ex.rdt, ex.qa, ex.qb, P);
+            add_bulk_visc(H, tr * rJ * ex.rdt, ex.qa, ex.qb, P);
         }
         hex_stress_columns<T>(P, cJ, dJ, Q);
 #pragma unroll
@@ -316,82 +317,43 @@ __device__ __forceinline__ void hex_spread_force(T* __restrict__ sc, T* __restri
 }
 
 // Stable dt of the eight elements of a force wave, by a wave of their own: the 96 face triangles over its lanes, then one
-// lane per element.  sc: the elements' coefficients (FP32 form), sp: their node positions (FP32 form).  Returns the
-// element's dt in lanes 0-7.
-template <typename T>
+// lane per element.  Returns the element's dt in lanes 0-7.
 __device__ __forceinline__ double hex_spread_dt(const double* __restrict__ sn, int ss, const uint16_t* __restrict__ slx,
-                                                const T* __restrict__ sc, T* __restrict__ sa, T* __restrict__ sp, int lane,
-                                                double c, double l0) {
+                                                double* __restrict__ sa, int lane, double c, double l0) {
 #pragma clang fp contract(off)
-    if constexpr (sizeof(T) == 4) {  // node positions relative to the centroid (hex8_element), node j of element el
-        const int el = lane >> 3, j = lane & 7;
-        T A[44];
-        lds_read<44>(sc + el * kCoef, A);
-        const T ig = (T)(1.0 / MPS_GP), ig2 = (T)(1.0 / (MPS_GP * MPS_GP));
-        const T zs = unit_signed(T(), (j >> 2) ^ 1);
-        T tss[3], tsd[3], tds[3], tdd[3], x[3];
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-            tss[d] = zs * (A[6 + d] + A[27 + d]);
-            tsd[d] = (A[3 + d] + A[24 + d]) + zs * ((A[12 + d] + A[33 + d]) * ig);
-            tds[d] = (A[d] + A[21 + d]) + zs * ((A[15 + d] + A[36 + d]) * ig);
-            tdd[d] = (A[9 + d] + A[30 + d]) * ig + zs * ((A[18 + d] + A[39 + d]) * ig2);
-        }
-        unbutterfly_node<T>(j, tss, tsd, tds, tdd, x);
-#pragma unroll
-        for (int d = 0; d < 3; d++) sp[el * kPos + j * 3 + d] = x[d];
-        wave_sync();
-    }
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         const int it = lane + 64 * r;
         if (it < 96) {
             const int el = it / 12, t = it - 12 * el, code = hex_triangle(t);
-            T p[3][3];
+            double p[3][3];
 #pragma unroll
             for (int v = 0; v < 3; v++) {
                 const int a = (code >> (3 * v)) & 7;
 #pragma unroll
-                for (int d = 0; d < 3; d++)
-                    p[v][d] = sizeof(T) == 8 ? (T)sn[(6 + d) * ss + slx[el * 8 + a]] : sp[el * kPos + a * 3 + d];
+                for (int d = 0; d < 3; d++) p[v][d] = sn[(6 + d) * ss + slx[el * 8 + a]];
             }
-            if constexpr (sizeof(T) == 8) {
-                double n2 = tri_norm2(p[0], p[1], p[2]);
-                sqrt_n<1>(&n2);
-                sa[it] = 0.5 * n2;
-            } else {
-                sa[it] = 0.5f * norm_tri_pf(p[0], p[1], p[2]);
-            }
+            double n2 = tri_norm2(p[0], p[1], p[2]);
+            sqrt_n<1>(&n2);
+            sa[it] = 0.5 * n2;
         }
     }
     wave_sync();
     if (lane >= 8) return 0.0;
-    T a[12], A = T(0);
+    double a[12], A = 0.0;
     lds_read<12>(sa + lane * kArea, a);
 #pragma unroll
     for (int q = 0; q < 6; q++) {
-        const T s = a[2 * q] + a[2 * q + 1];
-        if constexpr (sizeof(T) == 8) A = q == 0 ? fabs(s) : A + fabs(s);
-        else A += s;
+        const double s = a[2 * q] + a[2 * q + 1];
+        A = q == 0 ? fabs(s) : A + fabs(s);
     }
-    if constexpr (sizeof(T) == 8) {
-        double x[5][3];
-        const int nd[4] = {0, 1, 3, 4};
+    double x[5][3];
+    const int nd[4] = {0, 1, 3, 4};
 #pragma unroll
-        for (int v = 0; v < 4; v++)
+    for (int v = 0; v < 4; v++)
 #pragma unroll
-            for (int d = 0; d < 3; d++) x[nd[v]][d] = sn[(6 + d) * ss + slx[lane * 8 + nd[v]]];
-        return elem_dt(length_of(hex_corner_volume((const double(*)[3])x), A), l0, c);
-    } else {
-        float M[9];
-        const int cn[3] = {1, 3, 4};
-        const T* x = sp + lane * kPos;
-#pragma unroll
-        for (int q = 0; q < 3; q++)
-#pragma unroll
-            for (int d = 0; d < 3; d++) M[q * 3 + d] = x[cn[q] * 3 + d] - x[d];
-        return elem_dt((double)hex_length_pf(M, A), l0, c);
-    }
+        for (int d = 0; d < 3; d++) x[nd[v]][d] = sn[(6 + d) * ss + slx[lane * 8 + nd[v]]];
+    return elem_dt(length_of(hex_corner_volume((const double(*)[3])x), A), l0, c);
 }
 
 // Threads of a workgroup: hex8 eight lanes per element for the forces and as many for the stable dt; tet4 a wave for the
@@ -402,7 +364,7 @@ constexpr int spread_threads() {
 }
 template <typename T, int NEN>
 constexpr size_t fixed_lds() {
-    return NEN == 8 ? sizeof(T) * MPS_SPREAD_HEX * (kCol + kCoef + kArea + (sizeof(T) == 4 ? kPos : 0)) : 0;
+    return NEN == 8 ? sizeof(T) * MPS_SPREAD_HEX * (kCol + kCoef + kArea) : 0;
 }
 // Bytes of dynamic LDS: staged node values (hex8 X, u, X + u; tet4 X, u; with viscosity the increments, with energies the
 // velocities), then the element phase's arrays.
@@ -630,7 +592,7 @@ struct StepControl {
 // Step k = A + ci, ci its index in the launch sequence: solve of step k-1 (ci > 0), begin of step k, its element forces
 // and the stable dt for step k+1 (the file's head).  eflags (energies): MPS_E_KIN.
 template <typename T, int NEN, int LAW, int MODE>
-__global__ __launch_bounds__(spread_threads<NEN>()) __attribute__((amdgpu_waves_per_eu(NEN == 8 ? (MODE == kPlain && sizeof(T) == 4 ? 5 : 4) : MODE == kPlain && sizeof(T) == 4 ? 4 : 3))) void k_spread(MpsInst I, int ci, unsigned eflags) {
+__global__ __launch_bounds__(spread_threads<NEN>()) __attribute__((amdgpu_waves_per_eu(NEN == 8 ? 4 : MODE == kPlain && sizeof(T) == 4 ? 4 : 3))) void k_spread(MpsInst I, int ci, unsigned eflags) {
     extern __shared__ __align__(16) double smem[];
     constexpr int EB = NEN == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET;  // elements of a workgroup
     __shared__ uint16_t slx[NEN == 8 ? EB * 8 : 1];
@@ -782,8 +744,7 @@ __global__ __launch_bounds__(spread_threads<NEN>()) __attribute__((amdgpu_waves_
             ex.qb = (T)db;
             ex.rdt = (T)(nx.dt == 0.0 ? 0.0 : 1 / nx.dt);
         }
-        if constexpr (sizeof(T) == 4) __syncthreads();  // the FP32 lengths are taken from the coefficients
-        else wave_sync();
+        wave_sync();
         if (force) {
             T f[3];
             hex_spread_force<T, LAW, MODE>(sc + el * kCoef, base + el * kCol, j, kc.pa, kc.pb, f, ex);
@@ -818,8 +779,7 @@ __global__ __launch_bounds__(spread_threads<NEN>()) __attribute__((amdgpu_waves_
             }
             return;
         }
-        const double dte = hex_spread_dt<T>(smem, ss, slx, sc, base + EB * (kCol + kCoef), base + EB * (kCol + kCoef + kArea),
-                                            lane, kc.c, kc.l0);
+        const double dte = hex_spread_dt(smem, ss, slx, base + EB * (kCol + kCoef), lane, kc.c, kc.l0);
         if (lane < 8 && mine) dmin = d2bits(dte);
     } else {
         if (t >= 128) {
@@ -833,7 +793,11 @@ __global__ __launch_bounds__(spread_threads<NEN>()) __attribute__((amdgpu_waves_
         if (force) {
             T f[4][3];
             double r[4];
-            tet4_core<T, LAW, false, MODE == kEnergy>(I, e, nullptr, x, uu, kc, f, false, 0.0, r);
+            tet4_core<T, LAW, false, MODE == kEnergy && sizeof(T) == 8>(I, e, nullptr, x, uu, kc, f, false, 0.0, r);
+            if constexpr (MODE == kEnergy && sizeof(T) == 4) {  // the energies in FP64
+                double f64[4][3];
+                tet4_core<double, LAW, false, true>(I, e, nullptr, x, uu, kc, f64, false, 0.0, r);
+            }
             if (mine) {
 #pragma unroll
                 for (int a = 0; a < 4; a++) {
@@ -991,22 +955,15 @@ hipError_t launch_spread(const MpsInst& I, int ci, unsigned eflags, hipStream_t 
         default: MPS_SPREAD(T, NEN, 3, M); break;       \
     }
     const int mode = spread_mode(I);
+    const bool f32 = I.precision == 1;
     if (I.nen == 8) {
-        if (I.precision == 1) {
-            if (mode == kVisc) { MPS_SPREAD_LAW(float, 8, kVisc) } else { MPS_SPREAD_LAW(float, 8, kPlain) }
-        } else if (mode == kVisc) {
-            MPS_SPREAD_LAW(double, 8, kVisc)
-        } else if (mode == kEnergy) {
-            MPS_SPREAD_LAW(double, 8, kEnergy)
-        } else {
-            MPS_SPREAD_LAW(double, 8, kPlain)
-        }
-    } else if (I.precision == 1) {
-        MPS_SPREAD_LAW(float, 4, kPlain)
+        if (mode == kVisc) { MPS_SPREAD_LAW(double, 8, kVisc) }
+        else if (mode == kEnergy) { MPS_SPREAD_LAW(double, 8, kEnergy) }
+        else { MPS_SPREAD_LAW(double, 8, kPlain) }
     } else if (mode == kEnergy) {
-        MPS_SPREAD_LAW(double, 4, kEnergy)
+        if (f32) { MPS_SPREAD_LAW(float, 4, kEnergy) } else { MPS_SPREAD_LAW(double, 4, kEnergy) }
     } else {
-        MPS_SPREAD_LAW(double, 4, kPlain)
+        if (f32) { MPS_SPREAD_LAW(float, 4, kPlain) } else { MPS_SPREAD_LAW(double, 4, kPlain) }
     }
 #undef MPS_SPREAD_LAW
 #undef MPS_SPREAD
@@ -1017,15 +974,16 @@ hipError_t launch_spread_end(const MpsInst& I, hipStream_t st) {
     const unsigned nb = (unsigned)I.sp_nb;
     const bool en = spread_mode(I) == kEnergy;
 #define MPS_SPREAD_END(T, NEN, M) k_spread_end<T, NEN, M><<<nb, spread_threads<NEN>(), 0, st>>>(I)
+#define MPS_SPREAD_END_T(NEN, M)                         \
+    if (I.precision == 1) MPS_SPREAD_END(float, NEN, M); \
+    else MPS_SPREAD_END(double, NEN, M)
     if (I.nen == 8) {
-        if (I.precision == 1) MPS_SPREAD_END(float, 8, kPlain);
-        else if (en) MPS_SPREAD_END(double, 8, kEnergy);
+        if (en) MPS_SPREAD_END(double, 8, kEnergy);
         else MPS_SPREAD_END(double, 8, kPlain);
     } else {
-        if (I.precision == 1) MPS_SPREAD_END(float, 4, kPlain);
-        else if (en) MPS_SPREAD_END(double, 4, kEnergy);
-        else MPS_SPREAD_END(double, 4, kPlain);
+        if (en) { MPS_SPREAD_END_T(4, kEnergy); } else { MPS_SPREAD_END_T(4, kPlain); }
     }
+#undef MPS_SPREAD_END_T
 #undef MPS_SPREAD_END
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
