@@ -1725,6 +1725,7 @@ extern "C" int mps_run(mps_handle h, int64_t max_steps, mps_report* rep) {
         if (e != hipSuccess) return h->fail(MPS_ERR_HIP, fmt("first dt: %s", hipGetErrorString(e)));
         h->primed = true;
     }
+    const long long first = c.A;
     HCHK(h, hipEventRecord(h->ev0, h->stream));
     float total_ms = 0.f;
     for (long long n : chunk_plan(h, max_steps)) {
@@ -1753,8 +1754,10 @@ extern "C" int mps_run(mps_handle h, int64_t max_steps, mps_report* rep) {
     }
     HCHK(h, hipEventElapsedTime(&total_ms, h->ev0, h->ev1));
     r.device_ms = total_ms;
-    h->part_valid = true;  // the forces are those of the last completed step's u
-    h->spread_forces = use_spread(h);
+    if (c.A > first) {  // a run that found the end before a step leaves the forces where they were
+        h->part_valid = true;  // the forces are those of the last completed step's u
+        h->spread_forces = use_spread(h);
+    }
     if (rep) *rep = r;
     return status_code(r.status);
 }
