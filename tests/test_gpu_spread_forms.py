@@ -54,3 +54,38 @@ def test_forces_after_a_first_step_that_fails(series):
     with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=10) as s:
         s.set_state(u)
         assert np.array_equal(s.internal_force_dofs(dofs), f)
+
+
+def spread(s):
+    """True when the next steps of s run in the spread form: one launch per step and one at the end, where the patch form
+    has a node kernel in every step."""
+    s.profile(True)
+    before = s.kernel_times()["node"][1]
+    rc, rep = s.run(3)
+    assert rc == 0, rep
+    n = s.kernel_times()["node"][1] - before
+    s.profile(False)
+    assert n in (1, 3), n
+    return n == 1
+
+
+def form(m, **kw):
+    dd, dv = clamp_and_pull(m)
+    with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=10, **kw) as s:
+        return spread(s)
+
+
+@pytest.mark.parametrize("shape,tet,precision,every,expected", [
+    ((33, 33, 33), False, G.PREC_FP64, 0, True), ((34, 34, 34), False, G.PREC_FP64, 0, False),
+    ((34, 34, 34), False, G.PREC_FP64, 1, True), ((34, 34, 34), False, G.PREC_FP64, 2, True),
+    ((34, 34, 34), False, G.PREC_FP64, 3, False), ((33, 33, 33), False, G.PREC_FP64, 100, True),
+    ((36, 36, 35), False, G.PREC_FP64, 1, False), ((36, 36, 35), False, G.PREC_FP64, 100, False),
+    ((22, 22, 22), True, G.PREC_FP64, 0, True), ((22, 23, 22), True, G.PREC_FP64, 0, False),
+    ((24, 24, 24), True, G.PREC_FP64, 2, True), ((24, 24, 24), True, G.PREC_FP64, 5, False),
+    ((22, 22, 22), True, G.PREC_FP32_ELEM, 100, True), ((24, 24, 24), True, G.PREC_FP32_ELEM, 100, False),
+    ((24, 24, 24), True, G.PREC_FP32_ELEM, 1, True), ((25, 25, 26), True, G.PREC_FP64, 1, False),
+])
+def test_form_by_size_and_energy_interval(shape, tet, precision, every, expected, monkeypatch):
+    """The limits of the one-launch form where the energy interval moves them."""
+    monkeypatch.delenv("MPS_SPREAD", raising=False)
+    assert form(box(*shape, tet=tet), precision=precision, energy_every=every) == expected

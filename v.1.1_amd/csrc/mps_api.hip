@@ -423,14 +423,25 @@ int prepare(const mps_mesh* mesh, const mps_material* mat, const mps_bcs* bcs, c
 }
 
 // Meshes up to this many elements step in the spread form.  us per step, spread / patch form: hex8 FP64 29,800 elements
-// 16.8 / 19.2, 35,900 18.9 / 20.4, 46,700 23.2 / 19.4; tet4 FP64 63,900 11.6 / 12.3, 93,800 16.8 / 13.6, FP32 form 35,000
-// 9.8 / 9.9, 48,000 10.3 / 10.0.  With energies every step the patch form gives up more (its energy kernels and sums): hex8
-// 35,800 24.5 / 30.9, 50,700 32.2 / 31.1; tet4 55,600 13.4 / 21.6, 82,900 (FP32 form) 18.1 / 24.6.  Loads and viscosity come
-// after creation: at 31,700 elements with both 22.8 / 29.2, at 46,700 30.3 / 27.3.  MPS_SPREAD=0 in the environment keeps
-// the patch form, MPS_SPREAD=1 takes the spread form at any size; so do the switches of the patch kernels (MPS_GATHER32,
-// MPS_DT_SKIP, MPS_TET_STAGING), which have no meaning in the spread form.  Both forms give the same bits.
+// 16.8 / 19.2, 37,000 19.6 / 20.3, 39,300 20.2 / 19.6, 46,700 23.2 / 19.4; tet4 FP64 63,900 11.6 / 12.3, 93,800 16.8 / 13.6,
+// FP32 form 35,000 9.8 / 9.9, 48,000 10.3 / 10.0.  The spread form computes the energies on every step, the patch form on
+// energy steps only, so that their interval moves the limit.  Every step: hex8 39,300 25.3 / 27.2, 41,700 26.5 / 26.7 (with
+// gravity 27.2 / 26.9), 47,900 29.2 / 27.1; tet4 93,800 18.7 / 20.4, FP32 form 18.5 / 22.0.  Every 2nd: hex8 39,300 24.4 /
+// 26.1, tet4 93,800 18.6 / 20.1.  Every 5th: hex8 39,300 23.9 / 24.1; tet4 93,800 18.6 / 18.3, FP32 form 18.1 / 17.3.
+// Every 100th: hex8 37,000 23.0 / 23.2, 39,300 23.6 / 22.8, 47,900 27.6 / 22.9; tet4 63,900 13.4 / 16.1, 82,800 17.8 / 17.4,
+// FP32 form 63,900 12.9 / 13.7, 69,800 15.0 / 14.5.  Loads and viscosity come after creation: at 31,700 elements with both
+// 22.8 / 29.2, at 46,700 30.3 / 27.3.  MPS_SPREAD=0 in the environment keeps the patch form, MPS_SPREAD=1 takes the spread
+// form at any size; so do the switches of the patch kernels (MPS_GATHER32, MPS_DT_SKIP, MPS_TET_STAGING), which have no
+// meaning in the spread form.  Both forms give the same bits.
 static const int64_t kSpreadMaxHex = 36864, kSpreadMaxTet = 64000, kSpreadMaxTet32 = 40000;
-static const int64_t kSpreadMaxHexEnergy = 49152, kSpreadMaxTetEnergy = 96000;
+static const int64_t kSpreadMaxHexEnergy = 40000, kSpreadMaxTetEnergy = 96000;  // energies every step or every second
+
+static int64_t spread_limit(const HostPrep& hp) {
+    const int every = hp.cfg.energy_every;
+    const bool often = every == 1 || every == 2;
+    if (hp.nen == 8) return often ? kSpreadMaxHexEnergy : kSpreadMaxHex;
+    return often ? kSpreadMaxTetEnergy : every > 0 || hp.cfg.precision == MPS_PREC_FP64 ? kSpreadMaxTet : kSpreadMaxTet32;
+}
 
 void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const int64_t N = hp.N, Ne = hp.Ne, nen = hp.nen;
@@ -438,13 +449,9 @@ void build_spread(const HostPrep& hp, SpreadTables* sp) {
     const char* env = getenv("MPS_SPREAD");
     const bool force = env && strcmp(env, "1") == 0;
     if (env && !force && strcmp(env, "0") == 0) return;
-    const bool fp64 = hp.cfg.precision == MPS_PREC_FP64, en = hp.cfg.energy_every > 0;
-    const int64_t most = nen == 8 ? (en ? kSpreadMaxHexEnergy : kSpreadMaxHex)
-                                  : (en ? kSpreadMaxTetEnergy : fp64 ? kSpreadMaxTet : kSpreadMaxTet32);
     if (hp.bcval.size() / 3 > (1u << 23)) return;  // Dirichlet records of an entry
     if (nen == 8 && hp.cfg.precision != MPS_PREC_FP64) return;  // its roundings are those of the patch kernels (mps_device.h)
-    if (!force && (Ne > most || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") ||
-                   getenv("MPS_TET_STAGING")))
+    if (!force && (Ne > spread_limit(hp) || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") || getenv("MPS_TET_STAGING")))
         return;
     const int64_t EB = nen == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET, nb = (Ne + EB - 1) / EB, S = Ne * nen;
     // positions in node order: a node's slots ascending, so grouped by patch
