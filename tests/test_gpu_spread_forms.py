@@ -89,3 +89,20 @@ def test_form_by_size_and_energy_interval(shape, tet, precision, every, expected
     """The limits of the one-launch form where the energy interval moves them."""
     monkeypatch.delenv("MPS_SPREAD", raising=False)
     assert form(box(*shape, tet=tet), precision=precision, energy_every=every) == expected
+
+
+@pytest.mark.parametrize("cells,window,precision,every,expected", [
+    (14, 1, G.PREC_FP64, 0, True), (14, 512, G.PREC_FP64, 0, False), (14, 256, G.PREC_FP64, 0, True),
+    (14, 256, G.PREC_FP32_ELEM, 0, False), (12, 256, G.PREC_FP32_ELEM, 0, True), (8, 1 << 20, G.PREC_FP32_ELEM, 0, False),
+    (9, 1 << 20, G.PREC_FP64, 0, True), (17, 1 << 20, G.PREC_FP64, 0, False), (17, 1, G.PREC_FP32_ELEM, 0, True),
+    (18, 1, G.PREC_FP32_ELEM, 0, False), (14, 512, G.PREC_FP64, 1, True), (20, 512, G.PREC_FP64, 1, False),
+    (14, 512, G.PREC_FP32_ELEM, 50, False), (12, 512, G.PREC_FP32_ELEM, 50, True),
+])
+def test_form_by_element_order(cells, window, precision, every, expected, monkeypatch):
+    """Tet4 elements shuffled in windows: the one-launch form is for meshes whose workgroups share few nodes."""
+    monkeypatch.delenv("MPS_SPREAD", raising=False)
+    m = box(cells, cells, cells, tet=True)
+    rng, ne = np.random.default_rng(1), m["n_elem"]
+    order = np.concatenate([i + rng.permutation(min(window, ne - i)) for i in range(0, ne, window)])
+    m["conn"] = np.ascontiguousarray(m["conn"].reshape(-1, 4)[order].ravel())
+    assert form(m, precision=precision, energy_every=every) == expected

@@ -424,7 +424,7 @@ int prepare(const mps_mesh* mesh, const mps_material* mat, const mps_bcs* bcs, c
 
 // Meshes up to this many elements step in the spread form.  us per step, spread / patch form: hex8 FP64 29,800 elements
 // 16.8 / 19.2, 37,000 19.6 / 20.3, 39,300 20.2 / 19.6, 46,700 23.2 / 19.4; tet4 FP64 63,900 11.6 / 12.3, 93,800 16.8 / 13.6,
-// FP32 form 35,000 9.8 / 9.9, 48,000 10.3 / 10.0.  The spread form computes the energies on every step, the patch form on
+// FP32 form 29,500 8.1 / 9.8, 39,000 9.8 / 10.0, with the nodes numbered at random 9.4 / 10.7 and 11.7 / 10.8.  The spread form computes the energies on every step, the patch form on
 // energy steps only, so that their interval moves the limit.  Every step: hex8 39,300 25.3 / 27.2, 41,700 26.5 / 26.7 (with
 // gravity 27.2 / 26.9), 47,900 29.2 / 27.1; tet4 93,800 18.7 / 20.4, FP32 form 18.5 / 22.0.  Every 2nd: hex8 39,300 24.4 /
 // 26.1, tet4 93,800 18.6 / 20.1.  Every 5th: hex8 39,300 23.9 / 24.1; tet4 93,800 18.6 / 18.3, FP32 form 18.1 / 17.3.
@@ -433,7 +433,7 @@ int prepare(const mps_mesh* mesh, const mps_material* mat, const mps_bcs* bcs, c
 // 22.8 / 29.2, at 46,700 30.3 / 27.3.  MPS_SPREAD=0 in the environment keeps the patch form, MPS_SPREAD=1 takes the spread
 // form at any size; so do the switches of the patch kernels (MPS_GATHER32, MPS_DT_SKIP, MPS_TET_STAGING), which have no
 // meaning in the spread form.  Both forms give the same bits.
-static const int64_t kSpreadMaxHex = 36864, kSpreadMaxTet = 64000, kSpreadMaxTet32 = 40000;
+static const int64_t kSpreadMaxHex = 36864, kSpreadMaxTet = 64000, kSpreadMaxTet32 = 32768;
 static const int64_t kSpreadMaxHexEnergy = 40000, kSpreadMaxTetEnergy = 96000;  // energies every step or every second
 
 static int64_t spread_limit(const HostPrep& hp) {
@@ -441,6 +441,23 @@ static int64_t spread_limit(const HostPrep& hp) {
     const bool often = every == 1 || every == 2;
     if (hp.nen == 8) return often ? kSpreadMaxHexEnergy : kSpreadMaxHex;
     return often ? kSpreadMaxTetEnergy : every > 0 || hp.cfg.precision == MPS_PREC_FP64 ? kSpreadMaxTet : kSpreadMaxTet32;
+}
+
+// Tet4 elements keep the caller's order, so the workgroups of a mesh numbered without locality hold up to 256 distinct
+// nodes where a structured one holds 50.  A workgroup updates 64 nodes at a time: the limits above are those of one pass,
+// and a mesh of more passes takes the spread form only while its workgroups times their passes are few.  us per step,
+// spread / patch form, tet4 boxes with their elements shuffled in windows (or all): plain FP64 2 passes 918 11.6 / 12.6,
+// 1,156 13.1 / 12.6, 3 passes 573 11.0 / 13.5, 774 14.5 / 13.5, 4 passes 764 13.1 / 15.1 (all 16.1 / 22.6); FP32 form 2 passes
+// 382 9.0 / 9.9, 516 11.2 / 9.9, 3 passes 204 11.1 / 10.3; energies every step 2 passes 1,500 15.0 / 19.2, 3 passes 1,377
+// 16.9 / 19.4, 1,734 19.8 / 19.4, FP32 form 4 passes 1,536 19.4 / 22.1; rare energies, FP32 form 3 passes 573 12.9 / 15.1,
+// 774 16.5 / 14.9.  Without this rule 58,000 elements in random order took 36.0 us against 28.0.
+static bool spread_passes_fit(const HostPrep& hp, int64_t nb, int64_t stride) {
+    const int64_t passes = (3 * stride + 3 * MPS_SPREAD_TET - 1) / (3 * MPS_SPREAD_TET);
+    if (hp.nen == 8 || passes <= 1) return true;
+    const int every = hp.cfg.energy_every;
+    if (every == 1 || every == 2) return nb * passes <= 1500;
+    if (every > 0) return nb * passes <= 600;
+    return hp.cfg.precision == MPS_PREC_FP64 ? nb * passes <= 700 : passes == 2 && nb * passes <= 400;
 }
 
 void build_spread(const HostPrep& hp, SpreadTables* sp) {
@@ -494,6 +511,7 @@ void build_spread(const HostPrep& hp, SpreadTables* sp) {
         for (int64_t s = s0; s < s1; s++) sp->lx[(size_t)s] = (uint16_t)loc[(size_t)hp.conn[(size_t)s]];
         off[(size_t)b + 1] = (int32_t)list.size();
         stride = std::max<int64_t>(stride, (int64_t)(list.size() - l0));
+        if (!force && !spread_passes_fit(hp, nb, stride)) return;
     }
     if (nb * stride > INT_MAX) return;
     sp->own.assign((size_t)N, -1);
