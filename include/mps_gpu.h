@@ -301,14 +301,16 @@ int mps_destroy(mps_handle h);
 int mps_set_graphs(mps_handle h, int32_t enable);
 
 /* Capture and instantiate, without running anything, the graphs that mps_run(h, max_steps) would
- * replay from the current step, so that the capture cost does not fall inside a later timed call.
- * Does nothing when mps_run would launch the kernels one by one.  No reference counterpart. */
+ * replay from the current step, so that the capture cost does not fall inside a later timed call (no graphs when
+ * mps_run would launch the kernels one by one).  Small meshes: also sets the one-launch form of the step up, which
+ * mps_run does once the steps asked for are worth it.  No reference counterpart. */
 int mps_prepare_run(mps_handle h, int64_t max_steps);
 
 /* Kernel timing: when enabled, mps_run records HIP events around every kernel
  * launch on the solver's stream.  mps_kernel_times returns, per kernel kind
  * [0 element, 1 node, 2 begin, 3 energy], the summed device milliseconds and the
- * launch count since the last mps_profile call.
+ * launch count since the last mps_profile call.  Small meshes in the one-launch form: [0] the steps, [1] the end
+ * of each run's launch sequences.
  * Replaces: the wall/CPU timers of the reference (solvers.cpp:22-32,
  * solverExplicit.cpp:358) with per-kernel device times. */
 int mps_profile(mps_handle h, int32_t enable);

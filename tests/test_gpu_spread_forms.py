@@ -1,4 +1,6 @@
 """Which form of the step a solve takes, and what must hold when the form changes between two runs."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -28,10 +30,12 @@ def test_forces_after_a_run_without_a_step(series_first, tet):
         n = rep["steps"]
     with window(m, 0.02) as s:
         s.set_dof_series(*(SERIES if series_first else ([], [])))
+        s.prepare_run(n)
         rc, rep = s.run(n)
         assert rc == 0 and rep["steps"] == n and rep["status"] == G.MPS_RUNNING
         f = s.internal_force_dofs(dofs)
         s.set_dof_series(*(([], []) if series_first else SERIES))
+        s.prepare_run(5)
         rc, rep = s.run(5)
         assert rc == 0 and rep["steps"] == n and rep["status"] == G.MPS_DONE
         assert np.array_equal(s.internal_force_dofs(dofs), f)
@@ -59,6 +63,7 @@ def test_forces_after_a_first_step_that_fails(series):
 def spread(s):
     """True when the next steps of s run in the spread form: one launch per step and one at the end, where the patch form
     has a node kernel in every step."""
+    s.prepare_run(3)
     s.profile(True)
     before = s.kernel_times()["node"][1]
     rc, rep = s.run(3)
@@ -106,3 +111,67 @@ def test_form_by_element_order(cells, window, precision, every, expected, monkey
     order = np.concatenate([i + rng.permutation(min(window, ne - i)) for i in range(0, ne, window)])
     m["conn"] = np.ascontiguousarray(m["conn"].reshape(-1, 4)[order].ravel())
     assert form(m, precision=precision, energy_every=every) == expected
+
+
+def test_set_up_only_where_it_is_used(monkeypatch):
+    """The tables and buffers of the one-launch form (18 MB for this mesh) are those of solves that step in it: not of one
+    with a pressure load, nor of one that is only created, and with a series of one from which it is taken away."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    monkeypatch.delenv("MPS_SPREAD", raising=False)
+    m = perturb(box(33, 33, 33), 0.1, 3)
+    dd, dv = clamp_and_pull(m)
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value / 2 ** 20
+
+    def grown(**kw):
+        """MB in use once created, after 3 steps with a pressure load or a series, after 3 more without the series."""
+        start = free()
+        with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=10) as s:
+            out = [start - free()]
+            if kw.get("pressure"):
+                s.set_loads(loads=[("pressure_inst", 5.0, 0.0, 1e9, np.array([m["n_elem"] - 1]), np.array([2]))])
+            if kw.get("series"):
+                s.set_dof_series(*SERIES)
+            s.prepare_run(3)
+            assert s.run(3)[0] == 0
+            out.append(start - free())
+            s.set_dof_series([], [])
+            s.prepare_run(3)
+            assert s.run(3)[0] == 0
+            out.append(start - free())
+        return np.array(out)
+
+    grown()
+    created, run, _ = grown()
+    assert run > created + 12
+    assert grown(pressure=True).max() < created + 6
+    _, with_series, without = grown(series=True)
+    assert with_series < created + 6 and without > created + 12
+
+
+def test_set_up_after_enough_steps(monkeypatch):
+    """Without mps_prepare_run the set-up waits for as many steps as pay for it (a 64th of the elements); the steps before it
+    run in the patch form, and the state is the same as in either form alone."""
+    m = perturb(box(16, 16, 16), 0.1, 3)  # 4,096 elements: 64 steps
+    dd, dv = clamp_and_pull(m)
+    out = []
+    for env in (None, "0", "1"):
+        monkeypatch.setenv("MPS_SPREAD", env) if env else monkeypatch.delenv("MPS_SPREAD", raising=False)
+        with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=100) as s:
+            s.profile(True)
+            nodes = []
+            for n in (30, 30, 3, 1, 36):
+                before = s.kernel_times()["node"][1]
+                assert s.run(n)[0] == 0
+                nodes.append(s.kernel_times()["node"][1] - before)
+            assert nodes == {None: [30, 30, 3, 1, 1], "0": [30, 30, 3, 1, 36], "1": [1] * 5}[env]
+            out.append([*s.get_state(), s.internal_force_dofs(np.arange(3 * m["n_nodes"], dtype=np.int32))])
+    for a, b, c in zip(*out):
+        assert np.array_equal(a, b) and np.array_equal(a, c)
+    monkeypatch.delenv("MPS_SPREAD", raising=False)
+    with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=63) as s:  # asked for more than the solve has
+        s.profile(True)
+        assert s.run(1 << 40)[1]["steps"] == 63 and s.kernel_times()["node"][1] == 63

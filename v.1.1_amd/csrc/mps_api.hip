@@ -14,6 +14,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -460,72 +461,92 @@ static bool spread_passes_fit(const HostPrep& hp, int64_t nb, int64_t stride) {
     return hp.cfg.precision == MPS_PREC_FP64 ? nb * passes <= 700 : passes == 2 && nb * passes <= 400;
 }
 
-void build_spread(const HostPrep& hp, SpreadTables* sp) {
-    const int64_t N = hp.N, Ne = hp.Ne, nen = hp.nen;
-    sp->nb = 0;
+// How a mesh takes the spread form, before its tables are looked at (build_spread).
+SpreadUse spread_wanted(const HostPrep& hp) {
     const char* env = getenv("MPS_SPREAD");
-    const bool force = env && strcmp(env, "1") == 0;
-    if (env && !force && strcmp(env, "0") == 0) return;
-    if (hp.bcval.size() / 3 > (1u << 23)) return;  // Dirichlet records of an entry
-    if (nen == 8 && hp.cfg.precision != MPS_PREC_FP64) return;  // its roundings are those of the patch kernels (mps_device.h)
-    if (!force && (Ne > spread_limit(hp) || getenv("MPS_GATHER32") || getenv("MPS_DT_SKIP") || getenv("MPS_TET_STAGING")))
-        return;
-    const int64_t EB = nen == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET, nb = (Ne + EB - 1) / EB, S = Ne * nen;
-    // positions in node order: a node's slots ascending, so grouped by patch
-    std::vector<int32_t> first((size_t)N + 1, 0);
-    for (int64_t s = 0; s < S; s++) first[(size_t)hp.conn[(size_t)s] + 1]++;
+    if (env && strcmp(env, "0") == 0) return SpreadUse::Never;
+    if (hp.bcval.size() / 3 > (1u << 23)) return SpreadUse::Never;  // Dirichlet records of an entry
+    // FP32 hex8: its roundings are those of the patch kernels (mps_device.h)
+    if (hp.nen == 8 && hp.cfg.precision != MPS_PREC_FP64) return SpreadUse::Never;
+    if (env && strcmp(env, "1") == 0) return SpreadUse::Forced;
+    const bool fits = hp.Ne <= spread_limit(hp) && !getenv("MPS_GATHER32") && !getenv("MPS_DT_SKIP") && !getenv("MPS_TET_STAGING");
+    return fits ? SpreadUse::Faster : SpreadUse::Never;
+}
+
+// Tables of the spread form from those of the patches: a patch's distinct nodes are sorted and its contributions grouped by
+// node, so a position is the next one of its node, and a workgroup's distinct nodes are the set flags, in order, among the
+// patch's nodes.
+void build_spread(const HostPrep& hp, SpreadUse use, SpreadTables* sp) {
+    const int64_t N = hp.N, Ne = hp.Ne, nen = hp.nen, S = Ne * nen;
+    sp->nb = 0;
+    const int64_t EB = nen == 8 ? MPS_SPREAD_HEX : MPS_SPREAD_TET, nb = (Ne + EB - 1) / EB;
+    const std::vector<int32_t>& first = hp.rowptr;  // positions in node order: a node's slots ascending, so grouped by patch
     for (int64_t n = 0; n < N; n++) {
         // a node of no element belongs to no workgroup; the end bits hold 32 positions
-        if (first[(size_t)n + 1] == 0 || first[(size_t)n + 1] > 32) return;
-        first[(size_t)n + 1] += first[(size_t)n];
+        const int32_t count = first[(size_t)n + 1] - first[(size_t)n];
+        if (count == 0 || count > 32) return;
     }
-    std::vector<int32_t> fill(first.begin(), first.end() - 1), patch((size_t)N, -1);
+    std::vector<int32_t> fill(first.begin(), first.end() - 1), off((size_t)nb + 1, 0);
     std::vector<uint32_t> ends((size_t)N, 0u);
+    std::unique_ptr<int32_t[]> list(new int32_t[(size_t)S]);  // the workgroups' distinct nodes, one after the other
+    int32_t* out = list.get();
     sp->pos.resize((size_t)S);
-    for (int64_t s = 0; s < S; s++) {
-        const size_t n = (size_t)hp.conn[(size_t)s];
-        const int32_t p = (int32_t)(s / nen / MPS_PATCH);
-        const int r = fill[n] - first[n];
-        if (patch[n] >= 0 && patch[n] != p) ends[n] |= 1u << (r - 1);
-        patch[n] = p;
-        sp->pos[(size_t)s] = fill[n]++;
-    }
-    for (int64_t n = 0; n < N; n++) ends[(size_t)n] |= 1u << (first[(size_t)n + 1] - first[(size_t)n] - 1);
-    // the workgroups' distinct nodes, ascending
-    std::vector<int32_t> mark((size_t)N, -1), loc((size_t)N), list, off((size_t)nb + 1, 0);
-    list.reserve((size_t)(4 * Ne));
     sp->lx.resize((size_t)S);
-    int64_t stride = 0;
-    for (int64_t b = 0; b < nb; b++) {
-        const int64_t s0 = b * EB * nen, s1 = std::min((b + 1) * EB * nen, S);
-        const size_t l0 = list.size();
-        for (int64_t s = s0; s < s1; s++) {
-            const int32_t n = hp.conn[(size_t)s];
-            if (mark[(size_t)n] != (int32_t)b) {
-                mark[(size_t)n] = (int32_t)b;
-                list.push_back(n);
+    int64_t stride = 0, b = 0;
+    uint16_t local[MPS_PATCH * MPS_MAX_NEN], loc[MPS_PATCH * MPS_MAX_NEN];  // index among the nodes of the patch, the workgroup
+    uint8_t in[MPS_PATCH * MPS_MAX_NEN] = {0};  // nodes of the patch that are in the workgroup
+    for (int64_t p = 0; p < hp.n_patch; p++) {
+        const int64_t s0 = p * MPS_PATCH * nen, s1 = std::min(s0 + MPS_PATCH * nen, S);
+        const int32_t* nd = hp.pnd.data() + hp.poff[(size_t)p];
+        const int U = hp.poff[(size_t)p + 1] - hp.poff[(size_t)p];
+        const uint16_t* row = hp.prow.data() + hp.poff[(size_t)p] + p;
+        const uint16_t* slot = hp.pcol.data() + s0;
+        for (int j = 0; j < U; j++) {
+            const size_t n = (size_t)nd[j];
+            int32_t at = fill[n];
+            for (int q = row[j]; q < row[j + 1]; q++) {
+                local[slot[q]] = (uint16_t)j;
+                sp->pos[(size_t)s0 + slot[q]] = at++;
             }
+            ends[n] |= 1u << (at - 1 - first[n]);
+            fill[n] = at;
         }
-        std::sort(list.begin() + (int64_t)l0, list.end());
-        for (size_t i = l0; i < list.size(); i++) loc[(size_t)list[i]] = (int32_t)(i - l0);
-        for (int64_t s = s0; s < s1; s++) sp->lx[(size_t)s] = (uint16_t)loc[(size_t)hp.conn[(size_t)s]];
-        off[(size_t)b + 1] = (int32_t)list.size();
-        stride = std::max<int64_t>(stride, (int64_t)(list.size() - l0));
-        if (!force && !spread_passes_fit(hp, nb, stride)) return;
+        for (int64_t t0 = s0; t0 < s1; t0 += EB * nen, b++) {
+            const int64_t t1 = std::min(t0 + EB * nen, s1);
+            for (int64_t s = t0; s < t1; s++) in[local[s - s0]] = 1;
+            int count = 0;
+            for (int w = 0; w < U; w += 8) {
+                uint64_t m;
+                memcpy(&m, in + w, 8);
+                if (!m) continue;
+                memset(in + w, 0, 8);
+                for (; m; m &= m - 1) {  // the lowest set byte
+                    const int j = w + (__builtin_ctzll(m) >> 3);
+                    loc[j] = (uint16_t)count++;
+                    *out++ = nd[j];
+                }
+            }
+            for (int64_t s = t0; s < t1; s++) sp->lx[(size_t)s] = loc[local[s - s0]];
+            off[(size_t)b + 1] = off[(size_t)b] + count;
+            stride = std::max<int64_t>(stride, count);
+            if (use != SpreadUse::Forced && !spread_passes_fit(hp, nb, stride)) return;
+        }
     }
     if (nb * stride > INT_MAX) return;
     sp->own.assign((size_t)N, -1);
-    sp->node.assign((size_t)(nb * stride), make_int4(-1, 0, 0, 0));
-    for (int64_t b = 0; b < nb; b++)
-        for (int32_t i = off[(size_t)b]; i < off[(size_t)b + 1]; i++) {
-            const int32_t n = list[(size_t)i];
-            const int64_t g = b * stride + (i - off[(size_t)b]);
-            const bool own = sp->own[(size_t)n] < 0;
-            if (own) sp->own[(size_t)n] = (int32_t)g;
-            const uint32_t z = (uint32_t)(first[(size_t)n + 1] - first[(size_t)n]) | hp.ninfo[(size_t)n] << 6;
-            sp->node[(size_t)g] = make_int4(own ? (int32_t)((uint32_t)n | 0x80000000u) : n, first[(size_t)n], (int32_t)z,
-                                            (int32_t)ends[(size_t)n]);
+    sp->node.resize((size_t)(nb * stride));
+    for (b = 0; b < nb; b++) {
+        int4* node = sp->node.data() + b * stride;
+        const int32_t count = off[(size_t)b + 1] - off[(size_t)b];
+        for (int32_t i = 0; i < count; i++) {
+            const size_t n = (size_t)list[(size_t)(off[(size_t)b] + i)];
+            const bool own = sp->own[n] < 0;
+            if (own) sp->own[n] = (int32_t)(b * stride + i);
+            const uint32_t z = (uint32_t)(first[n + 1] - first[n]) | hp.ninfo[n] << 6;
+            node[i] = make_int4(own ? (int32_t)((uint32_t)n | 0x80000000u) : (int32_t)n, first[n], (int32_t)z, (int32_t)ends[n]);
         }
+        std::fill(node + count, node + stride, make_int4(-1, 0, 0, 0));
+    }
     sp->nb = (int32_t)nb;
     sp->stride = (int32_t)stride;
 }
@@ -556,6 +577,8 @@ struct mps_solver_s {
     double* uprev_buf = nullptr;     // previous-step displacement for bulk viscosity (in allocs)
     double* fint_part = nullptr;     // partial forces of mps_internal_force (allocated on first use, in allocs)
     bool part_valid = false;         // I.part holds the forces of the current u (false: set-up scratch)
+    SpreadUse spread_use = SpreadUse::Never;
+    std::unique_ptr<HostPrep> spread_prep;  // what the spread tables are built from, until they are or can't be (set_up_spread)
     bool spread_forces = false;      // the last step ran in the spread form: its forces are in I.sp_f
     bool pressure_loads = false;     // the loads hold a pressure block
     bool primed = false;       // prologue (first dt) done
@@ -793,32 +816,6 @@ static int upload_instance(mps_solver_s* h, const HostPrep& hp) {
             I.pu_max = pu;
         }
     }
-    SpreadTables sp;
-    build_spread(hp, &sp);
-    if (sp.nb > 0) {
-        int4* spn;
-        uint16_t* spl;
-        int32_t *spp, *spo;
-        HCHK(h, dalloc(h, &spn, sp.node.size() * 16));
-        HCHK(h, dalloc(h, &spl, sp.lx.size() * 2));
-        HCHK(h, dalloc(h, &spp, sp.pos.size() * 4));
-        HCHK(h, dalloc(h, &spo, N * 4));
-        HCHK(h, dalloc(h, &I.sp_f, 2 * 3 * Ne * nen * (I.precision == MPS_PREC_FP32_ELEM ? 4 : 8)));
-        HCHK(h, dalloc(h, &I.sp_uw, 6 * N * 8));
-        HCHK(h, hipMemcpyAsync(spn, sp.node.data(), sp.node.size() * 16, hipMemcpyHostToDevice, h->stream));
-        HCHK(h, hipMemcpyAsync(spl, sp.lx.data(), sp.lx.size() * 2, hipMemcpyHostToDevice, h->stream));
-        HCHK(h, hipMemcpyAsync(spp, sp.pos.data(), sp.pos.size() * 4, hipMemcpyHostToDevice, h->stream));
-        HCHK(h, hipMemcpyAsync(spo, sp.own.data(), N * 4, hipMemcpyHostToDevice, h->stream));
-        HCHK(h, hipStreamSynchronize(h->stream));  // the host tables must outlive the copies
-        I.sp_node = spn;
-        I.sp_lx = spl;
-        I.sp_pos = spp;
-        I.sp_own = spo;
-        I.sp_nb = sp.nb;
-        I.sp_stride = sp.stride;
-        I.n_patch = hp.n_patch;
-        if (I.energy_every > 0) HCHK(h, dalloc(h, &I.sp_ep, mpsk::spread_energy_doubles(I) * 8));
-    }
     HCHK(h, hipMemcpyAsync(bcval, hp.bcval.data(), hp.bcval.size() * 8, hipMemcpyHostToDevice, h->stream));
     HCHK(h, hipMemsetAsync(hist, 0xFF, MPS_HIST_COLS * (size_t)cap * 8, h->stream));  // NaN
     I.X = X;
@@ -921,6 +918,19 @@ extern "C" int mps_create(const mps_mesh* mesh, const mps_material* mat, const m
     resolve_scratch(h->device);  // once per device, with the device current; a failure surfaces in its user
     rc = upload_instance(h, hp);
     if (rc == MPS_OK) rc = device_setup(h);
+    if (rc == MPS_OK) h->spread_use = spread_wanted(hp);
+    if (h->spread_use != SpreadUse::Never) {  // its vectors are swapped out of hp: it is of no further use here
+        h->spread_prep.reset(new HostPrep());
+        HostPrep& k = *h->spread_prep;
+        k.N = hp.N;
+        k.Ne = hp.Ne;
+        k.nen = hp.nen;
+        k.n_patch = hp.n_patch;
+        k.cfg = hp.cfg;
+        for (auto v : {&HostPrep::rowptr, &HostPrep::poff, &HostPrep::pnd}) (k.*v).swap(hp.*v);
+        for (auto v : {&HostPrep::prow, &HostPrep::pcol}) (k.*v).swap(hp.*v);
+        k.ninfo.swap(hp.ninfo);
+    }
     if (rc != MPS_OK) {
         set_global_error("mps_create: %s", h->err.c_str());
         release(h);
@@ -1523,18 +1533,64 @@ static void collect_times(mps_solver_s* h, const std::vector<int>& kinds) {
     h->ev_used = 0;
 }
 
-// Launch sequence of `count` steps starting at h->next_step; the first step is begun by the standalone begin
-// kernel unless it already is; the last node pass is unfused.  With energies every `every` steps, step k
-// computes DEFO_ENERGY and VOLUME of u_k (k % every == 0) and KIN_ENERGY of step k-1 from the velocity that
-// still holds it before the node pass (when (k-1) % every == 0 and k-1 is in this chunk), in the element kernel
-// (FP64 inviscid form) or in the standalone pass before the node kernel; after the last node pass, the pass for
-// the KIN_ENERGY of the chunk's last step.  The node kernels accumulate the work sums every step.
-// True when the steps run in the spread form: set up at creation, and nothing in the step that only the patch form has
-// (DOF series, pressure loads, which need the step's displacement, energies with viscosity, viscous tet4 elements).
-static bool use_spread(const mps_solver_s* h) {
+// True when nothing in the steps needs the patch form (DOF series, pressure loads, which need the step's displacement,
+// energies with viscosity, viscous tet4 elements).
+static bool spread_allowed(const mps_solver_s* h) {
     const MpsInst& I = h->I;
-    return I.sp_nb > 0 && !h->step_begun && I.n_series == 0 && !h->pressure_loads &&
+    return !h->step_begun && I.n_series == 0 && !h->pressure_loads &&
            (I.uprev == nullptr || (I.energy_every == 0 && I.nen == 8));
+}
+// True when the steps run in the spread form.
+static bool use_spread(const mps_solver_s* h) { return h->I.sp_nb > 0 && spread_allowed(h); }
+
+// Sets the spread form up once it pays: when mps_prepare_run asks for the steady rate, or when the steps run and asked for
+// (`steps` more) are worth its host tables.  Those take 0.5 ms for 11,339 hex8 elements, 1.3 for 35,937, 0.5 for 55,566 tet4,
+// which save 10, 1.4 and 1.3 us per step: paid back after 50, 900 and 400 steps; an element's share of a step, Ne / 64 steps
+// (tet4 128), lies near that over the whole range.  Until then, and in solves that keep a DOF series or a pressure load, the
+// steps run in the patch form, with the same bits; solves with energies, whose node sums have an order in each form, do not
+// wait.  Where memory is short they stay in the patch form.
+static int set_up_spread(mps_solver_s* h, bool now, long long steps) {
+    if (!h->spread_prep || !spread_allowed(h)) return MPS_OK;
+    if (h->I.time_mode == MPS_TIME_FIXED) steps = std::min<long long>(steps, h->I.n_steps - (h->next_step - 1));
+    const long long worth = h->I.Ne / (h->I.nen == 8 ? 64 : 128);
+    now = now || h->spread_use == SpreadUse::Forced || h->I.energy_every > 0;
+    if (!now && steps < worth - (h->next_step - 1)) return MPS_OK;
+    const std::unique_ptr<HostPrep> prep = std::move(h->spread_prep);
+    SpreadTables sp;
+    try {
+        build_spread(*prep, h->spread_use, &sp);
+    } catch (const std::bad_alloc&) {
+        return MPS_OK;
+    }
+    if (sp.nb == 0) return MPS_OK;
+    MpsInst I = h->I;
+    I.sp_nb = sp.nb;
+    I.sp_stride = sp.stride;
+    const size_t N = (size_t)I.N, S = (size_t)I.Ne * I.nen, ts = I.precision == MPS_PREC_FP32_ELEM ? 4 : 8;
+    const size_t bytes[7] = {sp.node.size() * 16, S * 2, S * 4, N * 4, 2 * 3 * S * ts, 6 * N * 8,
+                             I.energy_every > 0 ? mpsk::spread_energy_doubles(I) * 8 : 0};
+    const void* from[4] = {sp.node.data(), sp.lx.data(), sp.pos.data(), sp.own.data()};
+    size_t off[8] = {};
+    for (int i = 0; i < 7; i++) off[i + 1] = off[i] + (bytes[i] + 255) / 256 * 256;
+    char* block = nullptr;
+    if (hipMalloc(&block, off[7]) != hipSuccess) {
+        (void)hipGetLastError();
+        return MPS_OK;
+    }
+    h->allocs.push_back(block);
+    void* at[7];
+    for (int i = 0; i < 7; i++) at[i] = block + off[i];
+    for (int i = 0; i < 4; i++) HCHK(h, hipMemcpyAsync(at[i], from[i], bytes[i], hipMemcpyHostToDevice, h->stream));
+    HCHK(h, hipStreamSynchronize(h->stream));  // the host tables must outlive the copies
+    I.sp_node = (const int4*)at[0];
+    I.sp_lx = (const uint16_t*)at[1];
+    I.sp_pos = (const int32_t*)at[2];
+    I.sp_own = (const int32_t*)at[3];
+    I.sp_f = at[4];
+    I.sp_uw = (double*)at[5];
+    I.sp_ep = bytes[6] ? (double*)at[6] : nullptr;
+    h->I = I;
+    return MPS_OK;
 }
 
 // Spread form of enqueue_steps: one launch per step, and the end of the sequence.
@@ -1564,6 +1620,12 @@ static hipError_t enqueue_spread(mps_solver_s* h, long long count, std::vector<i
     return e;
 }
 
+// Launch sequence of `count` steps starting at h->next_step; the first step is begun by the standalone begin
+// kernel unless it already is; the last node pass is unfused.  With energies every `every` steps, step k
+// computes DEFO_ENERGY and VOLUME of u_k (k % every == 0) and KIN_ENERGY of step k-1 from the velocity that
+// still holds it before the node pass (when (k-1) % every == 0 and k-1 is in this chunk), in the element kernel
+// (FP64 inviscid form) or in the standalone pass before the node kernel; after the last node pass, the pass for
+// the KIN_ENERGY of the chunk's last step.  The node kernels accumulate the work sums every step.
 static hipError_t enqueue_steps(mps_solver_s* h, long long count, std::vector<int>* kinds) {
     if (use_spread(h)) return enqueue_spread(h, count, kinds);
     const MpsInst& I = h->I;
@@ -1714,6 +1776,8 @@ extern "C" int mps_prepare_run(mps_handle h, int64_t max_steps) {
     if (!h) return MPS_ERR_ARG;
     if (max_steps < 0) return h->fail(MPS_ERR_ARG, "mps_prepare_run: max_steps < 0");
     (void)hipSetDevice(h->device);
+    const int rc = set_up_spread(h, true, max_steps);
+    if (rc != MPS_OK) return rc;
     if (!graph_replay(h)) return MPS_OK;  // mps_run will launch the kernels one by one
     const long long k0 = h->next_step;
     for (long long n : chunk_plan(h, max_steps)) {  // each chunk's graph depends on its first step (energies)
@@ -1743,6 +1807,8 @@ extern "C" int mps_run(mps_handle h, int64_t max_steps, mps_report* rep) {
         if (rep) *rep = r;
         return status_code(r.status);
     }
+    rc = set_up_spread(h, false, max_steps);
+    if (rc) return rc;
     if (!h->primed) {
         // dt of step 1 uses uK = u0 only when t0 < 1e-12 (solverExplicit.cpp:109,176-178)
         const double* uK = (h->I.t0 < 1E-12) ? h->I.u : nullptr;

@@ -36,7 +36,9 @@ struct SpreadTables {
     std::vector<uint16_t> lx;
     std::vector<int32_t> pos, own;
 };
-void build_spread(const HostPrep& hp, SpreadTables* sp);
+enum class SpreadUse { Never, Faster, Forced };  // Forced: whatever its size
+SpreadUse spread_wanted(const HostPrep& hp);
+void build_spread(const HostPrep& hp, SpreadUse use, SpreadTables* sp);
 
 std::string fmt(const char* f, ...);
 void material_consts(int law, double E, double nu, double rho, double* pa, double* pb, double* c);
