@@ -1488,10 +1488,13 @@ extern "C" int mps_get_internal_force_dofs(mps_handle h, int64_t n, const int32_
         h->pick_cap = n;
     }
     HCHK(h, hipMemcpyAsync(h->pick_idx, dof, (size_t)n * 4, hipMemcpyHostToDevice, h->stream));
-    if (h->spread_forces) (void)mpsk::launch_spread_pick(h->I, h->pick_idx, n, h->pick_out, h->stream);
-    else hipLaunchKernelGGL(k_pick_fint, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->I, h->pick_idx, n,
-                       h->pick_out);
-    HCHK(h, hipGetLastError());
+    if (h->spread_forces) {
+        HCHK(h, mpsk::launch_spread_pick(h->I, h->pick_idx, n, h->pick_out, h->stream));
+    } else {
+        hipLaunchKernelGGL(k_pick_fint, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, h->stream, h->I, h->pick_idx, n,
+                           h->pick_out);
+        HCHK(h, hipGetLastError());
+    }
     HCHK(h, hipMemcpyAsync(out, h->pick_out, (size_t)n * 8, hipMemcpyDeviceToHost, h->stream));
     HCHK(h, hipStreamSynchronize(h->stream));
     return MPS_OK;
