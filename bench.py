@@ -307,9 +307,9 @@ def serving_leg(lambdas, n_req=200, precision=G.PREC_FP32_ELEM, plain_sample=32,
                            "p50_ms": st["p50_ms"], "p99_ms": st["p99_ms"], "max_ms": st["max_ms"],
                            "queue_p50_ms": st["queue_p50_ms"], "completed": st["completed"],
                            "elem_block": st["elem_block"], "grid_mult": st["grid_mult"],
-                           "tuned_mixes": st["tunings"]})
+                           "mixes": st["tunings"]})
             note(f"serving lambda={lam:g}/s: {st['solves_per_s']:.1f} solves/s, p50 {st['p50_ms']:.0f} ms, "
-                 f"p99 {st['p99_ms']:.0f} ms, tuned (bs {st['elem_block']}, grid x{st['grid_mult']})")
+                 f"p99 {st['p99_ms']:.0f} ms, launch shape bs {st['elem_block']}, grid x{st['grid_mult']}")
             last = (reqs, us)
     # one-at-a-time plain launches of a sample of the same request distribution
     reqs, us = last

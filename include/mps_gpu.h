@@ -407,8 +407,9 @@ typedef struct mps_server_stats {
     double span_ms;                 /* first submission -> last completion */
     double solves_per_s;            /* completed / span */
     double busy_ms;                 /* time with a graph launch in flight */
-    int32_t elem_block, grid_mult;  /* tuning of the latest launch */
-    int32_t tunings;                /* mix sizes launched so far (half-decades of active elements) */
+    int32_t elem_block, grid_mult;  /* shape of the latest launch */
+    int32_t tunings;                /* mix sizes (half-decades of active elements) whose shape the launch rule has
+                                       chosen; 0 where the configuration gives elem_block or grid_mult */
     int32_t _pad;
 } mps_server_stats;
 

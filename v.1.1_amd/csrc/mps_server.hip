@@ -80,7 +80,7 @@ struct mps_server_s {
     Clock::time_point t_first, t_last;
     bool have_first = false;
     double busy_ms = 0.0;
-    std::set<int> mixes;         // mix sizes launched (active elements, in half-decade buckets)
+    std::set<int> mixes;         // mix sizes whose launch shape the rule chose (active elements, in half-decade buckets)
     int cur_bs = 0, cur_gm = 0;  // tuning of the latest launch (under mu)
     std::string err;
 };
@@ -198,7 +198,8 @@ static void worker_loop(mps_server_s* S) {
             const double active = (double)std::max<int64_t>(1, mps_batch_active_elements(S->batch));
             std::lock_guard<std::mutex> lk(S->mu);
             mps_batch_tuning(S->batch, &S->cur_bs, &S->cur_gm);
-            S->mixes.insert((int)std::floor(2.0 * std::log10(active)));
+            if (S->cfg.batch.elem_block == 0 && S->cfg.batch.grid_mult == 0)
+                S->mixes.insert((int)std::floor(2.0 * std::log10(active)));
             S->launches++;
         }
         admit(S);  // overlaps with the launch in flight
