@@ -463,11 +463,13 @@ static int flush_tables(mps_batch_s* b) {
         for (int n0 = 0; n0 < S.inst.N; n0 += bs) wn.push_back({s, n0, std::min(n0 + bs, S.inst.N), n0 == 0});
     }
     // one workgroup per patch up to 16 per CU: the hardware then places them as CUs become free, where a smaller
-    // persistent grid fixes each workgroup's patches beforehand.  The multiple moves in powers of two, so that an
-    // admission rarely needs a new graph (workgroups without a patch end at once).
+    // persistent grid fixes each workgroup's patches beforehand.  A new grid needs a new graph (40 us), so the multiple moves
+    // in powers of two and comes down only when a quarter of it would do: content that hovers around a power of two keeps its
+    // graph (workgroups without a patch end at once).
     if (b->grid_rule) {
-        b->grid_mult = 1;
-        while (b->grid_mult < 16 && (size_t)b->grid_mult * b->cus < we.size()) b->grid_mult *= 2;
+        int need = 1;
+        while (need < 16 && (size_t)need * b->cus < we.size()) need *= 2;
+        if (need > b->grid_mult || 4 * need <= b->grid_mult) b->grid_mult = need;
     }
     const int nt = 1 - b->cur;
     Table& T = b->tab[nt];
