@@ -646,7 +646,8 @@ extern "C" int mps_batch_autotune(mps_batch b, int32_t* elem_block, int32_t* gri
         }
     };
     snapshot(true);
-    const int gm0 = b->grid_mult;
+    const int gm0 = b->grid_mult, bs0 = b->bs;
+    const bool rule0 = b->grid_rule;
     float best = 1e30f;
     int best_gm = gm0;
     b->grid_rule = false;
@@ -683,6 +684,11 @@ extern "C" int mps_batch_autotune(mps_batch b, int32_t* elem_block, int32_t* gri
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     b->grid_mult = best_gm;
+    if (rc != MPS_OK) {  // a trial failed: the launch shape stays what it was
+        b->grid_mult = gm0;
+        b->bs = bs0;
+        b->grid_rule = rule0;
+    }
     b->dirty = true;
     for (auto& t : b->tab)
         if (t.exec) {
