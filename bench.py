@@ -234,7 +234,7 @@ def plain_solve(c, precision):
 
 
 def batch_leg(precision, n_inst=512, steps=1000, plain_sample=48):
-    """512 independent cubes n^3, n ~ U{6..40}, 1000 steps each, in one arena; autotuned hipGraph replay,
+    """512 independent cubes n^3, n ~ U{6..40}, 1000 steps each, in one arena; hipGraph replay on the grid that the autotuner fixes,
     against the same solves launched one at a time with plain launches (random sample)."""
     sols = configs.batch_meshes(n_inst, steps=steps)
     gp = sum(c["mesh"]["n_elem"] * 8 for c in sols) * steps

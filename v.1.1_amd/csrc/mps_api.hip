@@ -1723,11 +1723,13 @@ static bool graph_replay(const mps_solver_s* h) { return h->use_graphs && !h->pr
 
 // The graph that replays a chunk of n steps (begin, (element, node+begin) x (n-1), element, node), captured
 // and instantiated on its second use, or at once (`now`: mps_prepare_run); *out = nullptr: the caller launches the steps
-// one by one.  A captured step costs 1.2 us of host time once and saves 0.5 us per replay (launches one by one keep the GPU
-// busy from 200 elements up), so a chunk that runs only once is cheaper without: a solve of 2,431 elements over 500 steps
-// with its set-up 5.1 -> 4.5 ms.  Capture does not execute anything: the host mirror of the step counter is restored
-// afterwards.  The kernels read the step index from the control block, so one graph serves every chunk of n steps wherever
-// it starts.
+// one by one.  us per step of a chunk of 256, launched one by one / replayed / captured: 1,000 hex8 elements 6.4 / 5.9 / 2.7 in
+// the spread form, 19.6 / 19.1 / 4.8 in the patch form, 46,700 21.5 / 21.4 / 4.9.  A capture is paid back by 6 replays in the
+// spread form, by 10 in the patch form of a small mesh, and hardly ever above 40,000 elements.  So a chunk that runs once goes
+// without (a solve of 2,431 elements over 500 steps with its set-up 5.1 -> 4.7 ms); from the second use on the chunk is taken
+// for one of many, which costs a solve that is never more than one chunk of single launches beyond a capture on first use.
+// Capture does not execute anything: the host mirror of the step counter is restored afterwards.  The kernels read the step
+// index from the control block, so one graph serves every chunk of n steps wherever it starts.
 static hipError_t chunk_graph(mps_solver_s* h, long long n, bool now, hipGraphExec_t* out) {
     const long long phase = h->cfg.energy_every > 0 ? h->next_step % h->cfg.energy_every : 0;
     *out = nullptr;

@@ -41,7 +41,8 @@ __device__ __forceinline__ float fma_t(float a, float b, float c) { return __bui
 
 // The arithmetic of the element forces is written with explicit FMAs and without contraction, so that an element's
 // forces have the same bits in every kernel that computes them (one work-item per element, eight per element, batched,
-// with energies), whatever the compiler places around it.
+// with energies), whatever the compiler places around it.  The exception is FP32 hex8 (cof3_c below): there the compiler
+// chooses, and equal bits of two kernels hold as far as it chooses alike, which the tests check.
 template <typename T>
 __device__ __forceinline__ T diff2(T a, T b, T c, T d) {  // a b - c d
 #pragma clang fp contract(off)
