@@ -153,9 +153,9 @@ def test_set_up_only_where_it_is_used(monkeypatch):
 
 
 def test_set_up_after_enough_steps(monkeypatch):
-    """Without mps_prepare_run the set-up waits for as many steps as pay for it (a 64th of the elements); the steps before it
-    run in the patch form, and the state is the same as in either form alone."""
-    m = perturb(box(16, 16, 16), 0.1, 3)  # 4,096 elements: 64 steps
+    """Without mps_prepare_run the set-up waits for as many steps as pay for it (n^2 / 2^21 of n hex8 elements); the steps
+    before it run in the patch form, and the state is the same as in either form alone."""
+    m = perturb(box(16, 16, 32), 0.1, 3)  # 8,192 elements: 32 steps
     dd, dv = clamp_and_pull(m)
     out = []
     for env in (None, "0", "1"):
@@ -163,15 +163,15 @@ def test_set_up_after_enough_steps(monkeypatch):
         with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=100) as s:
             s.profile(True)
             nodes = []
-            for n in (30, 30, 3, 1, 36):
+            for n in (15, 15, 1, 1, 36):
                 before = s.kernel_times()["node"][1]
                 assert s.run(n)[0] == 0
                 nodes.append(s.kernel_times()["node"][1] - before)
-            assert nodes == {None: [30, 30, 3, 1, 1], "0": [30, 30, 3, 1, 36], "1": [1] * 5}[env]
+            assert nodes == {None: [15, 15, 1, 1, 1], "0": [15, 15, 1, 1, 36], "1": [1] * 5}[env]
             out.append([*s.get_state(), s.internal_force_dofs(np.arange(3 * m["n_nodes"], dtype=np.int32))])
     for a, b, c in zip(*out):
         assert np.array_equal(a, b) and np.array_equal(a, c)
     monkeypatch.delenv("MPS_SPREAD", raising=False)
-    with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=63) as s:  # asked for more than the solve has
+    with G.Solver(m, dir_dof=dd, dir_val=dv, n_steps=31) as s:  # asked for more than the solve has
         s.profile(True)
-        assert s.run(1 << 40)[1]["steps"] == 63 and s.kernel_times()["node"][1] == 63
+        assert s.run(1 << 40)[1]["steps"] == 31 and s.kernel_times()["node"][1] == 31

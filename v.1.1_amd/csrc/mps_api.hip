@@ -1547,15 +1547,15 @@ static bool spread_allowed(const mps_solver_s* h) {
 static bool use_spread(const mps_solver_s* h) { return h->I.sp_nb > 0 && spread_allowed(h); }
 
 // Sets the spread form up once it pays: when mps_prepare_run asks for the steady rate, or when the steps run and asked for
-// (`steps` more) are worth its host tables.  Those take 0.5 ms for 11,339 hex8 elements, 1.3 for 35,937, 0.5 for 55,566 tet4,
-// which save 10, 1.4 and 1.3 us per step: paid back after 50, 900 and 400 steps; an element's share of a step, Ne / 64 steps
-// (tet4 128), lies near that over the whole range.  Until then, and in solves that keep a DOF series or a pressure load, the
+// (`steps` more) are worth its host tables.  Those take 0.43 ms for 11,339 hex8 elements, 0.7 for 19,656, 1.2 for 35,937, 0.5
+// for 55,566 tet4, which save 9.5, 6.5, 1.4 and 1.4 us per step: paid back after 45, 110, 860 and 360 steps.  Ne^2 / 2^21
+// steps (tet4 2^23) are 61, 184, 615 and 368.  Until then, and in solves that keep a DOF series or a pressure load, the
 // steps run in the patch form, with the same bits; solves with energies, whose node sums have an order in each form, do not
 // wait.  Where memory is short they stay in the patch form.
 static int set_up_spread(mps_solver_s* h, bool now, long long steps) {
     if (!h->spread_prep || !spread_allowed(h)) return MPS_OK;
     if (h->I.time_mode == MPS_TIME_FIXED) steps = std::min<long long>(steps, h->I.n_steps - (h->next_step - 1));
-    const long long worth = h->I.Ne / (h->I.nen == 8 ? 64 : 128);
+    const long long worth = (long long)h->I.Ne * h->I.Ne >> (h->I.nen == 8 ? 21 : 23);
     now = now || h->spread_use == SpreadUse::Forced || h->I.energy_every > 0;
     if (!now && steps < worth - (h->next_step - 1)) return MPS_OK;
     const std::unique_ptr<HostPrep> prep = std::move(h->spread_prep);
